@@ -496,9 +496,10 @@ __device__ __attribute__((always_inline)) void absorbed_panel(const Args& a, con
     if (refactored) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the inverse is read back below
     __syncthreads();
     const uint32_t om = *s_word;
+    constexpr int LDA = lda<T>();
     T* la = reinterpret_cast<T*>(lds);
     T* lb = la + TS * LDA;
-    tile_to_lds_masked<COH>(pool + (size_t)oslot * TE, lp ? la : lb, lp ? LDA : LDB, tid, om);
+    tile_to_lds<COH>(pool + (size_t)oslot * TE, lp ? la : lb, lp ? LDA : LDB, tid, om, pr.b < 0);
     if (refactored) tile_to_lds<true>(pool + (size_t)(lp ? lu.out3 : lu.out2) * TE, icopy, lp ? LDB : LDA, tid);
     __syncthreads();
     acc_t acc[2][2];
@@ -510,20 +511,17 @@ __device__ __attribute__((always_inline)) void absorbed_panel(const Args& a, con
     if (!MASKS || (ma != 0 && mb != 0)) {  // a zero product is skipped, as in the GEMM task
         uint32_t kuse = 0xFu;
         if constexpr (MASKS) kuse = k_blocks_used(ma, mb, wr >> 4, wc >> 4);
-        gemm_lds<T, false>(acc, lp ? la : icopy, lp ? icopy : lb, pr.b < 0 ? T(-1) : T(1), wr, wc, li, lk, kuse);
+        gemm_lds<T, false>(acc, lp ? la : icopy, lp ? icopy : lb, wr, wc, li, lk, kuse);
     }
     T* C = pool + (size_t)pd.out0 * TE;
     bool nz[2][2] = {{false, false}, {false, false}};
 #pragma unroll
     for (int m = 0; m < 2; m++)
 #pragma unroll
-        for (int n = 0; n < 2; n++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const T v = acc[m][n][r];
-                gst(&C[(wr + m * 16 + MfmaOp<T>::row(lk, r)) * TS + wc + n * 16 + li], v);
-                if constexpr (MASKS) nz[m][n] |= fabs(v) > T(MASK_TINY);
-            }
+        for (int n = 0; n < 2; n++) {
+            acc_store_global(acc[m][n], C, wr + m * 16, wc + n * 16, li, lk);
+            if constexpr (MASKS) nz[m][n] = acc_nonzero(acc[m][n], MASK_TINY);
+        }
     if constexpr (MASKS) {
         const uint32_t qm = quad_mask(nz, wr >> 4, wc >> 4);
         if (lane == 0) out_mask[w] = qm;
@@ -566,7 +564,7 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
     // beyond what any task kind uses.  The kernels built for two (no registers to spare)
     // run them as after-links instead: right after the lu, in the same workgroup.
     constexpr bool ABSORB = sizeof(T) == 4 && !BF16 && !LLT && ONE;
-    constexpr int XCOPY_BYTES = ABSORB ? TS * LDA * (int)sizeof(T) : 0;
+    constexpr int XCOPY_BYTES = ABSORB ? TS * lda<T>() * (int)sizeof(T) : 0;
     constexpr int ZCOPY_BYTES = ABSORB ? TS * LDB * (int)sizeof(T) : 0;
     __shared__ __attribute__((aligned(16))) char lds[lds_bytes<T>() + XCOPY_BYTES + ZCOPY_BYTES];
     T* const xcopy = ABSORB ? reinterpret_cast<T*>(lds + lds_bytes<T>()) : nullptr;

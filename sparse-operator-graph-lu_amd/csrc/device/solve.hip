@@ -400,6 +400,7 @@ __device__ inline void panel_to_lds(const double* __restrict__ v, int64_t ld, in
 
 template <typename T, int NP>
 __global__ __launch_bounds__(NT, 2) void k_trsm_persistent(SolveArgs a) {
+    constexpr int LDA = lda<double>();
     __shared__ __attribute__((aligned(16))) double la[TS * LDA];
     __shared__ __attribute__((aligned(16))) double lb[TS * LDB];
     __shared__ int s_row, s_abort;
@@ -445,7 +446,7 @@ __global__ __launch_bounds__(NT, 2) void k_trsm_persistent(SolveArgs a) {
                 for (int n = 0; n < 2; n++)
 #pragma unroll
                     for (int r = 0; r < 4; r++) {
-                        const int row = wr + m * 16 + M::row(lk, r), col = p * TS + wc + n * 16 + li;
+                        const int row = wr + m * 16 + M::row(li, lk, r), col = p * TS + wc + n * 16 + li;
                         acc[p][m][n][r] = col < a.nrhs ? a.in[rowI + row + (int64_t)col * a.ld] : 0.0;
                     }
         // dependencies oldest first; each L tile is staged once for all panels
@@ -480,7 +481,7 @@ __global__ __launch_bounds__(NT, 2) void k_trsm_persistent(SolveArgs a) {
                 for (int n = 0; n < 2; n++)
 #pragma unroll
                     for (int r = 0; r < 4; r++)
-                        lb[(wr + m * 16 + M::row(lk, r)) * LDB + wc + n * 16 + li] = acc[p][m][n][r];
+                        lb[(wr + m * 16 + M::row(li, lk, r)) * LDB + wc + n * 16 + li] = acc[p][m][n][r];
             __syncthreads();
             acc_t o[2][2];
 #pragma unroll
@@ -494,7 +495,7 @@ __global__ __launch_bounds__(NT, 2) void k_trsm_persistent(SolveArgs a) {
                 for (int n = 0; n < 2; n++)
 #pragma unroll
                     for (int r = 0; r < 4; r++) {
-                        const int row = wr + m * 16 + M::row(lk, r), col = p * TS + wc + n * 16 + li;
+                        const int row = wr + m * 16 + M::row(li, lk, r), col = p * TS + wc + n * 16 + li;
                         if (col < a.nrhs) a.out[rowI + row + (int64_t)col * a.ld] = o[m][n][r];
                     }
         }

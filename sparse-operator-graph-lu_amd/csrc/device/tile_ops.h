@@ -31,8 +31,15 @@ namespace sogl_dev {
 constexpr int NT = 256;      // threads per workgroup
 constexpr int TS = 64;       // tile edge
 constexpr int TE = TS * TS;  // tile elements
-constexpr int LDA = TS + 1;  // LDS row stride of row-read operands (odd: column reads hit distinct banks)
-constexpr int LDB = TS + 2;  // LDS row stride of column-read operands (keeps 16-byte row alignment)
+
+// LDS row strides of a tile, in elements of T.  Rows start on 16 bytes, so tiles move in
+// and out of LDS 16 bytes per lane.  LDA: operands read by rows, 4 consecutive k per lane
+// (gemm_lds): 16 rows of 16-byte pieces must fall on distinct banks of 64, which a stride
+// of 4 banks (mod 64) gives: 68 floats, 66 doubles.  LDB: operands read by columns, lane
+// group lk at rows 4 lk + k4: 4 LDB = 16 elements (mod 64 floats, mod 32 doubles).
+template <typename T>
+constexpr int lda() { return sizeof(T) == 8 ? TS + 2 : TS + 4; }
+constexpr int LDB = TS + 4;
 
 typedef double v4d __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -41,6 +48,7 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
 
 // LDS elements of the blocked LU (defined with it below)
+template <typename C>
 constexpr int lu_lds_elems();
 
 // LDS bytes one workgroup needs for any task kind, per storage type: the GEMM's A and
@@ -48,8 +56,8 @@ constexpr int lu_lds_elems();
 // refactorisation (tile + 2 x 64 doubles)
 template <typename T>
 constexpr int lds_bytes() {
-    return cmax(cmax((TS * LDA + TS * LDB) * (int)sizeof(T), lu_lds_elems() * (int)sizeof(T)),
-                sizeof(T) == 8 ? 0 : (TS * LDA + 2 * TS) * 8);
+    return cmax(cmax((TS * lda<T>() + TS * LDB) * (int)sizeof(T), lu_lds_elems<T>() * (int)sizeof(T)),
+                sizeof(T) == 8 ? 0 : (TS * lda<double>() + 2 * TS) * 8);
 }
 
 // ------------------------------------------------------------------ publishing
@@ -79,6 +87,16 @@ template <typename T>
 __device__ __forceinline__ void gst(T* p, T v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// 16 bytes at byte offset `off` of a tile, written through as gst does (the same sc1 cache
+// policy on a buffer store; atomics are at most 8 bytes)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const void* tile);
+constexpr int CPOL_SC1 = 16;  // the sc1 bit of a buffer instruction's cache policy
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+template <typename V>
+__device__ __forceinline__ void gst16(void* tile, int off, V v) {
+    static_assert(sizeof(V) == 16, "16-byte vectors");
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), tile_rsrc(tile), off, 0, CPOL_SC1);
+}
 // The wave's own stores (and loads) have completed: with gst stores, the wave's part
 // of a workgroup release at agent scope (a barrier after it orders the flag store).
 // The comment marks the wait in the assembly, where a test checks that the publish
@@ -93,7 +111,6 @@ __device__ __forceinline__ void wave_stores_done() { asm volatile("s_waitcnt vmc
 // invalidated, so plain loads read the right bytes (and hit in L2 when they can).  The
 // form is fixed per kernel: a choice per operand inside the pair loop cost registers
 // (measured: spills in the kernels built for two workgroups per CU).
-constexpr int CPOL_SC1 = 16;  // the sc1 bit of a buffer instruction's cache policy
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const void* tile) {
     // raw buffer over one tile (at most 64 x 64 doubles); dword 3: 32-bit data format
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(tile), 0, TE * 8, 0x00020000);
@@ -139,90 +156,98 @@ __device__ __forceinline__ void load16c(const T* tile, int i, C (&v)[16]) {
         }
     }
 }
-template <typename T, typename C>
-__device__ __forceinline__ void load16(const T* tile, int i, bool coh, C (&v)[16]) {
-    if (coh)
-        load16c<true>(tile, i, v);
-    else
-        load16c<false>(tile, i, v);
-}
 
 // ------------------------------------------------------------------ loads
-// thread t moves row t/4, columns (t%4)*16 .. +15 of a tile between global and LDS
-// (that segment lies in 16x16 block (t/64, t%4))
-template <bool COH = false, typename T>
-__device__ inline void tile_to_lds(const T* __restrict__ g, T* __restrict__ s, int ld, int tid) {
-    const int r = tid >> 2, c0 = (tid & 3) * 16;
-    T v[16];
-    load16c<COH>(g, r * TS + c0, v);
-    T* dst = s + r * ld + c0;
-#pragma unroll
-    for (int q = 0; q < 16; q++) dst[q] = v[q];
-}
-
-// One thread's segment of a tile (the same row segment as tile_to_lds) held in
-// registers: the next pair's operands are loaded into it while the current pair
-// multiplies from LDS, then written to LDS.
+// How the 256 threads hold a tile: as 16-byte vectors, NV per thread, consecutive lanes on
+// consecutive vectors of a row.  Wave w has rows 16w .. 16w+15 (block row w); one load
+// instruction of it covers 1 KiB of whole lines (FP32: 4 rows, FP64: 2).  With 16
+// consecutive elements per thread instead, every instruction touched 64 lines, 16 bytes
+// of each: the loads of a pair took about 4 times the cache's address cycles (FP64: 8
+// times), and a coherent load, which has no L1 to hit, fetched each line as often.
+// Measured together with the 16-byte LDS rows and conflict-free operand reads (lda, LDB,
+// gemm_lds) and the 16-byte stores (MfmaOp<float>, blk_store_global): C2 (3D 48^3) factor
+// FP64 98.4 -> 79.2 ms, FP32 57.3 -> 51.9; 2D 128^2 FP64 with slot reuse 11.6 -> 8.4; C3
+// (random band, n = 16,384) FP32 47.2 -> 41.4; a one-pair dense FP64 GEMM task 6.7 -> 4.7
+// us; C5, whose tiles are mostly zero blocks, unchanged (349 -> 348 ms).
 template <typename T>
-struct Seg;
+struct TileVec;
 template <>
-struct Seg<float> {
-    float4 v[4];
+struct TileVec<float> {
+    typedef float4 V;
+    static constexpr int NV = 4, PER = 4, LANES = 16;  // vectors per thread, elements of one, lanes per row
 };
 template <>
-struct Seg<double> {
-    double2 v[8];
+struct TileVec<double> {
+    typedef double2 V;
+    static constexpr int NV = 8, PER = 2, LANES = 32;
 };
-// on = false: the segment's 16x16 block is zero by the tile's mask and is not loaded
+// row of vector q of thread tid, its first column (the same for every q), and the column
+// of 16x16 blocks it lies in
+template <typename T>
+__device__ __forceinline__ int vec_row(int q, int tid) {
+    constexpr int L = TileVec<T>::LANES;
+    return 16 * (tid >> 6) + q * (64 / L) + ((tid & 63) / L);
+}
+template <typename T>
+__device__ __forceinline__ int vec_col(int tid) { return (tid % TileVec<T>::LANES) * TileVec<T>::PER; }
+template <typename T>
+__device__ __forceinline__ int vec_block(int tid) { return vec_col<T>(tid) >> 4; }
+
+__device__ __forceinline__ float vabsmax(const float4& v) {
+    return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
+}
+__device__ __forceinline__ double vabsmax(const double2& v) { return fmax(fabs(v.x), fabs(v.y)); }
+
+// One thread's vectors of a tile held in registers: the next pair's operands are loaded
+// into them while the current pair multiplies from LDS, then written to LDS.
+template <typename T>
+struct Seg {
+    typename TileVec<T>::V v[TileVec<T>::NV];
+};
+// on = false: the thread's 16x16 block is zero by the tile's mask and is not loaded
 template <bool COH = false, typename T>
 __device__ __forceinline__ void seg_load(const T* __restrict__ g, Seg<T>& s, int tid, bool on) {
     if (!on) return;
-    const int r = tid >> 2, c0 = (tid & 3) * 16;
-    typedef typename std::remove_reference<decltype(s.v[0])>::type V;
-    constexpr int NV = (int)(sizeof(s.v) / sizeof(V));
 #pragma unroll
-    for (int q = 0; q < NV; q++) s.v[q] = ld16c<COH, V>(g, r * TS + c0 + q * (16 / NV));
+    for (int q = 0; q < TileVec<T>::NV; q++)
+        s.v[q] = ld16c<COH, typename TileVec<T>::V>(g, vec_row<T>(q, tid) * TS + vec_col<T>(tid));
 }
-// on = false: write zeros (the block is zero by the tile's mask)
+__device__ __forceinline__ float4 vneg(const float4& v) { return make_float4(-v.x, -v.y, -v.z, -v.w); }
+__device__ __forceinline__ double2 vneg(const double2& v) { return make_double2(-v.x, -v.y); }
+// on = false: write zeros (the block is zero by the tile's mask); neg: the negated tile
+// (of a subtracted product's first operand)
 template <typename T>
-__device__ __forceinline__ void seg_store(const Seg<T>& s, T* __restrict__ lds, int ld, int tid, bool on) {
-    const int r = tid >> 2, c0 = (tid & 3) * 16;
-    T* dst = lds + r * ld + c0;
+__device__ __forceinline__ void seg_store(const Seg<T>& s, T* __restrict__ lds, int ld, int tid, bool on,
+                                          bool neg = false) {
+    typedef typename TileVec<T>::V V;
+    T* dst = lds + vec_row<T>(0, tid) * ld + vec_col<T>(tid);
+    constexpr int step = 64 / TileVec<T>::LANES;
     if (on) {
-        if constexpr (sizeof(T) == 8) {
+        if (neg) {  // uniform
 #pragma unroll
-            for (int q = 0; q < 8; q++) {
-                dst[2 * q] = s.v[q].x;
-                dst[2 * q + 1] = s.v[q].y;
-            }
+            for (int q = 0; q < TileVec<T>::NV; q++) *reinterpret_cast<V*>(dst + q * step * ld) = vneg(s.v[q]);
         } else {
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                dst[4 * q] = s.v[q].x;
-                dst[4 * q + 1] = s.v[q].y;
-                dst[4 * q + 2] = s.v[q].z;
-                dst[4 * q + 3] = s.v[q].w;
-            }
+            for (int q = 0; q < TileVec<T>::NV; q++) *reinterpret_cast<V*>(dst + q * step * ld) = s.v[q];
         }
     } else {
 #pragma unroll
-        for (int q = 0; q < 16; q++) dst[q] = T(0);
+        for (int q = 0; q < TileVec<T>::NV; q++) *reinterpret_cast<V*>(dst + q * step * ld) = V{};
     }
 }
-// whether thread tid's segment lies in a block whose bit is set in mask m
-__device__ __forceinline__ bool seg_on(uint32_t m, int tid) { return (m >> (4 * (tid >> 6) + (tid & 3))) & 1u; }
+// whether thread tid's vectors lie in a block whose bit is set in mask m
+template <typename T>
+__device__ __forceinline__ bool seg_on(uint32_t m, int tid) { return (m >> (4 * (tid >> 6) + vec_block<T>(tid))) & 1u; }
 
-// The same with the blocks whose mask bit is clear written as zeros, not loaded.
+// a whole tile from global memory to LDS (row stride ld); m: blocks whose bit is clear are
+// written as zeros, not loaded
 template <bool COH = false, typename T>
-__device__ inline void tile_to_lds_masked(const T* __restrict__ g, T* __restrict__ s, int ld, int tid, uint32_t m) {
-    const int r = tid >> 2, c0 = (tid & 3) * 16;
-    if ((m >> (4 * (r >> 4) + (tid & 3))) & 1u) {
-        tile_to_lds<COH>(g, s, ld, tid);
-    } else {
-        T* dst = s + r * ld + c0;
-#pragma unroll
-        for (int q = 0; q < 16; q++) dst[q] = T(0);
-    }
+__device__ inline void tile_to_lds(const T* __restrict__ g, T* __restrict__ s, int ld, int tid, uint32_t m = 0xFFFFu,
+                                   bool neg = false) {
+    Seg<T> v;
+    const bool on = seg_on<T>(m, tid);
+    seg_load<COH>(g, v, tid, on);
+    seg_store(v, s, ld, tid, on, neg);
 }
 
 // ------------------------------------------------------------------ 16x16 block masks
@@ -249,25 +274,83 @@ __host__ __device__ inline uint32_t mask_row(uint32_t m, int I) { return (m >> (
 // ------------------------------------------------------------------ GEMM
 template <typename T>
 struct MfmaOp;
-// Output row held by register r of lane group g = lane/16 (column = lane%16).
-// Measured on gfx950: the f32 16x16x4 accumulator keeps 4 consecutive rows per
-// lane group (row 4g + r); the f64 one interleaves them (row 4r + g).
+// A 16x16 block of accumulators: v_mfma_*_16x16x4 takes A[i][k] in lane i + 16k and
+// B[k][j] in lane j + 16k.  Measured on gfx950: register r of lane li + 16 g holds, in
+// FP32, four consecutive entries along the first operand's index (4g + r) at the second's
+// li; in FP64 the entry (4r + g, li).  FP32 therefore passes B first: the accumulator is
+// the product's row li, columns 4g .. 4g+3, and moves to and from memory 16 bytes per
+// lane.  (row, col: the block's entry in register r.)
 template <>
 struct MfmaOp<double> {
     typedef v4d acc_t;
     static __device__ inline acc_t mma(double a, double b, acc_t c) {
         return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
     }
-    static __device__ inline int row(int g, int r) { return 4 * r + g; }
+    static __device__ inline int row(int, int lk, int r) { return 4 * r + lk; }
+    static __device__ inline int col(int li, int, int) { return li; }
 };
 template <>
 struct MfmaOp<float> {
     typedef v4f acc_t;
     static __device__ inline acc_t mma(float a, float b, acc_t c) {
-        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(b, a, c, 0, 0, 0);
     }
-    static __device__ inline int row(int g, int r) { return 4 * g + r; }
+    static __device__ inline int row(int li, int, int) { return li; }
+    static __device__ inline int col(int, int lk, int r) { return 4 * lk + r; }
 };
+
+// An accumulator block from and to LDS (block at p, row stride ld; FP32: 16-byte rows) and
+// from and to a tile in global memory (block at row r0, column c0; COH as ld16c).
+template <typename T>
+__device__ __forceinline__ typename MfmaOp<T>::acc_t acc_load(const T* p, int ld, int li, int lk) {
+    if constexpr (sizeof(T) == 4) {
+        return *reinterpret_cast<const v4f*>(p + li * ld + 4 * lk);
+    } else {
+        v4d a;
+#pragma unroll
+        for (int r = 0; r < 4; r++) a[r] = p[(4 * r + lk) * ld + li];
+        return a;
+    }
+}
+template <typename T>
+__device__ __forceinline__ void acc_store(const typename MfmaOp<T>::acc_t& a, T* p, int ld, int li, int lk) {
+    if constexpr (sizeof(T) == 4) {
+        *reinterpret_cast<v4f*>(p + li * ld + 4 * lk) = a;
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; r++) p[(4 * r + lk) * ld + li] = a[r];
+    }
+}
+template <bool COH, typename T>
+__device__ __forceinline__ typename MfmaOp<T>::acc_t acc_load_global(const T* tile, int r0, int c0, int li, int lk) {
+    if constexpr (sizeof(T) == 4) {
+        return ld16c<COH, v4f>(tile, (r0 + li) * TS + c0 + 4 * lk);
+    } else {
+        v4d a;
+#pragma unroll
+        for (int r = 0; r < 4; r++) a[r] = ld1c<COH>(tile, (r0 + 4 * r + lk) * TS + c0 + li);
+        return a;
+    }
+}
+template <typename T>
+__device__ __forceinline__ void acc_store_global(const typename MfmaOp<T>::acc_t& a, T* tile, int r0, int c0, int li,
+                                                 int lk) {
+    if constexpr (sizeof(T) == 4) {
+        gst16(tile, ((r0 + li) * TS + c0 + 4 * lk) * 4, a);
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; r++) gst(&tile[(r0 + 4 * r + lk) * TS + c0 + li], a[r]);
+    }
+}
+// some |v| > 1e-18 among a lane's entries of a block (its mask bit, by ballot)
+template <typename A>
+__device__ __forceinline__ bool acc_nonzero(const A& a, double tiny) {
+    typedef decltype(a[0] + a[0]) E;
+    bool nz = false;
+#pragma unroll
+    for (int r = 0; r < 4; r++) nz |= fabs(a[r]) > E(tiny);
+    return nz;
+}
 
 // One (A,B) pair of a GEMM task.  a, b: the operands' pool slots (tile data and block
 // masks); b < 0 encodes a subtracted product (mulneg): slot = -b - 1; a < 0 encodes a
@@ -282,29 +365,56 @@ struct Pair {
 __host__ __device__ inline int pair_a(const Pair& p) { return p.a < 0 ? -p.a - 1 : p.a; }
 __host__ __device__ inline int pair_b(const Pair& p) { return p.b < 0 ? -p.b - 1 : p.b; }
 
-// acc += sg * A B (or A B^T) from LDS: A rows with stride LDA; B row-major with stride
-// LDB, or, transposed, stored row-major with stride LDA and read by columns.
-// kuse: bit K set when the wave's products need the 16-wide k block K (k ascending,
-// as in the dense loop, so nothing changes where every block is used).
+// acc += A B (or A B^T) from LDS: A rows with stride lda<T>(); B row-major with stride
+// LDB, or, transposed, stored row-major with stride lda<T>() and read by columns.
+// kuse: bit K set when the wave's products need the 16-wide k block K (k ascending by
+// block, as in the dense loop, so nothing changes where every block is used).  Inside a
+// block, MFMA step k4 takes k = 4 lk + k4 of lane group lk, so that a lane reads its four
+// k of a row at once, 16 bytes at a time, on distinct banks (lda, LDB).
+template <typename T>
+__device__ __forceinline__ void read4(const T* p, T (&v)[4]) {
+    if constexpr (sizeof(T) == 4) {
+        const float4 x = *reinterpret_cast<const float4*>(p);
+        v[0] = x.x, v[1] = x.y, v[2] = x.z, v[3] = x.w;
+    } else {
+        const double2 x = *reinterpret_cast<const double2*>(p), y = *reinterpret_cast<const double2*>(p + 2);
+        v[0] = x.x, v[1] = x.y, v[2] = y.x, v[3] = y.y;
+    }
+}
 template <typename T, bool TB, typename acc_t>
-__device__ __forceinline__ void gemm_lds(acc_t (&acc)[2][2], const T* la, const T* lb, T sg, int wr, int wc,
-                                         int li, int lk, uint32_t kuse) {
-    for (int K = 0; K < 4; K++) {
-        if (!((kuse >> K) & 1u)) continue;  // wave-uniform
+__device__ __forceinline__ void gemm_lds_k(acc_t (&acc)[2][2], const T* la, const T* lb, int wr, int wc, int li,
+                                           int lk, int K) {
+    constexpr int LDA = lda<T>();
+    const int k0 = 16 * K + 4 * lk;
+    T af[2][4], bf[2][4];
 #pragma unroll
-        for (int k4 = 0; k4 < 4; k4++) {
-            const int k = 16 * K + 4 * k4 + lk;
-            T af[2], bf[2];
+    for (int m = 0; m < 2; m++) read4(la + (wr + m * 16 + li) * LDA + k0, af[m]);
 #pragma unroll
-            for (int m = 0; m < 2; m++) af[m] = sg * la[(wr + m * 16 + li) * LDA + k];
+    for (int n = 0; n < 2; n++) {
+        if constexpr (TB) {
+            read4(lb + (wc + n * 16 + li) * LDA + k0, bf[n]);
+        } else {
 #pragma unroll
-            for (int n = 0; n < 2; n++)
-                bf[n] = TB ? lb[(wc + n * 16 + li) * LDA + k] : lb[k * LDB + wc + n * 16 + li];
-#pragma unroll
-            for (int m = 0; m < 2; m++)
-#pragma unroll
-                for (int n = 0; n < 2; n++) acc[m][n] = MfmaOp<T>::mma(af[m], bf[n], acc[m][n]);
+            for (int k4 = 0; k4 < 4; k4++) bf[n][k4] = lb[(k0 + k4) * LDB + wc + n * 16 + li];
         }
+    }
+#pragma unroll
+    for (int k4 = 0; k4 < 4; k4++)
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int n = 0; n < 2; n++) acc[m][n] = MfmaOp<T>::mma(af[m][k4], bf[n][k4], acc[m][n]);
+}
+template <typename T, bool TB, typename acc_t>
+__device__ __forceinline__ void gemm_lds(acc_t (&acc)[2][2], const T* la, const T* lb, int wr, int wc, int li, int lk,
+                                         uint32_t kuse) {
+    if (kuse == 0xFu) {  // wave-uniform; the usual dense case reads ahead across the blocks
+#pragma unroll
+        for (int K = 0; K < 4; K++) gemm_lds_k<T, TB>(acc, la, lb, wr, wc, li, lk, K);
+    } else {
+#pragma unroll 1
+        for (int K = 0; K < 4; K++)
+            if ((kuse >> K) & 1u) gemm_lds_k<T, TB>(acc, la, lb, wr, wc, li, lk, K);
     }
 }
 
@@ -379,15 +489,15 @@ struct NoWait {
 template <bool COH, typename T, typename acc_t>
 __device__ __forceinline__ void add_tile(acc_t (&acc)[2][2], const T* __restrict__ X, bool neg, int wr, int wc,
                                          int li, int lk) {
+    acc_t x[2][2];
 #pragma unroll
     for (int m = 0; m < 2; m++)
 #pragma unroll
-        for (int n = 0; n < 2; n++)
+        for (int n = 0; n < 2; n++) x[m][n] = acc_load_global<COH>(X, wr + m * 16, wc + n * 16, li, lk);
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const T x = ld1c<COH>(X, (wr + m * 16 + MfmaOp<T>::row(lk, r)) * TS + wc + n * 16 + li);
-                acc[m][n][r] += neg ? -x : x;
-            }
+    for (int m = 0; m < 2; m++)
+#pragma unroll
+        for (int n = 0; n < 2; n++) acc[m][n] += neg ? -x[m][n] : x[m][n];
 }
 
 // TBOK: pairs may carry a transposed second operand (only L L^T factors have them; the
@@ -403,6 +513,7 @@ __device__ __attribute__((always_inline)) void gemm_task(T* __restrict__ pool, c
                           int out, char* lds_raw, uint32_t* out_mask, const Wait& wait, int add = -1,
                           bool add_neg = false, int fadd = -1, bool to_lds = false) {
     typedef typename MfmaOp<T>::acc_t acc_t;
+    constexpr int LDA = lda<T>();
     T* la = reinterpret_cast<T*>(lds_raw);
     T* lb = la + TS * LDA;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -414,12 +525,8 @@ __device__ __attribute__((always_inline)) void gemm_task(T* __restrict__ pool, c
 #pragma unroll
         for (int n = 0; n < 2; n++) {
             acc[m][n] = acc_t{0, 0, 0, 0};
-            if constexpr (ACC) {  // C += ... : start from the stored tile
-                const T* C0 = pool + (size_t)out * TE;
-#pragma unroll
-                for (int r = 0; r < 4; r++)
-                    acc[m][n][r] = C0[(wr + m * 16 + MfmaOp<T>::row(lk, r)) * TS + wc + n * 16 + li];
-            }
+            if constexpr (ACC)  // C += ... : start from the stored tile
+                acc[m][n] = acc_load_global<false>(pool + (size_t)out * TE, wr + m * 16, wc + n * 16, li, lk);
         }
     // A product is zero when either operand's mask is (B taken in (k, j) orientation).
     auto zero_product = [&](const Pair& q, uint32_t qa, uint32_t qb) {
@@ -439,7 +546,7 @@ __device__ __attribute__((always_inline)) void gemm_task(T* __restrict__ pool, c
     uint32_t sma = 0, smb = 0;
     // the added tile: 0 none or not seen yet, 1 ready (read after the loop), 2 in xr
     int add_state = 0;
-    T xr[2][2][4];
+    acc_t xr[2][2];
     const T* X = pool + (size_t)(add >= 0 ? add : 0) * TE;
     for (int s = 0; s < npairs; s++) {
         const Pair p = pairs[s];
@@ -459,33 +566,30 @@ __device__ __attribute__((always_inline)) void gemm_task(T* __restrict__ pool, c
                         for (int m = 0; m < 2; m++)
 #pragma unroll
                             for (int n = 0; n < 2; n++)
-#pragma unroll
-                                for (int r = 0; r < 4; r++)
-                                    xr[m][n][r] =
-                                        ld1c<COH>(X, (wr + m * 16 + MfmaOp<T>::row(lk, r)) * TS + wc + n * 16 + li);
+                                xr[m][n] = acc_load_global<COH>(X, wr + m * 16, wc + n * 16, li, lk);
                         add_state = 2;
                     }
                 }
             }
             wait.pair_masks(s, p, ma, mbs);
             if (zero_product(p, ma, mbs)) continue;  // every thread skips
-            seg_load<COH>(pool + (size_t)pair_a(p) * TE, ga, tid, !MASKS || seg_on(ma, tid));
-            seg_load<COH>(pool + (size_t)pair_b(p) * TE, gb, tid, !MASKS || seg_on(mbs, tid));
+            seg_load<COH>(pool + (size_t)pair_a(p) * TE, ga, tid, !MASKS || seg_on<T>(ma, tid));
+            seg_load<COH>(pool + (size_t)pair_b(p) * TE, gb, tid, !MASKS || seg_on<T>(mbs, tid));
         } else {
             ma = sma;
             mbs = smb;
         }
         if (!synced) __syncthreads();  // every wave is done reading the previous pair from LDS
-        seg_store(ga, la, LDA, tid, !MASKS || seg_on(ma, tid));
-        seg_store(gb, lb, tb ? LDA : LDB, tid, !MASKS || seg_on(mbs, tid));
+        seg_store(ga, la, LDA, tid, !MASKS || seg_on<T>(ma, tid), neg);
+        seg_store(gb, lb, tb ? LDA : LDB, tid, !MASKS || seg_on<T>(mbs, tid));
         staged = -1;
         for (int n = s + 1; STAGE && n < ready; n++) {
             const Pair q = pairs[n];
             uint32_t qa, qb;
             wait.pair_masks(n, q, qa, qb);
             if (zero_product(q, qa, qb)) continue;
-            seg_load<COH>(pool + (size_t)pair_a(q) * TE, ga, tid, !MASKS || seg_on(qa, tid));
-            seg_load<COH>(pool + (size_t)pair_b(q) * TE, gb, tid, !MASKS || seg_on(qb, tid));
+            seg_load<COH>(pool + (size_t)pair_a(q) * TE, ga, tid, !MASKS || seg_on<T>(qa, tid));
+            seg_load<COH>(pool + (size_t)pair_b(q) * TE, gb, tid, !MASKS || seg_on<T>(qb, tid));
             staged = n;
             sma = qa;
             smb = qb;
@@ -494,17 +598,14 @@ __device__ __attribute__((always_inline)) void gemm_task(T* __restrict__ pool, c
         __syncthreads();
         uint32_t kuse = 0xFu;
         if constexpr (MASKS) kuse = k_blocks_used(ma, tb ? mask_transpose(mbs) : mbs, wr >> 4, wc >> 4);
-        const T sg = neg ? T(-1) : T(1);
-        if (tb) gemm_lds<T, TBOK>(acc, la, lb, sg, wr, wc, li, lk, kuse);
-        else gemm_lds<T, false>(acc, la, lb, sg, wr, wc, li, lk, kuse);
+        if (tb) gemm_lds<T, TBOK>(acc, la, lb, wr, wc, li, lk, kuse);
+        else gemm_lds<T, false>(acc, la, lb, wr, wc, li, lk, kuse);
     }
     if (add_state == 2) {
 #pragma unroll
         for (int m = 0; m < 2; m++)
 #pragma unroll
-            for (int n = 0; n < 2; n++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) acc[m][n][r] += add_neg ? -xr[m][n][r] : xr[m][n][r];
+            for (int n = 0; n < 2; n++) acc[m][n] += add_neg ? -xr[m][n] : xr[m][n];
     } else if (add >= 0) {
         if (add_state == 0) {
             uint32_t m0, m1;
@@ -518,13 +619,10 @@ __device__ __attribute__((always_inline)) void gemm_task(T* __restrict__ pool, c
 #pragma unroll
     for (int m = 0; m < 2; m++)
 #pragma unroll
-        for (int n = 0; n < 2; n++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const T v = acc[m][n][r];
-                gst(&C[(wr + m * 16 + MfmaOp<T>::row(lk, r)) * TS + wc + n * 16 + li], v);
-                if constexpr (MASKS) nz[m][n] |= fabs(v) > T(MASK_TINY);
-            }
+        for (int n = 0; n < 2; n++) {
+            acc_store_global(acc[m][n], C, wr + m * 16, wc + n * 16, li, lk);
+            if constexpr (MASKS) nz[m][n] = acc_nonzero(acc[m][n], MASK_TINY);
+        }
     if constexpr (MASKS) {
         const uint32_t qm = quad_mask(nz, wr >> 4, wc >> 4);
         if (lane == 0) out_mask[w] = qm;
@@ -534,18 +632,18 @@ __device__ __attribute__((always_inline)) void gemm_task(T* __restrict__ pool, c
 #pragma unroll
         for (int m = 0; m < 2; m++)
 #pragma unroll
-            for (int n = 0; n < 2; n++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) la[(wr + m * 16 + MfmaOp<T>::row(lk, r)) * LDA + wc + n * 16 + li] = acc[m][n][r];
+            for (int n = 0; n < 2; n++) acc_store<T>(acc[m][n], la + (wr + m * 16) * LDA + wc + n * 16, LDA, li, lk);
     }
 }
 
 // bf16 experiment: FP32 tiles, operands rounded to bf16, FP32 accumulation
-// (v_mfma_f32_16x16x32_bf16: A[i][8q..8q+7] in lane i + 16q, same D layout).
+// (v_mfma_f32_16x16x32_bf16: A[i][8q..8q+7] in lane i + 16q, D as v_mfma_f32_16x16x4_f32;
+// B is passed first, as in MfmaOp<float>).
 template <bool TBOK = false, bool MASKS = true, typename Wait = NoWait, bool COH = false>
 __device__ __attribute__((always_inline)) void gemm_task_bf16(float* __restrict__ pool, const Pair* __restrict__ pairs,
                                       int npairs, int out, char* lds_raw, uint32_t* out_mask, const Wait& wait,
                                       int add = -1, bool add_neg = false, int fadd = -1) {
+    constexpr int LDA = lda<float>();
     float* la = reinterpret_cast<float*>(lds_raw);
     float* lb = la + TS * LDA;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -562,16 +660,10 @@ __device__ __attribute__((always_inline)) void gemm_task_bf16(float* __restrict_
         const int sa = pair_a(p), sb = pair_b(p);
         uint32_t ma, mbs;
         wait(s, p.fa, p.fb, sa, sb, ma, mbs);
-        if constexpr (MASKS) {
-            if (ma == 0 || mbs == 0) continue;  // a zero product: every thread skips
-            tile_to_lds_masked<COH>(pool + (size_t)sa * TE, la, LDA, tid, ma);
-            tile_to_lds_masked<COH>(pool + (size_t)sb * TE, lb, TBOK && tb ? LDA : LDB, tid, mbs);
-        } else {
-            tile_to_lds<COH>(pool + (size_t)sa * TE, la, LDA, tid);
-            tile_to_lds<COH>(pool + (size_t)sb * TE, lb, TBOK && tb ? LDA : LDB, tid);
-        }
+        if (MASKS && (ma == 0 || mbs == 0)) continue;  // a zero product: every thread skips
+        tile_to_lds<COH>(pool + (size_t)sa * TE, la, LDA, tid, MASKS ? ma : MASK_ALL, neg);
+        tile_to_lds<COH>(pool + (size_t)sb * TE, lb, TBOK && tb ? LDA : LDB, tid, MASKS ? mbs : MASK_ALL);
         __syncthreads();
-        const float sg = neg ? -1.f : 1.f;
         // B[k][j] at k * LDB + j, or (transposed operand) at j * LDA + k
         const int bsk = TBOK && tb ? 1 : LDB, bsj = TBOK && tb ? LDA : 1;
 #pragma unroll
@@ -581,7 +673,7 @@ __device__ __attribute__((always_inline)) void gemm_task_bf16(float* __restrict_
             for (int m = 0; m < 2; m++)
 #pragma unroll
                 for (int e = 0; e < 8; e++)
-                    af[m][e] = (__bf16)(sg * la[(wr + m * 16 + li) * LDA + kk * 32 + lk * 8 + e]);
+                    af[m][e] = (__bf16)la[(wr + m * 16 + li) * LDA + kk * 32 + lk * 8 + e];
 #pragma unroll
             for (int n = 0; n < 2; n++)
 #pragma unroll
@@ -591,7 +683,7 @@ __device__ __attribute__((always_inline)) void gemm_task_bf16(float* __restrict_
             for (int m = 0; m < 2; m++)
 #pragma unroll
                 for (int n = 0; n < 2; n++)
-                    acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[m], bf[n], acc[m][n], 0, 0, 0);
+                    acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[n], af[m], acc[m][n], 0, 0, 0);
         }
     }
     if (add >= 0) {  // the bf16 kernel's accumulator rows follow the f32 layout
@@ -605,34 +697,30 @@ __device__ __attribute__((always_inline)) void gemm_task_bf16(float* __restrict_
 #pragma unroll
     for (int m = 0; m < 2; m++)
 #pragma unroll
-        for (int n = 0; n < 2; n++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const float v = acc[m][n][r];
-                gst(&C[(wr + m * 16 + 4 * lk + r) * TS + wc + n * 16 + li], v);
-                if constexpr (MASKS) nz[m][n] |= fabsf(v) > float(MASK_TINY);
-            }
+        for (int n = 0; n < 2; n++) {
+            acc_store_global<float>(acc[m][n], C, wr + m * 16, wc + n * 16, li, lk);
+            if constexpr (MASKS) nz[m][n] = acc_nonzero(acc[m][n], MASK_TINY);
+        }
     if constexpr (MASKS) {
         const uint32_t qm = quad_mask(nz, wr >> 4, wc >> 4);
         if (lane == 0) out_mask[w] = qm;
     }
 }
 
-// Mask of a stored tile, by one workgroup: wave w covers block row w; lane l reads
-// row 16w + l/4 (and + 16 more rows each round), columns 16(l%4) .. +15.
+// Mask of a stored tile, by one workgroup: wave w returns the bits of block row w.
 template <typename T>
 __device__ inline uint32_t tile_mask(const T* __restrict__ g, int tid) {
-    const int lane = tid & 63, w = tid >> 6;
+    constexpr int L = TileVec<T>::LANES;
+    Seg<T> s;
+    seg_load(g, s, tid, true);
     bool any = false;
-    // the thread's segments: rows 16w + lane/4 (lanes cover rows 16w .. 16w+15), cols 16 * (lane % 4)
-    const T* p = g + (16 * w + (lane >> 2)) * TS + 16 * (lane & 3);
 #pragma unroll
-    for (int q = 0; q < 16; q++) any |= fabs((double)p[q]) > MASK_TINY;
+    for (int q = 0; q < TileVec<T>::NV; q++) any |= (double)vabsmax(s.v[q]) > MASK_TINY;
     const unsigned long long b = __ballot(any);
     uint32_t bits = 0;
 #pragma unroll
-    for (int J = 0; J < 4; J++)
-        if (b & (0x1111111111111111ull << J)) bits |= 1u << (4 * w + J);
+    for (int l = 0; l < 64; l += L / 4)  // L / 4 lanes hold the same block column
+        if (b & (((1ull << (L / 4)) - 1) << l)) bits |= 1u << (4 * (tid >> 6) + (l % L) / (L / 4));
     return bits;
 }
 
@@ -716,6 +804,7 @@ __device__ inline void bcast_row(const C* v, C* bro, int lane, int k, C* out) {
 // y_ij = -(sum_k l_ik y_kj) / l_ii).  UNIT skips the divisions by l_ii = 1.
 template <typename C, bool UNIT>
 __device__ inline void inv_lower_regs(const C* ls, C* y, C* bro, int lane, int w) {
+    constexpr int LDA = lda<C>();
 #pragma unroll
     for (int c = 0; c < 16; c++) y[c] = (16 * w + c == lane) ? C(1) : C(0);
 #pragma unroll 1
@@ -739,6 +828,7 @@ __device__ inline void inv_lower_regs(const C* ls, C* y, C* bro, int lane, int w
 // by 1/u_kk once final (inv_upper, MatrixStdDouble.cpp:2829-2866).
 template <typename C>
 __device__ inline void inv_upper_regs(const C* us, C* y, C* bro, int lane, int w) {
+    constexpr int LDA = lda<C>();
 #pragma unroll
     for (int c = 0; c < 16; c++) y[c] = (16 * w + c == lane) ? C(1) : C(0);
 #pragma unroll 1
@@ -779,13 +869,19 @@ __device__ __forceinline__ float wave_absmax(float x) {
 // entries as in the unblocked ludcmpSimple (MatrixStdDouble.cpp:2711-2784), clamped
 // the same way.  The dependent chain is 4 x 16 short in-wave steps plus 10 barriers,
 // instead of 64 barrier-separated steps and two 64-step inverse sweeps.
-constexpr int BS = 17;        // LDS row stride of a 16x16 block
-constexpr int BE = 16 * BS;   // LDS elements of a 16x16 block
+// LDS row stride and elements of a 16x16 block.  FP32: 16-byte rows, and both operand reads
+// of mm16 on distinct banks (20 li + 4 lk .. + 3, and 80 lk + li, mod 64); FP64: odd, for
+// 8-byte reads (two workgroups' blocks have to fit in a CU's LDS).
+template <typename C>
+constexpr int bs() { return sizeof(C) == 8 ? 17 : 20; }
+template <typename C>
+constexpr int be() { return 16 * bs<C>(); }
 
 // LDS elements (in the compute type) of lu_inv_blocked: the tile, 8 diagonal-block
 // inverses, 12 blocks of partial inverse products, 8 reduction slots, the 2 x 64
 // column scales of the Cholesky form, and one slot for the look-ahead's panel counter
-constexpr int lu_lds_elems() { return TS * LDA + 8 * BE + 12 * BE + 8 + 2 * TS + 1; }
+template <typename C>
+constexpr int lu_lds_elems() { return TS * lda<C>() + 8 * be<C>() + 12 * be<C>() + 8 + 2 * TS + 1; }
 
 // Lane k of each 16-lane row to every lane of that row (DPP row_newbcast).  A DPP
 // read of a lane that EXEC disables returns 0, so callers evaluate it where every
@@ -855,63 +951,74 @@ __device__ __forceinline__ void static_for(F&& f) {
     }
 }
 
-// acc += sg * A (16 x 4*KS) B (4*KS x 16), A and B row-major in LDS
-template <typename C, int KS>
-__device__ __forceinline__ void mm16(typename MfmaOp<C>::acc_t& acc, const C* pa, int lda, const C* pb,
-                                     int ldb, int li, int lk, C sg = C(1)) {
+// acc += sg * A (16 x 16) B (16 x 16), A and B row-major in LDS.  FP32: MFMA step s takes
+// k = 4 lk + s of lane group lk, so a lane reads its four k of A at once.
+template <typename C>
+__device__ __forceinline__ void mm16(typename MfmaOp<C>::acc_t& acc, const C* pa, int ldpa, const C* pb, int ldpb, int li,
+                                     int lk, C sg = C(1)) {
+    if constexpr (sizeof(C) == 4) {
+        C av[4], bv[4];
+        read4(pa + li * ldpa + 4 * lk, av);
 #pragma unroll
-    for (int s = 0; s < KS; s++)
-        acc = MfmaOp<C>::mma(sg * pa[li * lda + 4 * s + lk], pb[(4 * s + lk) * ldb + li], acc);
+        for (int s = 0; s < 4; s++) bv[s] = pb[(4 * lk + s) * ldpb + li];
+#pragma unroll
+        for (int s = 0; s < 4; s++) acc = MfmaOp<C>::mma(sg * av[s], bv[s], acc);
+    } else {
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+            acc = MfmaOp<C>::mma(sg * pa[li * ldpa + 4 * s + lk], pb[(4 * s + lk) * ldpb + li], acc);
+    }
 }
 
 template <typename C>
-__device__ __forceinline__ void st16(const typename MfmaOp<C>::acc_t& acc, C* pd, int ld, int li, int lk,
-                                     C sg = C(1)) {
-#pragma unroll
-    for (int r = 0; r < 4; r++) pd[MfmaOp<C>::row(lk, r) * ld + li] = sg * acc[r];
+__device__ __forceinline__ void st16(const typename MfmaOp<C>::acc_t& acc, C* pd, int ld, int li, int lk, C sg = C(1)) {
+    acc_store<C>(acc * sg, pd, ld, li, lk);
 }
 
-template <typename T, typename C>
-__device__ __forceinline__ void st16_global(const typename MfmaOp<C>::acc_t& acc, T* tile, int I, int J,
-                                            int li, int lk, C sg = C(1)) {
-#pragma unroll
-    for (int r = 0; r < 4; r++)
-        gst(&tile[(16 * I + MfmaOp<C>::row(lk, r)) * TS + 16 * J + li], T(sg * acc[r]));
+template <typename C>
+__device__ __forceinline__ void st16_global(const typename MfmaOp<C>::acc_t& acc, C* tile, int I, int J, int li, int lk,
+                                            C sg = C(1)) {
+    acc_store_global<C>(acc * sg, tile, 16 * I, 16 * J, li, lk);
 }
 
-// 16x16 block of LDS (stride ld) to global block (I, J) of a tile; 4 elements per lane
-template <typename T, typename C>
-__device__ __forceinline__ void blk_to_global(const C* pb, int ld, T* tile, int I, int J, int lane) {
+// the same with row i of the tile scaled by rs[i]
+template <typename C>
+__device__ __forceinline__ void st16_global_rs(typename MfmaOp<C>::acc_t acc, C* tile, int I, int J, int li, int lk, C sg,
+                                               const C* rs) {
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const int r = 4 * q + (lane >> 4), c = lane & 15;
-        gst(&tile[(16 * I + r) * TS + 16 * J + c], T(pb[r * ld + c]));
+    for (int r = 0; r < 4; r++) acc[r] = sg * acc[r] * rs[16 * I + MfmaOp<C>::row(li, lk, r)];
+    acc_store_global<C>(acc, tile, 16 * I, 16 * J, li, lk);
+}
+
+// Block (I, J) of a tile, written 16 bytes per lane (FP32: one store of the wave, FP64:
+// two), entry (r, c) of the block from elem(r, c).
+template <typename C, typename F>
+__device__ __forceinline__ void blk_store_global(C* tile, int I, int J, int lane, F&& elem) {
+    constexpr int PER = 16 / (int)sizeof(C), LR = 16 / PER;  // entries per store of a lane, lanes per row
+    typedef typename TileVec<C>::V V;
+#pragma unroll
+    for (int q = 0; q < 4 / PER; q++) {
+        const int r = q * (64 / LR) + lane / LR, c = PER * (lane % LR);
+        V v;
+        C* e = reinterpret_cast<C*>(&v);
+#pragma unroll
+        for (int k = 0; k < PER; k++) e[k] = elem(r, c + k);
+        gst16(tile, ((16 * I + r) * TS + 16 * J + c) * (int)sizeof(C), v);
     }
 }
-
-// the same two stores with row i of the tile scaled by rs[i] (rs == nullptr: none)
-template <typename T, typename C>
-__device__ __forceinline__ void st16_global_rs(const typename MfmaOp<C>::acc_t& acc, T* tile, int I, int J,
-                                               int li, int lk, C sg, const C* rs) {
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        const int row = 16 * I + MfmaOp<C>::row(lk, r);
-        gst(&tile[row * TS + 16 * J + li], T(sg * acc[r] * rs[row]));
-    }
+// 16x16 block of LDS (stride ld) to block (I, J) of a tile
+template <typename C>
+__device__ __forceinline__ void blk_to_global(const C* pb, int ld, C* tile, int I, int J, int lane) {
+    blk_store_global(tile, I, J, lane, [&](int r, int c) { return pb[r * ld + c]; });
 }
-template <typename T, typename C>
-__device__ __forceinline__ void blk_to_global_rs(const C* pb, int ld, T* tile, int I, int J, int lane, const C* rs) {
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const int r = 4 * q + (lane >> 4), c = lane & 15;
-        gst(&tile[(16 * I + r) * TS + 16 * J + c], T(pb[r * ld + c] * rs[16 * I + r]));
-    }
+// the same with row i of the tile scaled by rs[i]
+template <typename C>
+__device__ __forceinline__ void blk_to_global_rs(const C* pb, int ld, C* tile, int I, int J, int lane, const C* rs) {
+    blk_store_global(tile, I, J, lane, [&](int r, int c) { return pb[r * ld + c] * rs[16 * I + r]; });
 }
-
-template <typename T>
-__device__ __forceinline__ void zero_blk_global(T* tile, int I, int J, int lane) {
-#pragma unroll
-    for (int q = 0; q < 4; q++) gst(&tile[(16 * I + 4 * q + (lane >> 4)) * TS + 16 * J + (lane & 15)], T(0));
+template <typename C>
+__device__ __forceinline__ void zero_blk_global(C* tile, int I, int J, int lane) {
+    blk_store_global(tile, I, J, lane, [](int, int) { return C(0); });
 }
 
 // One wave factors the 16x16 diagonal block at (r0, r0) of the LDS tile a in place
@@ -952,6 +1059,7 @@ __device__ __forceinline__ void diag16_elim_f32(float (&x)[8], float (&y)[8], fl
 template <typename C, bool CHOL = false>
 __device__ inline void diag16(C* a, int r0, C* xd, C* zd, int lane) {
     static_assert(sizeof(C) == 4, "FP32 only; FP64 tiles use diag16_split");
+    constexpr int LDA = lda<C>(), BS = bs<C>();
     const int i = lane & 15, h = lane >> 5;
     const bool colw = (lane >> 4) & 1;
     const int rs = colw ? 1 : LDA, cs = colw ? LDA : 1;
@@ -990,6 +1098,7 @@ __device__ inline void diag16(C* a, int r0, C* xd, C* zd, int lane) {
 // the same instructions (forward substitution, 1/u_ii scaling deferred to the end).
 template <typename C, bool CHOL = false>
 __device__ inline void diag16_split(C* a, int r0, C* xd, C* zd, int lane) {
+    constexpr int LDA = lda<C>(), BS = bs<C>();
     const int i = lane & 15, g = lane >> 4;
     C v[16];
 #pragma unroll
@@ -1036,34 +1145,28 @@ __device__ inline void diag16_split(C* a, int r0, C* xd, C* zd, int lane) {
     }
 }
 
-// Factor blocks of the LDS tile a (row stride LDA) to global block (I, J) of L or U,
-// 4 elements per lane (rows 4q + lane/16, column lane%16).  L (I >= J): the strict
-// lower part of a, 1 on the diagonal, 0 above; CHOL: L_u diag(d) with d = dsc.
-// U (I <= J): a on and above the diagonal (the clamped pivots on it), 0 below; um
-// collects max |u| for the growth check.
-template <typename T, typename C, bool CHOL>
-__device__ __forceinline__ void l_blk_to_global(const C* a, T* Lg, int I, int J, int lane, const C* dsc) {
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const int r = 4 * q + (lane >> 4), c = lane & 15;
-        const int gr = 16 * I + r, gc = 16 * J + c;
-        const C x = a[gr * LDA + gc];
+// Factor blocks of the LDS tile a (row stride lda) to global block (I, J) of L or U.
+// L (I >= J): the strict lower part of a, 1 on the diagonal, 0 above; CHOL: L_u diag(d)
+// with d = dsc.  U (I <= J): a on and above the diagonal (the clamped pivots on it), 0
+// below; um collects max |u| for the growth check.
+template <typename C, bool CHOL>
+__device__ __forceinline__ void l_blk_to_global(const C* a, C* Lg, int I, int J, int lane, const C* dsc) {
+    blk_store_global(Lg, I, J, lane, [&](int r, int c) {
+        const int gc = 16 * J + c;
+        const C x = a[(16 * I + r) * lda<C>() + gc];
         C v = (I > J || r > c) ? x : (r == c ? C(1) : C(0));
         if constexpr (CHOL) v = (I == J && r == c) ? dsc[gc] : v * dsc[gc];
-        gst(&Lg[gr * TS + gc], T(v));
-    }
+        return v;
+    });
 }
-template <typename T, typename C>
-__device__ __forceinline__ void u_blk_to_global(const C* a, T* Ug, int I, int J, int lane, C& um) {
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const int r = 4 * q + (lane >> 4), c = lane & 15;
-        const int gr = 16 * I + r, gc = 16 * J + c;
-        const C x = a[gr * LDA + gc];
+template <typename C>
+__device__ __forceinline__ void u_blk_to_global(const C* a, C* Ug, int I, int J, int lane, C& um) {
+    blk_store_global(Ug, I, J, lane, [&](int r, int c) {
+        const C x = a[(16 * I + r) * lda<C>() + 16 * J + c];
         const C v = (I < J || c >= r) ? x : C(0);
-        gst(&Ug[gr * TS + gc], T(v));
         um = fabs(v) > um ? fabs(v) : um;
-    }
+        return v;
+    });
 }
 
 // LU of one tile in compute type C plus, when their slots are given (>= 0), the
@@ -1083,8 +1186,8 @@ __device__ __forceinline__ void u_blk_to_global(const C* a, T* Ug, int I, int J,
 // accumulated term by term as the factors of column / row K appear (N and M live in
 // LDS; X_IJ and Z_IJ replace them once complete).  After block 3, X_3J and Z_I3 take
 // one product each, spread over the four waves.
-template <typename T, typename C, bool CHOL = false>
-__device__ __attribute__((always_inline)) void lu_inv_blocked(T* __restrict__ pool, int src, int outl, int outu,
+template <typename C, bool CHOL = false>
+__device__ __attribute__((always_inline)) void lu_inv_blocked(C* __restrict__ pool, int src, int outl, int outu,
                                                               int outli, int outui, char* lds_raw,
                                                               float* amax_out, float* umax_out, bool coh = false,
                                                               C* xcopy = nullptr, C* zcopy = nullptr, bool in_lds = false) {
@@ -1097,6 +1200,7 @@ __device__ __attribute__((always_inline)) void lu_inv_blocked(T* __restrict__ po
     // instead of being hoisted out of the step loop and held in registers throughout
     // (wave 0's own loop-invariant values stay hoisted).
     int bl = lane, bli = li, blk = lk;
+    constexpr int LDA = lda<C>(), BS = bs<C>(), BE = be<C>();
     C* a = reinterpret_cast<C*>(lds_raw);  // the tile, row stride LDA
     C* xd = a + TS * LDA;                  // X_II = L_II^-1, I = 0..3
     C* zd = xd + 4 * BE;                   // Z_II = U_II^-1
@@ -1105,27 +1209,22 @@ __device__ __attribute__((always_inline)) void lu_inv_blocked(T* __restrict__ po
     C* dsc = red + 8;                      // CHOL: d_j = sqrt(u_jj), then 1 / d_j
     int* pcnt = reinterpret_cast<int*>(dsc + 2 * TS);  // panel blocks written (look-ahead)
     enum { N10, N20, N30, N21, N31, N32, M01, M02, M03, M12, M13, M23 };
-    T* Lg = pool + (size_t)outl * TE;
-    T* Ug = (!CHOL && outu >= 0) ? pool + (size_t)outu * TE : nullptr;
-    T* Xg = outli >= 0 ? pool + (size_t)outli * TE : nullptr;
-    T* Zg = (!CHOL && outui >= 0) ? pool + (size_t)outui * TE : nullptr;
+    C* Lg = pool + (size_t)outl * TE;
+    C* Ug = (!CHOL && outu >= 0) ? pool + (size_t)outu * TE : nullptr;
+    C* Xg = outli >= 0 ? pool + (size_t)outli * TE : nullptr;
+    C* Zg = (!CHOL && outui >= 0) ? pool + (size_t)outui * TE : nullptr;
     auto ablk = [&](int I, int J) { return a + 16 * I * LDA + 16 * J; };
     auto slot = [&](int s) { return nm + s * BE; };
-    auto ldacc = [&](const C* p) {
-        acc_t acc;
-#pragma unroll
-        for (int r = 0; r < 4; r++) acc[r] = p[MfmaOp<C>::row(blk, r) * BS + bli];
-        return acc;
-    };
+    auto ldacc = [&](const C* p) { return acc_load<C>(p, BS, bli, blk); };
     // N_s (+)= L_IK X and M_s (+)= Z U_KJ, X and Z blocks of row stride BS
     auto n_add = [&](int s, bool first, int I, int K, const C* X) {
         acc_t acc = first ? acc_t{0, 0, 0, 0} : ldacc(slot(s));
-        mm16<C, 4>(acc, ablk(I, K), LDA, X, BS, bli, blk);
+        mm16<C>(acc, ablk(I, K), LDA, X, BS, bli, blk);
         st16(acc, slot(s), BS, bli, blk);
     };
     auto m_add = [&](int s, bool first, const C* Z, int K, int J) {
         acc_t acc = first ? acc_t{0, 0, 0, 0} : ldacc(slot(s));
-        mm16<C, 4>(acc, Z, BS, ablk(K, J), LDA, bli, blk);
+        mm16<C>(acc, Z, BS, ablk(K, J), LDA, bli, blk);
         st16(acc, slot(s), BS, bli, blk);
     };
     // X_IJ = -X_II N_IJ and Z_IJ = -M_IJ Z_JJ to HBM, and in place over N / M (keep)
@@ -1134,7 +1233,7 @@ __device__ __attribute__((always_inline)) void lu_inv_blocked(T* __restrict__ po
     const bool cpx = !CHOL && xcopy, cpz = !CHOL && zcopy;
     auto x_fin = [&](int s, int I, int J, bool keep) {
         acc_t acc = acc_t{0, 0, 0, 0};
-        mm16<C, 4>(acc, xd + I * BE, BS, slot(s), BS, bli, blk);
+        mm16<C>(acc, xd + I * BE, BS, slot(s), BS, bli, blk);
         if (keep) st16(acc, slot(s), BS, bli, blk, C(-1));
         if constexpr (CHOL) st16_global_rs(acc, Xg, I, J, bli, blk, C(-1), (const C*)(dsc + TS));
         else st16_global(acc, Xg, I, J, bli, blk, C(-1));
@@ -1142,17 +1241,21 @@ __device__ __attribute__((always_inline)) void lu_inv_blocked(T* __restrict__ po
     };
     auto z_fin = [&](int s, int I, int J, bool keep) {
         acc_t acc = acc_t{0, 0, 0, 0};
-        mm16<C, 4>(acc, slot(s), BS, zd + J * BE, BS, bli, blk);
+        mm16<C>(acc, slot(s), BS, zd + J * BE, BS, bli, blk);
         if (keep) st16(acc, slot(s), BS, bli, blk, C(-1));
         st16_global(acc, Zg, I, J, bli, blk, C(-1));
         if (cpz) st16(acc, zcopy + 16 * I * LDB + 16 * J, LDB, bli, blk, C(-1));
     };
     // 16x16 block (I, J) of a copy: from an LDS block of stride BS, or zeros
     auto cp_blk = [&](C* cp, const C* pb, int I, int J, int ld) {
+        typedef typename TileVec<C>::V V;
+        constexpr int PER = TileVec<C>::PER, LR = 16 / PER;
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int r = 4 * q + (bl >> 4), c = bl & 15;
-            cp[(16 * I + r) * ld + 16 * J + c] = pb ? pb[r * BS + c] : C(0);
+        for (int q = 0; q < 4 / PER; q++) {
+            const int r = q * (64 / LR) + bl / LR, c = PER * (bl % LR);
+            V v{};
+            if (pb) v = *reinterpret_cast<const V*>(pb + r * BS + c);
+            *reinterpret_cast<V*>(cp + (16 * I + r) * ld + 16 * J + c) = v;
         }
     };
     // block column K of L, block row K of U, the diagonal blocks of X and Z, and the zero
@@ -1160,11 +1263,11 @@ __device__ __attribute__((always_inline)) void lu_inv_blocked(T* __restrict__ po
     // diagonal blocks and U and U^-1 below, are stored by waves 1-3 while wave 0 factors
     // diagonal block 0)
     auto l_col = [&](int K) {
-        for (int I = K; I < 4; I++) l_blk_to_global<T, C, CHOL>(a, Lg, I, K, bl, dsc);
+        for (int I = K; I < 4; I++) l_blk_to_global<C, CHOL>(a, Lg, I, K, bl, dsc);
     };
     C um = 0;
     auto u_row = [&](int K) {
-        for (int J = K; J < 4; J++) u_blk_to_global<T, C>(a, Ug, K, J, bl, um);
+        for (int J = K; J < 4; J++) u_blk_to_global<C>(a, Ug, K, J, bl, um);
     };
     auto inv_diag = [&](int K) {
         if (Xg) {
@@ -1184,28 +1287,26 @@ __device__ __attribute__((always_inline)) void lu_inv_blocked(T* __restrict__ po
         }
     };
     {
-        const T* A = pool + (size_t)src * TE;
-        const int r = tid >> 2, c0 = (tid & 3) * 16;
+        typedef typename TileVec<C>::V V;
         if (tid == 0) *pcnt = 0;
         C m = 0;
+        Seg<C> av;
         if (in_lds) {  // the GEMM that made the source left it in a (CHOL: mirrored below)
+            if (amax_out) {
 #pragma unroll
-            for (int q = 0; q < 16; q++) {
-                const C x = a[r * LDA + c0 + q];
-                m = fabs(x) > m ? fabs(x) : m;
+                for (int q = 0; q < TileVec<C>::NV; q++)
+                    m = fmax(m, vabsmax(*reinterpret_cast<const V*>(a + vec_row<C>(q, tid) * LDA + vec_col<C>(tid))));
             }
         } else {
-            C av[16];
-            load16(A, r * TS + c0, coh, av);
+            const C* A = pool + (size_t)src * TE;
+            if (coh) seg_load<true>(A, av, tid, true);
+            else seg_load<false>(A, av, tid, true);
+            seg_store(av, a, LDA, tid, true);
 #pragma unroll
-            for (int q = 0; q < 16; q++) {
-                const int c = c0 + q;
-                const C x = av[q];
-                a[r * LDA + c] = x;
-                m = fabs(x) > m ? fabs(x) : m;
-            }
+            for (int q = 0; q < TileVec<C>::NV; q++) m = fmax(m, vabsmax(av.v[q]));
         }
         if constexpr (CHOL) {  // only the lower triangle is read: mirror it
+            const int r = tid >> 2, c0 = (tid & 3) * 16;
             __syncthreads();
 #pragma unroll
             for (int q = 0; q < 16; q++) {
@@ -1237,21 +1338,19 @@ __device__ __attribute__((always_inline)) void lu_inv_blocked(T* __restrict__ po
     auto u_panel = [&](int K, int J, int ci, int ck) {
         acc_t acc = acc_t{0, 0, 0, 0};
         C* d = ablk(K, J);
-        mm16<C, 4>(acc, xd + K * BE, BS, d, LDA, ci, ck);
+        mm16<C>(acc, xd + K * BE, BS, d, LDA, ci, ck);
         st16(acc, d, LDA, ci, ck);
     };
     auto l_panel = [&](int I, int K, int ci, int ck) {
         acc_t acc = acc_t{0, 0, 0, 0};
         C* d = ablk(I, K);
-        mm16<C, 4>(acc, d, LDA, zd + K * BE, BS, ci, ck);
+        mm16<C>(acc, d, LDA, zd + K * BE, BS, ci, ck);
         st16(acc, d, LDA, ci, ck);
     };
     auto trail = [&](int I, int J, int K, int ci, int ck) {
         C* d = ablk(I, J);
-        acc_t acc;
-#pragma unroll
-        for (int r = 0; r < 4; r++) acc[r] = d[MfmaOp<C>::row(ck, r) * LDA + ci];
-        mm16<C, 4>(acc, ablk(I, K), LDA, ablk(K, J), LDA, ci, ck, C(-1));
+        acc_t acc = acc_load<C>(d, LDA, ci, ck);
+        mm16<C>(acc, ablk(I, K), LDA, ablk(K, J), LDA, ci, ck, C(-1));
         st16(acc, d, LDA, ci, ck);
     };
     // Panel blocks of step K written by all four waves: each wave adds 1 to the LDS
@@ -1278,7 +1377,7 @@ __device__ __attribute__((always_inline)) void lu_inv_blocked(T* __restrict__ po
         // transpose of U and U^-1), 8 per wave; the tile is in LDS, so an output slot that
         // is the source's as well is not read again
         for (int e = w - 1; e < 24; e += 3) {
-            T* const o = e < 6 ? Lg : (e < 12 ? Xg : (e < 18 ? Ug : Zg));
+            C* const o = e < 6 ? Lg : (e < 12 ? Xg : (e < 18 ? Ug : Zg));
             const int q = e % 6, K = q < 3 ? 0 : (q < 5 ? 1 : 2), J = q < 3 ? q + 1 : (q < 5 ? q - 1 : 3);
             if (o) zero_blk_global(o, e < 12 ? K : J, e < 12 ? J : K, lane);
         }
@@ -1417,15 +1516,22 @@ __device__ inline void lu_inv_fp64_lds(T* __restrict__ pool, int src, int outl, 
                                        int outui, char* lds_raw, bool coh) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
+    constexpr int LDA = lda<double>();
     double* a = reinterpret_cast<double*>(lds_raw);
     double* lcol = a + TS * LDA;
     const T* A = pool + (size_t)src * TE;
     const int i = tid >> 2, j0 = (tid & 3) * 16;
     {
-        double av[16];
-        load16(A, i * TS + j0, coh, av);
+        Seg<T> av;
+        if (coh) seg_load<true>(A, av, tid, true);
+        else seg_load<false>(A, av, tid, true);
+        constexpr int PER = TileVec<T>::PER;
 #pragma unroll
-        for (int q = 0; q < 16; q++) a[i * LDA + j0 + q] = av[q];
+        for (int q = 0; q < TileVec<T>::NV; q++) {
+            const T* e = reinterpret_cast<const T*>(&av.v[q]);
+#pragma unroll
+            for (int k = 0; k < PER; k++) a[vec_row<T>(q, tid) * LDA + vec_col<T>(tid) + k] = e[k];
+        }
     }
     __syncthreads();
     const double TINY2 = 1e-9;
@@ -1482,12 +1588,11 @@ __device__ __attribute__((always_inline)) double lu_task(T* __restrict__ pool, i
                           char* lds_raw, double growth_limit, int* n_fp64, bool coh = false,
                           float* xcopy = nullptr, float* zcopy = nullptr, bool in_lds = false) {
     if constexpr (sizeof(T) == 8) {
-        lu_inv_blocked<T, double>(pool, src, outl, outu, outli, outui, lds_raw, nullptr, nullptr, coh, nullptr, nullptr,
-                                  in_lds);
+        lu_inv_blocked<T>(pool, src, outl, outu, outli, outui, lds_raw, nullptr, nullptr, coh, nullptr, nullptr, in_lds);
         return 1.0;
     } else {
         float amax = 0, umax = 0;
-        lu_inv_blocked<T, float>(pool, src, outl, outu, outli, outui, lds_raw, &amax, &umax, coh, xcopy, zcopy, in_lds);
+        lu_inv_blocked<T>(pool, src, outl, outu, outli, outui, lds_raw, &amax, &umax, coh, xcopy, zcopy, in_lds);
         const double growth = amax > 0 ? (double)umax / (double)amax : 1.0;
         if (!(growth <= growth_limit)) {
             __syncthreads();
@@ -1504,6 +1609,7 @@ __device__ __attribute__((always_inline)) void tri_inv_task(T* __restrict__ pool
     typedef typename std::conditional<sizeof(T) == 8, double, float>::type C;
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
+    constexpr int LDA = lda<C>();
     C* ts = reinterpret_cast<C*>(lds_raw);
     C* bro = ts + TS * LDA + 16 * w;
     C v[16];
@@ -1523,35 +1629,32 @@ __device__ __attribute__((always_inline)) void tri_inv_task(T* __restrict__ pool
 template <typename T>
 __device__ __attribute__((always_inline)) void llt_task(T* __restrict__ pool, int src, int out, int outinv,
                                                         char* lds_raw, bool coh = false, bool in_lds = false) {
-    typedef typename std::conditional<sizeof(T) == 8, double, float>::type C;
-    lu_inv_blocked<T, C, true>(pool, src, out, -1, outinv, -1, lds_raw, nullptr, nullptr, coh, nullptr, nullptr, in_lds);
+    lu_inv_blocked<T, true>(pool, src, out, -1, outinv, -1, lds_raw, nullptr, nullptr, coh, nullptr, nullptr, in_lds);
 }
 
-// R = A^T through LDS (odd row stride: the column reads hit distinct banks); wave w
-// leaves the mask bits of block row w of R in out_mask[w].
+// R = A^T through LDS; wave w leaves the mask bits of the rows it wrote in out_mask[w].
 template <typename T, bool MASKS = true, bool COH = false>
 __device__ __attribute__((always_inline)) void trans_task(T* __restrict__ pool, int src, int out, char* lds_raw,
                                                           uint32_t* out_mask) {
+    constexpr int LDA = lda<T>();
     T* s = reinterpret_cast<T*>(lds_raw);
     const int tid = threadIdx.x, lane = tid & 63;
-    const int r = tid >> 2, c0 = (tid & 3) * 16;
     tile_to_lds<COH>(pool + (size_t)src * TE, s, LDA, tid);
     __syncthreads();
     T* R = pool + (size_t)out * TE;
-    bool any = false;
-#pragma unroll
-    for (int q = 0; q < 16; q++) {
-        const T v = s[(c0 + q) * LDA + r];
-        gst(&R[r * TS + c0 + q], v);
-        any |= fabs(v) > T(MASK_TINY);
-    }
-    if constexpr (!MASKS) return;
-    const unsigned long long b = __ballot(any);  // lane l: block (w, l % 4)
     uint32_t bits = 0;
 #pragma unroll
-    for (int J = 0; J < 4; J++)
-        if (b & (0x1111111111111111ull << J)) bits |= 1u << (4 * (tid >> 6) + J);
-    if (lane == 0) out_mask[tid >> 6] = bits;
+    for (int q = 0; q < TS / 4; q++) {  // row 4q + wave, column lane, as sub_task
+        const T v = s[lane * LDA + 4 * q + (tid >> 6)];
+        gst(&R[q * NT + tid], v);
+        if constexpr (MASKS) {
+            const unsigned long long bb = __ballot(fabs(v) > T(MASK_TINY));
+#pragma unroll
+            for (int J = 0; J < 4; J++)
+                if (bb & (0xFFFFull << (16 * J))) bits |= 1u << (4 * (q >> 2) + J);
+        }
+    }
+    if (MASKS && lane == 0) out_mask[tid >> 6] = bits;
 }
 
 }  // namespace sogl_dev
