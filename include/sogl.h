@@ -231,9 +231,17 @@ int sogl_ctx_set_task_links(sogl_ctx* ctx, int32_t links);
  * builds whatever the context's setting. */
 int sogl_graph_check(const sogl_factor_desc* desc, int64_t* info);
 int sogl_graph_check_plan(const sogl_plan* plan, int32_t precision, int64_t* info);
-/* Convenience: sogl_factor_load from a host plan. */
+/* sogl_factor_load from a host plan.  The factorisation is the plan's, tile for tile, in
+ * tile-column order (sogl_tile_order_ops) where the plan allows it, else by the plan's own
+ * op list; sogl_graph_check_plan looks at the latter. */
 int sogl_factor_load_plan(sogl_ctx* ctx, const sogl_plan* plan, int32_t precision,
                           int32_t* factor_id);
+/* The op list sogl_factor_load_plan factors a plan by: for every block row the sum of its
+ * updates, the lu (or llt) and the panels, over the plan's input and factor tile ids and
+ * new ids (up to *n_ids) for the sums and the diagonal inverses.  L and U are those of the
+ * plan's list up to rounding.  ops may be NULL to ask for the count; n_ops receives 0 where
+ * the plan keeps its own list.  No reference counterpart. */
+int sogl_tile_order_ops(const sogl_plan* plan, sogl_op* ops, int64_t* n_ops, int32_t* n_ids);
 /* Factor on the device: replaces BlockPlanner::calculate() (BlockPlanner.cpp:376-651),
  * called from decompose_solveLU (solver.cpp:106).  Re-running refactors from the
  * resident input tiles. */

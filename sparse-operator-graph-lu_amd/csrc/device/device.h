@@ -11,6 +11,27 @@
 
 #include "../../../include/sogl.h"
 
+namespace sogl {
+// What a plan holds beyond its factor description (plan_capi.cpp).
+struct PlanView {
+    int32_t n;
+    int64_t N;
+    const int32_t* new_order;
+    int64_t nnz;
+    const int32_t* row;
+    const int32_t* col;
+    const double* val;
+    int64_t nnz_orig;  // entries of the original matrix (the rest is padding)
+    int64_t n_inputs;  // input tiles: block coordinates and cells (position row*64+col, value)
+    const int32_t* in_bi;
+    const int32_t* in_bj;
+    const int64_t* cell_begin;
+    const uint16_t* cell_pos;
+    const double* cell_val;
+};
+bool plan_view(const sogl_plan* p, PlanView* v);
+}  // namespace sogl
+
 namespace sogl_dev {
 
 struct Pair;  // tile_ops.h
@@ -109,6 +130,7 @@ struct Factor {
     bool absorb_panels = false;            // let lu tasks absorb a panel GEMM (set from the context)
     int64_t n_absorbed = 0;                // panel GEMMs absorbed by their lu task
     int64_t n_after = 0;                   // after-links (tasks run by their producer's workgroup)
+    bool tile_order = false;               // the op list is in tile-column order (tile_order.h)
     std::vector<int32_t> chain_head;       // per task: the queued task whose workgroup runs it
     int32_t chain_claims = 0;              // persistent executor: claims per finished task (0: off)
     std::vector<int32_t> queue;            // persistent executor: task indices handed out, in order

@@ -24,11 +24,13 @@
 #include <cstring>
 #include <deque>
 #include <map>
+#include <new>
 #include <string>
 #include <vector>
 
 #include "device.h"
 #include "tile_ops.h"
+#include "tile_order.h"
 
 namespace sogl {
 void set_last_error(const std::string& s);
@@ -895,11 +897,13 @@ constexpr double CHAIN_SLACK_US = 1.0;
 
 // The cost model of the critical path (microseconds, measured on the C2 / C5 factors):
 // task work, and a hand-off per edge that no chain link removes.
-double task_cost_us(const DevTask& k) {
+// In tile-column order a sum's pairs but the last are ready, and multiplied, while its
+// workgroup waits for that one.
+double task_cost_us(const DevTask& k, bool tile_order) {
     switch (k.kind) {
         case TK_LU: case TK_LLT: return 10.0;
         case TK_LINV: case TK_UINV: return 5.0;
-        case TK_GEMM: return 0.8 + 0.5 * k.b + (k.add >= 0 ? 0.2 : 0.0);
+        case TK_GEMM: return 0.8 + 0.5 * (tile_order ? std::min(k.b, 1) : k.b) + (k.add >= 0 ? 0.2 : 0.0);
         default: return 1.0;
     }
 }
@@ -918,7 +922,7 @@ void build_chains(Factor* f, HostGraph& hg) {
     for (size_t t = 0; t < T; t++)
         for (int32_t o : {f->tasks[t].out0, f->tasks[t].out1, f->tasks[t].out2, f->tasks[t].out3})
             if (o >= 0) slot_task[(size_t)o] = (int32_t)t;
-    auto cost = [&](const DevTask& k) { return task_cost_us(k); };
+    auto cost = [&](const DevTask& k) { return task_cost_us(k, f->tile_order); };
     auto edge = [&](size_t p, size_t t) { return f->tasks[p].next == (int32_t)t ? 0.0 : HANDOFF_US; };
     std::vector<double> tl(T, 0.0), bl(T, 0.0);
     std::vector<std::vector<int32_t>> succ(T);
@@ -1042,6 +1046,7 @@ void build_after_links(Factor* f, const HostGraph& hg, std::vector<char>& linked
     for (size_t t = 0; t < T; t++)
         for (int32_t o : {f->tasks[t].out0, f->tasks[t].out1, f->tasks[t].out2, f->tasks[t].out3})
             if (o >= 0) slot_task[(size_t)o] = (int32_t)t;
+    auto cost = [&](const DevTask& k) { return task_cost_us(k, f->tile_order); };
     auto edge = [&](size_t p, size_t t) { return f->tasks[p].next == (int32_t)t ? 0.0 : HANDOFF_US; };
     std::vector<double> fin(T, 0.0), bl(T, 0.0);  // earliest finish, longest path to the end
     std::vector<int32_t> crit(T, -1);              // the predecessor that finishes last
@@ -1059,17 +1064,17 @@ void build_after_links(Factor* f, const HostGraph& hg, std::vector<char>& linked
             }
             if (succ[(size_t)p].empty() || succ[(size_t)p].back() != (int32_t)t) succ[(size_t)p].push_back((int32_t)t);
         }
-        fin[t] = st + task_cost_us(k);
+        fin[t] = st + cost(k);
     }
     double cp = 0;
     for (size_t t = T; t-- > 0;) {
         double b = 0;
         for (int32_t u : succ[t]) b = std::max(b, edge(t, (size_t)u) + bl[(size_t)u]);
-        bl[t] = task_cost_us(f->tasks[t]) + b;
-        cp = std::max(cp, fin[t] - task_cost_us(f->tasks[t]) + bl[t]);
+        bl[t] = cost(f->tasks[t]) + b;
+        cp = std::max(cp, fin[t] - cost(f->tasks[t]) + bl[t]);
     }
     // slack of task t: the longest path minus the longest path through t
-    auto slack = [&](size_t t) { return cp - (fin[t] - task_cost_us(f->tasks[t]) + bl[t]); };
+    auto slack = [&](size_t t) { return cp - (fin[t] - cost(f->tasks[t]) + bl[t]); };
     std::vector<int32_t> head(T, -1), len(T, 0), pred(T, -1);
     std::vector<char> absorbed(T, 0);
     // every producer of u's operands other than t is an earlier task of t's chain or
@@ -2595,7 +2600,8 @@ extern "C" int sogl_ctx_sync(sogl_ctx* x) {
 
 namespace {
 // Loads a factor whose input tiles are dense (desc) or cells (plan storage).
-int load_factor(sogl_ctx* x, const sogl_factor_desc* d, const InputCells* cells, int32_t* factor_id) {
+int load_factor(sogl_ctx* x, const sogl_factor_desc* d, const InputCells* cells, int32_t* factor_id,
+                bool tile_order = false) {
     if (!x || !d || !factor_id) return set_error(x ? &x->c : nullptr, SOGL_ERR_ARG, "null argument");
     Context* c = &x->c;
     std::lock_guard<std::mutex> g(c->mu);
@@ -2608,6 +2614,7 @@ int load_factor(sogl_ctx* x, const sogl_factor_desc* d, const InputCells* cells,
     Factor* f = new Factor();
     f->precision = d->precision;
     f->elem = d->precision == SOGL_FP64 ? 8 : 4;
+    f->tile_order = tile_order;
     int rc = build_graph(c, d, cells, f);
     if (rc != SOGL_OK) {
         free_factor(f);
@@ -2689,6 +2696,34 @@ extern "C" int sogl_ctx_set_pool_reuse(sogl_ctx* x, int32_t mode) {
     return SOGL_OK;
 }
 
+namespace {
+// the factorisation the plan describes, in tile-column order (tile_order.h)
+bool plan_tile_order(const sogl_plan* plan, const sogl_factor_desc* d, TileOrderOps& to) {
+    sogl::PlanView pv;
+    try {
+        return sogl::plan_view(plan, &pv) && tile_order_ops(d, pv.in_bi, pv.in_bj, to);
+    } catch (const std::bad_alloc&) {  // no host memory for a second list: the plan's own
+        return false;
+    }
+}
+}  // namespace
+
+extern "C" int sogl_tile_order_ops(const sogl_plan* plan, sogl_op* ops, int64_t* n_ops, int32_t* n_ids) {
+    sogl_factor_desc d;
+    if (!n_ops || !n_ids || !sogl::plan_factor_desc(plan, SOGL_FP64, &d))
+        return set_error(nullptr, SOGL_ERR_ARG, "null argument");
+    TileOrderOps to;
+    if (!plan_tile_order(plan, &d, to)) {
+        *n_ops = 0;
+        *n_ids = 0;
+        return SOGL_OK;
+    }
+    if (ops) std::copy(to.ops.begin(), to.ops.end(), ops);
+    *n_ops = (int64_t)to.ops.size();
+    *n_ids = to.n_ids;
+    return SOGL_OK;
+}
+
 extern "C" int sogl_factor_load_plan(sogl_ctx* x, const sogl_plan* plan, int32_t precision,
                                      int32_t* factor_id) {
     sogl_factor_desc d;
@@ -2696,7 +2731,14 @@ extern "C" int sogl_factor_load_plan(sogl_ctx* x, const sogl_plan* plan, int32_t
     if (!sogl::plan_factor_desc(plan, precision, &d) ||
         !sogl::plan_input_cells(plan, &cells.begin, &cells.pos, &cells.val))
         return set_error(x ? &x->c : nullptr, SOGL_ERR_ARG, "null plan");
-    return load_factor(x, &d, &cells, factor_id);
+    TileOrderOps to;
+    const bool tile_order = plan_tile_order(plan, &d, to);
+    if (tile_order) {
+        d.ops = to.ops.data();
+        d.n_ops = (int64_t)to.ops.size();
+        d.n_ids = to.n_ids;
+    }
+    return load_factor(x, &d, &cells, factor_id, tile_order);
 }
 
 namespace sogl_dev {

@@ -126,23 +126,6 @@ void reduce_norms(const std::vector<double>& part, int c, double out[RED_VALUES]
 }  // namespace
 
 namespace sogl {
-struct PlanView {
-    int32_t n;
-    int64_t N;
-    const int32_t* new_order;
-    int64_t nnz;
-    const int32_t* row;
-    const int32_t* col;
-    const double* val;
-    int64_t nnz_orig;  // entries of the original matrix (the rest is padding)
-    int64_t n_inputs;  // input tiles: block coordinates and cells (position row*64+col, value)
-    const int32_t* in_bi;
-    const int32_t* in_bj;
-    const int64_t* cell_begin;
-    const uint16_t* cell_pos;
-    const double* cell_val;
-};
-bool plan_view(const sogl_plan* p, PlanView* v);
 void set_last_error(const std::string& s);
 }  // namespace sogl
 

@@ -143,6 +143,7 @@ def load(name: str = "libsogl.so") -> C.CDLL:
             "sogl_factor_get_graph": (C.c_int, [vp, i32, P(i64), P(i64), P(i32), P(i32), P(i32)]),
             "sogl_graph_check": (C.c_int, [P(FactorDesc), P(i64)]),
             "sogl_graph_check_plan": (C.c_int, [vp, i32, P(i64)]),
+            "sogl_tile_order_ops": (C.c_int, [vp, P(_Op), P(i64), P(i32)]),
             "sogl_solveLU": (C.c_int, [i32, i64, i32, P(i32), P(i32), P(dbl), P(dbl), P(dbl)]),
         })
     for fn, (res, args) in sig.items():
@@ -329,6 +330,21 @@ def graph_check(plan: "Plan", precision: int = FP64) -> dict:
     if rc != OK:
         raise SoglError(rc, lib.sogl_last_error().decode())
     return dict(zip(GRAPH_INFO, (int(v) for v in info)))
+
+
+def tile_order_ops(plan: "Plan"):
+    """(op list rows, id count) a plan is factored by (sogl_tile_order_ops), or None where it
+    keeps its own list."""
+    lib = load("libsogl.so")
+    n, ids = C.c_int64(), C.c_int32()
+    for k in range(2):
+        buf = (_Op * n.value)() if k else None
+        rc = lib.sogl_tile_order_ops(plan.h, buf, C.byref(n), C.byref(ids))
+        if rc != OK:
+            raise SoglError(rc, lib.sogl_last_error().decode())
+        if n.value == 0:
+            return None
+    return np.frombuffer(buf, dtype=np.int32).reshape(-1, 8).copy(), ids.value
 
 
 def canonical_ops(ops: np.ndarray) -> np.ndarray:
