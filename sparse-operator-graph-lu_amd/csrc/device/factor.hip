@@ -235,8 +235,7 @@ constexpr int PAIR_WINDOW = 32;
 constexpr int PAIR_RING = 2 * PAIR_WINDOW;
 constexpr int PM_LEN = 2 * PAIR_RING;          // two window counts
 constexpr int PM_SINGLE = PM_LEN + 2;          // two single-wait slots of two words
-constexpr int PM_ADD = PM_SINGLE + 4;          // the added tile: seen ready, its mask
-constexpr int PM_WAR = PM_ADD + 2;             // the result slot's readers all seen done
+constexpr int PM_WAR = PM_SINGLE + 4;          // the result slot's readers all seen done
 constexpr int PM_WORDS = PM_WAR + 1;
 // A task claimed by the workgroup that made one of its operands (dynamic chaining) has
 // every operand published already: `pre` holds the operands' masks (pair lanes 0-3, the
@@ -272,13 +271,14 @@ struct PairWait {
         }
         if (threadIdx.x < 64) {  // wave 0
             const int lane = threadIdx.x;
-            const int cnt = min(npairs - s, PAIR_WINDOW);
+            const bool has_add = fadd >= 0 && window == 0;  // its flag takes lane 63
+            const int cnt = min(npairs - s, has_add ? PAIR_WINDOW - 1 : PAIR_WINDOW);
             const int j = s + (lane >> 1);
             int slot = -1;
             const bool pl = lane < 2 * cnt;  // a pair's lane
-            // lane 63 polls the added tile's flag in the first window when no pair has it,
-            // and the lanes between the pairs' and 63 the write-after-read flags
-            const bool al = fadd >= 0 && window == 0 && lane == 63 && !pl;
+            // lane 63 polls the added tile's flag in the first window, and the lanes between
+            // the pairs' and 63 the write-after-read flags
+            const bool al = has_add && lane == 63;
             const int wj = lane - 2 * cnt;
             const bool wl = window == 0 && !pl && lane < 63 && wj < war_n;
             if (pl) {
@@ -290,9 +290,11 @@ struct PairWait {
                 slot = a->war[war_b + wj];
             }
             const unsigned long long want = (unsigned long long)(unsigned)a->epoch << 32;
-            auto poll = [&](bool on, unsigned long long& v) {  // leading pairs with both flags raised
+            // leading pairs with both flags raised (none while the added tile is not ready)
+            auto poll = [&](bool on, unsigned long long& v) {
                 if (on) v = __hip_atomic_load(a->ready + slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 const unsigned long long late = __ballot(on && pl && v < want);
+                if (__ballot(on && al && v < want)) return 0;
                 return (late ? __builtin_ctzll(late) : 2 * cnt) >> 1;
             };
             unsigned long long v = 0;
@@ -308,7 +310,7 @@ struct PairWait {
                 const long long t0 = wall_clock64();
                 for (unsigned spins = 1;; spins++) {
                     __builtin_amdgcn_s_sleep(1);
-                    const int got = poll(small ? slot >= 0 : lane < 2, v);
+                    const int got = poll(small ? slot >= 0 : lane < 2 || al, v);
                     if (got > 0) {
                         len = small ? got : poll(slot >= 0, v);
                         break;
@@ -326,10 +328,6 @@ struct PairWait {
                 }
             }
             if (lane < 2 * len) ring[2 * (j % PAIR_RING) + (lane & 1)] = (uint32_t)v & MASK_ALL;
-            if (fadd >= 0 && window == 0 && lane == 63) {  // not polled (a full window): not seen
-                s_pm[PM_ADD] = al && v >= want;
-                s_pm[PM_ADD + 1] = (uint32_t)v & MASK_ALL;
-            }
             if (window == 0 && war_n > 0) {  // wave-uniform
                 const bool late = __ballot(wl && v < want) != 0;
                 if (lane == 0) s_pm[PM_WAR] = !late && war_n <= 63 - 2 * cnt;
@@ -351,8 +349,8 @@ struct PairWait {
         return s + __builtin_amdgcn_readfirstlane(*s_len);
     }
     __device__ inline void pair_masks(int j, const Pair&, uint32_t& ma, uint32_t& mb) const {
-        ma = s_pm[2 * (j % PAIR_RING)];
-        mb = s_pm[2 * (j % PAIR_RING) + 1];
+        ma = __builtin_amdgcn_readfirstlane(s_pm[2 * (j % PAIR_RING)]);  // wave-uniform: scalar branches
+        mb = __builtin_amdgcn_readfirstlane(s_pm[2 * (j % PAIR_RING) + 1]);
     }
     // Before the first result store of a task whose result slot held another value in
     // this run: every task that read that value has published (its loads are done).
@@ -384,16 +382,6 @@ struct PairWait {
         }
         __syncthreads();
     }
-    // after the first window: was the added tile's flag up (written by that window, read
-    // before the next task's first window can write it again)
-    __device__ inline bool add_ready(int, uint32_t& m) const {
-        if (pre) {
-            m = pre[4];
-            return true;
-        }
-        m = s_pm[PM_ADD + 1];
-        return s_pm[PM_ADD] != 0;
-    }
     __device__ inline void operator()(int s, int fa, int fb, int, int, uint32_t& ma, uint32_t& mb) const {
         uint32_t* pm = s_pm + PM_SINGLE + 2 * (s & 1);
         if (threadIdx.x == 0) {
@@ -406,8 +394,8 @@ struct PairWait {
             if (a->trace) *t_wait = wall_clock64();
         }
         __syncthreads();
-        ma = pm[0];
-        mb = pm[1];
+        ma = __builtin_amdgcn_readfirstlane(pm[0]);
+        mb = __builtin_amdgcn_readfirstlane(pm[1]);
     }
 };
 
@@ -436,7 +424,7 @@ __device__ __attribute__((always_inline)) double run_task(const DevTask& t, cons
                 gemm_task_bf16<LLT, MASKS, Wait, COH>(reinterpret_cast<float*>(a.pool), a.pairs + t.a, t.b, t.out0,
                                                       lds, s_mask, wait, t.add, t.add_neg != 0, t.fadd);
             } else {
-                gemm_task<T, ACC, LLT, MASKS, Wait, ONE, COH>(pool, a.pairs + t.a, t.b, t.out0, lds, s_mask, wait,
+                gemm_task<T, ACC, LLT, MASKS, Wait, COH, ONE || sizeof(T) == 4>(pool, a.pairs + t.a, t.b, t.out0, lds, s_mask, wait,
                                                               t.add, t.add_neg != 0, t.fadd, LDS_HANDOFF && handoff);
             }
             break;
@@ -491,13 +479,13 @@ __device__ __attribute__((always_inline)) void absorbed_panel(const Args& a, con
     T* pool = reinterpret_cast<T*>(a.pool);
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int wr = (w >> 1) * 32, wc = (w & 1) * 32, li = lane & 15, lk = lane >> 4;
-    const Pair pr = a.pairs[pd.a];
+    const Pair pr = const_load(a.pairs + pd.a);
     T* icopy = copy;
     const int oslot = lp ? pair_a(pr) : pair_b(pr);
     if (tid == 0) *s_word = (uint32_t)spin_ready(a, lp ? pr.fa : pr.fb) & MASK_ALL;
     if (refactored) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the inverse is read back below
     __syncthreads();
-    const uint32_t om = *s_word;
+    const uint32_t om = __builtin_amdgcn_readfirstlane(*s_word);
     constexpr int LDA = lda<T>();
     T* la = reinterpret_cast<T*>(lds);
     T* lb = la + TS * LDA;
@@ -513,7 +501,7 @@ __device__ __attribute__((always_inline)) void absorbed_panel(const Args& a, con
     if (!MASKS || (ma != 0 && mb != 0)) {  // a zero product is skipped, as in the GEMM task
         uint32_t kuse = 0xFu;
         if constexpr (MASKS) kuse = k_blocks_used(ma, mb, wr >> 4, wc >> 4);
-        gemm_lds<T, false>(acc, lp ? la : icopy, lp ? icopy : lb, wr, wc, li, lk, kuse);
+        gemm_lds<T, false, true>(acc, lp ? la : icopy, lp ? icopy : lb, wr, wc, li, lk, kuse);
     }
     T* C = pool + (size_t)pd.out0 * TE;
     bool nz[2][2] = {{false, false}, {false, false}};
@@ -609,11 +597,11 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
         // alone reads it, which this workgroup runs at once, without a wait (the sum is
         // its only source, and the barrier below makes it visible to the workgroup);
         // then the tasks it claimed
-        int ti = a.queue[qi];
+        int ti = const_load(a.queue + qi);
         int mode = 0;  // 0: from the queue, 1: the static chain's next task, 2: claimed,
                        // 3: the after-link of the previous task (waits as a queued task)
         for (;;) {
-        const DevTask t = a.tasks[ti];
+        const DevTask t = const_load(a.tasks + ti);
         const int nxt = __builtin_amdgcn_readfirstlane(t.next);
         long long t_taken = 0, t_ready = 0, t_wait = 0;
         if (a.trace && tid == 0) t_taken = wall_clock64();
@@ -646,10 +634,12 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
             if (cs >= 0) cv = __hip_atomic_load(a.ready + cs, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         // an lu with absorbed panels (wave-uniform task fields): the panels' descriptors
-        const bool absorbs = ABSORB && t.kind == TK_LU && (t.pan_l >= 0 || t.pan_u >= 0);
+        // (with dynamic chaining on, panels run as after-links, whose outputs' candidates
+        // can be claimed)
+        const bool absorbs = ABSORB && !a.chain && t.kind == TK_LU && (t.pan_l >= 0 || t.pan_u >= 0);
         const bool has_l = absorbs && t.pan_l >= 0, has_u = absorbs && t.pan_u >= 0;
-        const DevTask pdl = has_l ? a.tasks[t.pan_l] : t;
-        const DevTask pdu = has_u ? a.tasks[t.pan_u] : t;
+        const DevTask pdl = const_load(a.tasks + (has_l ? t.pan_l : ti));
+        const DevTask pdu = const_load(a.tasks + (has_u ? t.pan_u : ti));
         // the task this workgroup runs next (the static chain): touch its descriptor now,
         // so that its fetch at the top of the loop hits the cache (the loads are consumed
         // after this task; a GEMM's first wait for its operands covers their latency)
@@ -2476,8 +2466,14 @@ int launch_factor(Context* c, Factor* f, int mode, int chunk, int wg_per_cu) {
         a.ntasks = (int32_t)f->tasks.size();
         a.queue = (const int32_t*)f->queue_d.p;
         a.nqueue = (int32_t)f->queue.size();
-        // one workgroup per CU: the kernel built for that occupancy
-        const bool one = wg_per_cu == 1;
+        // one workgroup per CU: the kernel built for that occupancy.  Where none is asked for,
+        // it takes the graphs of fewer than NARROW tasks per dependency level, whose time is
+        // the latency of the chain through the diagonal: its tasks are 10 to 30% shorter
+        // there (a CU of its own, twice the registers).  Factor ms, two per CU / one:
+        // 14 to 33 tasks per level: C2 FP64 56.7 / 51.3, symmetric 3D 37^3 FP64 25.9 / 21.8,
+        // 2D 64^2 FP64 1.93 / 1.68; 358: C3 FP32 35.7 / 39.5, FP64 61.2 / 75.5.
+        constexpr size_t NARROW = 64;
+        const bool one = wg_per_cu == 1 || (wg_per_cu == 0 && f->tasks.size() < NARROW * (f->level_begin.size() - 1));
         auto kern = one ? k_factor_persistent<T, BF16, LLT, MASKS, true, COH>
                         : k_factor_persistent<T, BF16, LLT, MASKS, false, COH>;
         int per_cu = 0;

@@ -60,6 +60,22 @@ constexpr int lds_bytes() {
                 sizeof(T) == 8 ? 0 : (TS * lda<double>() + 2 * TS) * 8);
 }
 
+// A copy of *p from memory that no kernel writes (task, pair and dependency tables): through
+// the constant address space, so that a wave-uniform address takes scalar loads, whatever
+// stores stand between.
+template <typename V>
+__device__ __forceinline__ V const_load(const V* p) {
+    static_assert(sizeof(V) % 4 == 0, "dwords");
+    typedef const __attribute__((address_space(4))) int CI;
+    struct Words {
+        int w[sizeof(V) / 4];
+    } u;
+    CI* q = (CI*)(uintptr_t)p;
+#pragma unroll
+    for (size_t i = 0; i < sizeof(V) / 4; i++) u.w[i] = q[i];
+    return __builtin_bit_cast(V, u);
+}
+
 // ------------------------------------------------------------------ publishing
 // Device-scope release: write the L2 back, then wait until the write-back is done, so
 // a flag stored next is seen only after every earlier store of the workgroup (the
@@ -381,40 +397,62 @@ __device__ __forceinline__ void read4(const T* p, T (&v)[4]) {
         v[0] = x.x, v[1] = x.y, v[2] = y.x, v[3] = y.y;
     }
 }
-template <typename T, bool TB, typename acc_t>
-__device__ __forceinline__ void gemm_lds_k(acc_t (&acc)[2][2], const T* la, const T* lb, int wr, int wc, int li,
-                                           int lk, int K) {
+// One k block's operands of a wave, and their 16 MFMA.
+template <typename T>
+struct Frag {
+    T a[2][4], b[2][4];
+};
+template <typename T, bool TB>
+__device__ __forceinline__ void frag_read(Frag<T>& f, const T* la, const T* lb, int wr, int wc, int li, int lk, int K) {
     constexpr int LDA = lda<T>();
     const int k0 = 16 * K + 4 * lk;
-    T af[2][4], bf[2][4];
 #pragma unroll
-    for (int m = 0; m < 2; m++) read4(la + (wr + m * 16 + li) * LDA + k0, af[m]);
+    for (int m = 0; m < 2; m++) read4(la + (wr + m * 16 + li) * LDA + k0, f.a[m]);
 #pragma unroll
     for (int n = 0; n < 2; n++) {
         if constexpr (TB) {
-            read4(lb + (wc + n * 16 + li) * LDA + k0, bf[n]);
+            read4(lb + (wc + n * 16 + li) * LDA + k0, f.b[n]);
         } else {
 #pragma unroll
-            for (int k4 = 0; k4 < 4; k4++) bf[n][k4] = lb[(k0 + k4) * LDB + wc + n * 16 + li];
+            for (int k4 = 0; k4 < 4; k4++) f.b[n][k4] = lb[(k0 + k4) * LDB + wc + n * 16 + li];
         }
     }
+}
+template <typename T, typename acc_t>
+__device__ __forceinline__ void frag_mma(acc_t (&acc)[2][2], const Frag<T>& f, int k0 = 0, int k1 = 4) {
 #pragma unroll
-    for (int k4 = 0; k4 < 4; k4++)
+    for (int k4 = k0; k4 < k1; k4++)
 #pragma unroll
         for (int m = 0; m < 2; m++)
 #pragma unroll
-            for (int n = 0; n < 2; n++) acc[m][n] = MfmaOp<T>::mma(af[m][k4], bf[n][k4], acc[m][n]);
+            for (int n = 0; n < 2; n++) acc[m][n] = MfmaOp<T>::mma(f.a[m][k4], f.b[n][k4], acc[m][n]);
 }
-template <typename T, bool TB, typename acc_t>
+// AHEAD (not the FP64 kernels built for two workgroups per CU, which lack the registers):
+// in the usual dense case the next k block is read while the current one multiplies; the
+// scheduler on its own reads each operand just before its use, and waits for it.
+template <typename T, bool TB, bool AHEAD, typename acc_t>
 __device__ __forceinline__ void gemm_lds(acc_t (&acc)[2][2], const T* la, const T* lb, int wr, int wc, int li, int lk,
                                          uint32_t kuse) {
-    if (kuse == 0xFu) {  // wave-uniform; the usual dense case reads ahead across the blocks
+    if (AHEAD && kuse == 0xFu) {  // wave-uniform
+        Frag<T> f[2];
+        frag_read<T, TB>(f[0], la, lb, wr, wc, li, lk, 0);
 #pragma unroll
-        for (int K = 0; K < 4; K++) gemm_lds_k<T, TB>(acc, la, lb, wr, wc, li, lk, K);
+        for (int K = 0; K < 4; K++) {
+            frag_mma<T>(acc, f[K & 1], 0, 1);  // (the reads queue behind its own)
+            __builtin_amdgcn_sched_barrier(0);
+            if (K < 3) frag_read<T, TB>(f[(K + 1) & 1], la, lb, wr, wc, li, lk, K + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            frag_mma<T>(acc, f[K & 1], 1, 4);
+            __builtin_amdgcn_sched_barrier(0);
+        }
     } else {
 #pragma unroll 1
-        for (int K = 0; K < 4; K++)
-            if ((kuse >> K) & 1u) gemm_lds_k<T, TB>(acc, la, lb, wr, wc, li, lk, K);
+        for (int K = 0; K < 4; K++) {
+            if (!((kuse >> K) & 1u)) continue;
+            Frag<T> f;
+            frag_read<T, TB>(f, la, lb, wr, wc, li, lk, K);
+            frag_mma<T>(acc, f);
+        }
     }
 }
 
@@ -453,27 +491,21 @@ __device__ __forceinline__ uint32_t quad_mask(const bool (&nz)[2][2], int I0, in
 // The pair loop asks in windows: `extend(pairs, s, npairs, window, fadd)` (every thread,
 // a barrier inside; window counts the calls) returns e > s such that pairs s .. e-1 are
 // all ready, and `pair_masks(j, p, ...)` then gives pair j's masks for j < e.  The first
-// window also looks at the flag of the added tile (value id fadd): after it,
-// `add_ready(add, m)` says whether that tile (slot add) could be read from then on
-// (every thread gets the same answer).
+// window also waits for the added tile (value id fadd).
 struct NoWait {
     const uint32_t* mask;
     __device__ inline void operator()(int, int, int, int sa, int sb, uint32_t& ma, uint32_t& mb) const {
         __syncthreads();
-        ma = mask[sa];
-        mb = mask[sb];
+        ma = __builtin_amdgcn_readfirstlane(mask[sa]);
+        mb = __builtin_amdgcn_readfirstlane(mask[sb]);
     }
     __device__ inline int extend(const Pair*, int, int npairs, int, int = -1) const {
         __syncthreads();
         return npairs;
     }
     __device__ inline void pair_masks(int, const Pair& p, uint32_t& ma, uint32_t& mb) const {
-        ma = mask[pair_a(p)];
-        mb = mask[pair_b(p)];
-    }
-    __device__ inline bool add_ready(int add, uint32_t& m) const {
-        m = mask[add];
-        return true;
+        ma = __builtin_amdgcn_readfirstlane(mask[pair_a(p)]);
+        mb = __builtin_amdgcn_readfirstlane(mask[pair_b(p)]);
     }
     // a result slot that held another value: its readers ran at earlier levels, i.e. in
     // earlier launches
@@ -481,11 +513,10 @@ struct NoWait {
 };
 
 // A task made by folding a later sub/neg into the GEMM adds (or subtracts) one more
-// tile, `add`, to the sum, after the last product (the same order in every executor).
-// Its flag is polled with the first window of pairs; a tile that is ready by then is
-// never waited for again (STAGE64 loads it at once, into registers held across the pair
-// loop; the other kernels, which lack the registers, read it after the loop); one that
-// is not is waited for after the pairs.
+// tile, `add`, to the sum, after the last product: a sum that started from it would round
+// every product to its size (C5 FP32: 1,000 times the error after one correction).  Its
+// flag is polled in the first window's round trip; it is the tile's previous part or
+// update (an input, mostly), made earlier.
 template <bool COH, typename T, typename acc_t>
 __device__ __forceinline__ void add_tile(acc_t (&acc)[2][2], const T* __restrict__ X, bool neg, int wr, int wc,
                                          int li, int lk) {
@@ -505,10 +536,8 @@ __device__ __forceinline__ void add_tile(acc_t (&acc)[2][2], const T* __restrict
 // MASKS: skip zero products and zero k blocks by the operands' masks, and leave the
 // mask bits of wave w's quadrant of the result in out_mask[w]; without, every pair is
 // multiplied in full and nothing is left (the result counts as full).
-// STAGE64: stage FP64 operands too, and hold an added tile that is ready early in
-// registers (the kernel built for one workgroup per CU has the registers for it).
-template <typename T, bool ACC = false, bool TBOK = false, bool MASKS = true, typename Wait = NoWait,
-          bool STAGE64 = false, bool COH = false>
+template <typename T, bool ACC = false, bool TBOK = false, bool MASKS = true, typename Wait = NoWait, bool COH = false,
+          bool AHEAD = sizeof(T) == 4>
 __device__ __attribute__((always_inline)) void gemm_task(T* __restrict__ pool, const Pair* __restrict__ pairs, int npairs,
                           int out, char* lds_raw, uint32_t* out_mask, const Wait& wait, int add = -1,
                           bool add_neg = false, int fadd = -1, bool to_lds = false) {
@@ -516,7 +545,7 @@ __device__ __attribute__((always_inline)) void gemm_task(T* __restrict__ pool, c
     constexpr int LDA = lda<T>();
     T* la = reinterpret_cast<T*>(lds_raw);
     T* lb = la + TS * LDA;
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = (w >> 1) * 32, wc = (w & 1) * 32;
     const int li = lane & 15, lk = lane >> 4;
     acc_t acc[2][2];
@@ -534,84 +563,75 @@ __device__ __attribute__((always_inline)) void gemm_task(T* __restrict__ pool, c
         const uint32_t qbk = (TBOK && q.a < 0) ? mask_transpose(qb) : qb;
         return qa == 0 || qbk == 0;
     };
-    // Pairs [0, ready) are known to be ready.  The operands of `staged` (the next
-    // nonzero pair inside that window) are loaded into ga / gb while the current pair
-    // multiplies; a pair outside the window is waited for (and the window extended)
-    // when the loop reaches it.  FP64 tiles are staged only in the kernel built for one
-    // workgroup per CU: 64 more live registers across the MFMA loop make the FP64
-    // kernels built for two spill.
-    constexpr bool STAGE = sizeof(T) == 4 || STAGE64;
-    Seg<T> ga, gb;
-    int ready = 0, staged = -1, window = 0;
-    uint32_t sma = 0, smb = 0;
-    // the added tile: 0 none or not seen yet, 1 ready (read after the loop), 2 in xr
-    int add_state = 0;
-    acc_t xr[2][2];
+    // Pairs [0, ready) are known to be ready.  Each turn loads the operands of the next
+    // nonzero pair into registers, multiplies the pair before it from LDS meanwhile, and
+    // then moves the loaded operands to LDS.  One place loads and one multiplies: operands
+    // carried from turn to turn in registers were copied, and waited for, at once.  A pair
+    // that is not known to be ready is waited for with nothing left to multiply.  Dense
+    // products of a resident set, one workgroup per CU: FP32 1.96 -> 1.61 us a pair (83
+    // TFLOP/s over the chip), FP64 3.20 -> 3.02; two: FP32 1.52 -> 1.25 (107 TFLOP/s).
+    int n = 0, window = 0;
+    bool pend = false;  // LDS holds a pair that is still to be multiplied
+    uint32_t kuse = 0xFu;
+    bool tb = false;
+    Pair pn = const_load(pairs);  // pair n, fetched one turn ahead
+    int ready = wait.extend(pairs, 0, npairs, window++, fadd);
+    if (ready < 0) return;  // another workgroup took the task over (wave-uniform)
+    // the added tile, ready as well: loaded behind the first pair's operands (loads complete
+    // in order, and an input tile comes from HBM) or, without AHEAD, after the products
+    bool x_due = AHEAD && add >= 0;
     const T* X = pool + (size_t)(add >= 0 ? add : 0) * TE;
-    for (int s = 0; s < npairs; s++) {
-        const Pair p = pairs[s];
-        const bool neg = p.b < 0, tb = TBOK && p.a < 0;
-        uint32_t ma, mbs;  // the tiles' masks as stored
-        bool synced = false;
-        if (s != staged) {
-            if (s == ready) {
-                ready = wait.extend(pairs, s, npairs, window++, fadd);  // its barrier also frees LDS
-                if (ready < 0) return;  // another workgroup took the task over (wave-uniform)
-                synced = true;
-                uint32_t mx;
-                if (s == 0 && add >= 0 && wait.add_ready(add, mx)) {
-                    add_state = 1;
-                    if constexpr (STAGE64) {  // 16 (FP32) or 32 (FP64) more live registers
-#pragma unroll
-                        for (int m = 0; m < 2; m++)
-#pragma unroll
-                            for (int n = 0; n < 2; n++)
-                                xr[m][n] = acc_load_global<COH>(X, wr + m * 16, wc + n * 16, li, lk);
-                        add_state = 2;
-                    }
-                }
-            }
-            wait.pair_masks(s, p, ma, mbs);
-            if (zero_product(p, ma, mbs)) continue;  // every thread skips
-            seg_load<COH>(pool + (size_t)pair_a(p) * TE, ga, tid, !MASKS || seg_on<T>(ma, tid));
-            seg_load<COH>(pool + (size_t)pair_b(p) * TE, gb, tid, !MASKS || seg_on<T>(mbs, tid));
-        } else {
-            ma = sma;
-            mbs = smb;
-        }
-        if (!synced) __syncthreads();  // every wave is done reading the previous pair from LDS
-        seg_store(ga, la, LDA, tid, !MASKS || seg_on<T>(ma, tid), neg);
-        seg_store(gb, lb, tb ? LDA : LDB, tid, !MASKS || seg_on<T>(mbs, tid));
-        staged = -1;
-        for (int n = s + 1; STAGE && n < ready; n++) {
-            const Pair q = pairs[n];
-            uint32_t qa, qb;
-            wait.pair_masks(n, q, qa, qb);
-            if (zero_product(q, qa, qb)) continue;
-            seg_load<COH>(pool + (size_t)pair_a(q) * TE, ga, tid, !MASKS || seg_on<T>(qa, tid));
-            seg_load<COH>(pool + (size_t)pair_b(q) * TE, gb, tid, !MASKS || seg_on<T>(qb, tid));
-            staged = n;
-            sma = qa;
-            smb = qb;
-            break;
-        }
-        __syncthreads();
-        uint32_t kuse = 0xFu;
-        if constexpr (MASKS) kuse = k_blocks_used(ma, tb ? mask_transpose(mbs) : mbs, wr >> 4, wc >> 4);
-        if (tb) gemm_lds<T, TBOK>(acc, la, lb, wr, wc, li, lk, kuse);
-        else gemm_lds<T, false>(acc, la, lb, wr, wc, li, lk, kuse);
-    }
-    if (add_state == 2) {
+    acc_t xr[2][2];
+    auto load_x = [&]() {
 #pragma unroll
         for (int m = 0; m < 2; m++)
 #pragma unroll
-            for (int n = 0; n < 2; n++) acc[m][n] += add_neg ? -xr[m][n] : xr[m][n];
-    } else if (add >= 0) {
-        if (add_state == 0) {
-            uint32_t m0, m1;
-            wait(npairs, fadd, fadd, add, add, m0, m1);
+            for (int q = 0; q < 2; q++) xr[m][q] = acc_load_global<COH>(X, wr + m * 16, wc + q * 16, li, lk);
+    };
+    for (;;) {
+        Pair p = pn;
+        uint32_t ma = MASK_ALL, mb = MASK_ALL;
+        while (n < ready) {  // every thread skips zero products
+            wait.pair_masks(n, p, ma, mb);
+            if (!zero_product(p, ma, mb)) break;
+            n++;
+            pn = p = const_load(pairs + min(n, npairs - 1));
         }
-        add_tile<COH, T>(acc, X, add_neg, wr, wc, li, lk);
+        const bool rdy = n < ready;
+        Seg<T> ga, gb;
+        if (rdy) {
+            seg_load<COH>(pool + (size_t)pair_a(p) * TE, ga, tid, !MASKS || seg_on<T>(ma, tid));
+            seg_load<COH>(pool + (size_t)pair_b(p) * TE, gb, tid, !MASKS || seg_on<T>(mb, tid));
+            pn = const_load(pairs + min(n + 1, npairs - 1));
+            if (x_due) load_x();
+            x_due = false;
+        }
+        if (pend) {
+            if (tb) gemm_lds<T, TBOK, AHEAD>(acc, la, lb, wr, wc, li, lk, kuse);
+            else gemm_lds<T, false, AHEAD>(acc, la, lb, wr, wc, li, lk, kuse);
+        }
+        if (!rdy) {
+            pend = false;
+            if (n >= npairs) break;
+            ready = wait.extend(pairs, n, npairs, window++);
+            if (ready < 0) return;
+            continue;
+        }
+        __syncthreads();  // every wave is done reading the previous pair from LDS
+        tb = TBOK && p.a < 0;
+        seg_store(ga, la, LDA, tid, !MASKS || seg_on<T>(ma, tid), p.b < 0);
+        seg_store(gb, lb, tb ? LDA : LDB, tid, !MASKS || seg_on<T>(mb, tid));
+        __syncthreads();
+        if constexpr (MASKS) kuse = k_blocks_used(ma, tb ? mask_transpose(mb) : mb, wr >> 4, wc >> 4);
+        pend = true;
+        n++;
+    }
+    if (add >= 0) {
+        if (!AHEAD || x_due) load_x();
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int q = 0; q < 2; q++) acc[m][q] += add_neg ? -xr[m][q] : xr[m][q];
     }
     wait.war_done(true);
     T* C = pool + (size_t)out * TE;
