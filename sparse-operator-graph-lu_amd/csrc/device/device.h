@@ -139,10 +139,12 @@ struct Factor {
     // triangular solve structure (block CSR by block row, off-diagonal only)
     std::vector<int32_t> l_diag, u_diag, linv_slot, uinv_slot;  // per block row
     DevBuf l_rowptr, l_col, l_slot, u_rowptr, u_col, u_slot, l_diag_d, u_diag_d, linv_d, uinv_d;
+    // the same by pairs of block rows and of block columns (pair_steps)
+    DevBuf lstep_ptr, lstep_col, lstep_slot, ustep_ptr, ustep_col, ustep_slot;
+    int64_t solve_entries = 0;  // off-diagonal tiles of L and U
     DevBuf pairx_d, pairy_d;  // per row pair: slot of X_p / Y_p (the two-row solve steps), -1: zero
-    DevBuf solve_ready, solve_ctrl, vec_b, vec_x, vec_y;
+    DevBuf solve_ctrl, vec_b, vec_x, vec_y;
     size_t vec_cap = 0;  // doubles per vector buffer
-    int32_t solve_epoch = 0;
     // factor tile lists in load order
     std::vector<int32_t> l_slots, u_slots;
     // refinement

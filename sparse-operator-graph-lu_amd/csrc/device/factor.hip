@@ -2226,6 +2226,40 @@ int validate_slots(Context* c, const Factor* f, const HostGraph& hg) {
     return SOGL_OK;
 }
 
+// The off-diagonal entries of a triangular factor's block rows (sorted by column) by pairs of
+// block rows (2p, 2p+1) and of block columns (2P, 2P+1), P != p: per row pair, the column pairs
+// in order, each with the slots of its tiles (2p, 2P), (2p, 2P+1), (2p+1, 2P), (2p+1, 2P+1),
+// -1 where there is none.  A repeated block opens another step.
+struct PairSteps {
+    std::vector<int32_t> ptr, col, slot;
+};
+PairSteps pair_steps(const std::vector<int32_t>& rp, const std::vector<int32_t>& ci, const std::vector<int32_t>& sl) {
+    PairSteps s;
+    const int32_t R = (int32_t)rp.size() - 1;
+    s.ptr.assign(1, 0);
+    for (int32_t r0 = 0; r0 < R; r0 += 2) {
+        size_t q[2] = {(size_t)rp[(size_t)r0], (size_t)rp[(size_t)r0 + 1]};
+        const size_t end[2] = {q[1], (size_t)rp[(size_t)std::min(r0 + 2, R)]};
+        for (;;) {
+            int32_t P = INT32_MAX;
+            for (int h = 0; h < 2; h++)
+                if (q[h] < end[h]) P = std::min(P, ci[q[h]] / 2);
+            if (P == INT32_MAX) break;
+            int32_t t[4] = {-1, -1, -1, -1};
+            for (int h = 0; h < 2; h++)
+                while (q[h] < end[h] && ci[q[h]] / 2 == P && t[2 * h + ci[q[h]] % 2] < 0) {
+                    t[2 * h + ci[q[h]] % 2] = sl[q[h]];
+                    q[h]++;
+                }
+            if (P == r0 / 2) continue;  // the pair's own block (pairinv)
+            s.col.push_back(P);
+            s.slot.insert(s.slot.end(), t, t + 4);
+        }
+        s.ptr.push_back((int32_t)s.col.size());
+    }
+    return s;
+}
+
 // Device arrays of a checked graph: pool, tasks, pairs, dependencies, flags, solve
 // structure, and the input tiles copied in.
 int upload_graph(Context* c, const sogl_factor_desc* d, const InputCells* cells, Factor* f,
@@ -2279,6 +2313,14 @@ int upload_graph(Context* c, const sogl_factor_desc* d, const InputCells* cells,
         (rc = up_i32(f->pairx_d, hg.pair_x, "row pair L blocks")) || (rc = up_i32(f->pairy_d, hg.pair_y, "row pair U blocks")) ||
         (rc = up_i32(f->inputs_d, f->input_slots, "input slots")))
         return rc;
+    f->solve_entries = (int64_t)hg.lc.size() + (int64_t)hg.uc.size();
+    for (int which = 0; which < 2; which++) {
+        const PairSteps s = which == 0 ? pair_steps(hg.lp, hg.lc, hg.ls) : pair_steps(hg.up, hg.uc, hg.us);
+        if ((rc = up_i32(which == 0 ? f->lstep_ptr : f->ustep_ptr, s.ptr, "solve steps")) ||
+            (rc = up_i32(which == 0 ? f->lstep_col : f->ustep_col, s.col, "solve step columns")) ||
+            (rc = up_i32(which == 0 ? f->lstep_slot : f->ustep_slot, s.slot, "solve step tiles")))
+            return rc;
+    }
     hipLaunchKernelGGL(k_fill<unsigned long long>, dim3(256), dim3(256), 0, st, (unsigned long long*)f->ready_d.p,
                        (size_t)f->n_slots, 0ull);
     // input tiles (slots 0..n_inputs-1) and the zero tile never change: always ready
@@ -2397,7 +2439,8 @@ void free_factor(Factor* f) {
     for (DevBuf* b : {&f->pool, &f->mask_d, &f->queue_d, &f->war_d, &f->uinv_chk_d, &f->pairx_d, &f->pairy_d, &f->cell_begin, &f->cell_pos, &f->cell_val, &f->chk_d, &f->tasks_d, &f->pairs_d, &f->deps_d, &f->ready_d, &f->ctrl_d,
                       &f->op_tasks_d, &f->op_pairs_d, &f->inputs_d, &f->l_rowptr, &f->l_col,
                       &f->l_slot, &f->u_rowptr, &f->u_col, &f->u_slot, &f->l_diag_d, &f->u_diag_d,
-                      &f->linv_d, &f->uinv_d, &f->solve_ready, &f->solve_ctrl, &f->vec_b, &f->vec_x,
+                      &f->linv_d, &f->uinv_d, &f->lstep_ptr, &f->lstep_col, &f->lstep_slot, &f->ustep_ptr, &f->ustep_col,
+                      &f->ustep_slot, &f->solve_ctrl, &f->vec_b, &f->vec_x,
                       &f->vec_y, &f->csr_ptr, &f->csr_col, &f->csr_val, &f->vec_r, &f->vec_d, &f->red, &f->perm_d, &f->vec_io, &f->trace_d})
         dev_free(*b);
     delete f;

@@ -3,18 +3,17 @@
 // (BlockPlanner.cpp:669-862), which recurse over the L and U quadtrees with
 // one right-hand side, serially.
 //
-// Here each block row (with 1-15 right-hand sides: each pair of block rows) is a task
-// of a persistent kernel: forward,
+// Here a persistent kernel solves, forward,
 //     y_I = Linv_II (b_I - sum_{J<I} L_IJ y_J)
 // backward,
 //     x_I = Uinv_II (y_I - sum_{J>I} U_IJ x_J)
-// with the inverses of the diagonal tiles (and, for row pairs, the off-diagonal block
-// of the pair's 2x2 diagonal block's inverse) made once per factor.  Tasks are taken in
-// dependency order (ascending / descending) and a task waits only for the rows it
-// reads, so independent rows overlap and the chain only serialises where the factor's
-// block structure does.  With 1-15 right-hand sides a task waits on the stored values
-// themselves (a pending marker until stored); the MFMA form for more right-hand sides
-// waits on per-row ready flags.  Sums run in FP64 for every tile precision.
+// with the inverses of the diagonal tiles and the off-diagonal block of each row pair's 2x2
+// diagonal block's inverse made once per factor.  Tasks are pairs of block rows, taken in
+// dependency order (ascending / descending); a task waits only for the rows it reads, on the
+// stored values themselves (a pending marker until stored), so independent rows overlap and
+// the chain only serialises where the factor's block structure does.  With 1-15 right-hand
+// sides every column is a chain of tasks of its own, from 16 on every panel of 16 columns is
+// (on MFMA).  Sums run in FP64 for every tile precision.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -27,7 +26,12 @@ namespace sogl_dev {
 
 constexpr long long SOLVE_SPIN_LIMIT = 20LL * 100 * 1000 * 1000;
 constexpr int TRSM_MIN_RHS = 16;   // from this many right-hand sides the block-row sums run on MFMA
-constexpr int TRSM_MAX_RHS = 256;  // columns per MFMA solve launch (4 panels of 64)
+// FP64 solves of 1-15 columns: off-diagonal tiles per block row, over L and U, from which the
+// kernel that loads a whole step ahead (KEEP) is taken.  A solve without / with it: 1.1 tiles
+// a row (2D 64^2) 0.103 / 0.116 ms, 1.9 (2D 128^2) 0.376 / 0.426; 3.6 (2D 253^2) 1.99 / 1.71,
+// 5.5 (2D 400^2) 7.8 / 5.1, 14 (3D 31^3) 1.83 / 1.41, 34 (3D 48^3) 8.1 / 7.0.
+constexpr int KEEP_ENTRIES = 2;
+constexpr int MAX_RHS = 1024;      // columns per launch: pairs x panels fit the 32-bit task counter
 
 struct SolveArgs {
     const void* pool;
@@ -41,52 +45,29 @@ struct SolveArgs {
     int32_t nrhs;
     int32_t nbr;
     int32_t forward;
-    int32_t epoch;
-    int* ready;
-    int* ctrl;            // [0] row counter, [1] abort
+    int* ctrl;            // [0] task counter, [1] abort
     const uint32_t* mask; // per slot: the factor's 16x16 block masks (a zero tile is skipped)
+    const int32_t* prow;     // the many-RHS form's steps (pair_steps): per row pair, its steps'
+    const int32_t* pcol;     // block column pairs
+    const int4* pslot;       // and tiles
     const int32_t* pairinv;  // per row pair: slot of the 2x2 diagonal block's inverse's
-                             // off-diagonal block (the one-to-15-RHS form), -1: zero
+                             // off-diagonal block, -1: zero
 };
 
 // The abort word and the wall clock are looked at every SOLVE_SPIN_CHECK polls only, so
 // that each poll costs one round trip to the device coherence point.
 constexpr int SOLVE_SPIN_CHECK = 64;
 
-__device__ inline void spin_row(const SolveArgs& a, int J) {
-    int* flag = a.ready + J;
-    if (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= a.epoch) return;
-    const long long t0 = wall_clock64();
-    for (int spins = 1;; spins++) {
-        __builtin_amdgcn_s_sleep(1);
-        if (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= a.epoch) return;
-        if (spins % SOLVE_SPIN_CHECK) continue;
-        if (__hip_atomic_load(a.ctrl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
-        if (wall_clock64() - t0 > SOLVE_SPIN_LIMIT) {
-            __hip_atomic_store(a.ctrl + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            return;
-        }
-    }
-}
-
-// Rows of the output that a one-to-15-RHS pass has not stored yet hold this signalling
-// NaN, written by k_fill_pending before the pass.  FP arithmetic never produces a
-// signalling NaN (a NaN result is quiet), so a stored value is never mistaken for it.
-// A row task sorts the rows it reads into those already published when it starts (an
-// oldest-first prefix: one check of their ready flags, one acquire, then ordinary
-// cached loads) and the rest, the newest, usually the one on the chain: for those it
-// polls the values themselves with agent-scope atomic loads until none of the 16 it
-// needs is the marker.  The task stores its row with agent-scope atomic stores (they
-// reach the coherence point without waiting for the release), then releases and
-// raises its ready flag for the tasks that start later.
+// Rows of the output that a pass has not stored yet hold this signalling NaN, written by
+// k_fill_pending before the pass.  FP arithmetic never produces a signalling NaN (a NaN
+// result is quiet), so a stored value is never mistaken for it.  A task polls the values it
+// reads themselves, with agent-scope atomic loads, until none is the marker, and stores its
+// rows with agent-scope atomic stores, which reach the coherence point without a release.
 constexpr unsigned long long SOLVE_PENDING = 0x7FF4C0DE5EED0001ull;
 
-__global__ void k_fill_pending(double* out, int64_t ld, int64_t rows, int nrhs) {
-    const int64_t n = rows * nrhs;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t c = i / rows, r = i - c * rows;
-        reinterpret_cast<unsigned long long*>(out)[c * ld + r] = SOLVE_PENDING;
-    }
+__global__ void k_fill_pending(double* out, int64_t n) {
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+        reinterpret_cast<unsigned long long*>(out)[i] = SOLVE_PENDING;
 }
 
 // The 64 values of one column of row J, which another task stores, into this wave's
@@ -170,17 +151,26 @@ __device__ inline double quad_sum(double v) {
     return v + dpp_f64<0x4E>(v);
 }
 
-template <typename T, int CW>
+//
+// KEEP (FP64 tiles, rows of many entries): a task there is bound by walking its entries, each
+// a load of two or four tiles, so the whole next step's tiles and a first read of its x are
+// loaded ahead, and the blocks of the diagonal products wait in LDS for want of registers.
+// Where rows have few entries the hand-off from pair to pair bounds the pass; it is shorter
+// with those blocks in registers.
+template <typename T, bool KEEP>
 __global__ __launch_bounds__(NTP) void k_trsv_persistent(SolveArgs a) {
-    __shared__ double vec[2][TS * CW];
+    constexpr int VE = 16 / sizeof(T);  // elements of a 16-byte vector
+    __shared__ __attribute__((aligned(16))) T kept_d[KEEP ? NTP / 64 : 1][16 / VE][64 * VE];
+    __shared__ __attribute__((aligned(16))) T kept_c[KEEP ? NT / 64 : 1][16 / VE][64 * VE];  // group 1
+    __shared__ double vec[2][TS];
     __shared__ double rowls[NTP / 64][2 * TS];  // per wave: one column of one or two polled rows
     __shared__ int s_row;
     const int tid = threadIdx.x, g = tid / NT, tg = tid % NT;
-    const int r = tg >> 2, kp = tg & 3, lane = tid & 63;
+    const int r = tg >> 2, kp = tg & 3, lane = tid & 63, w = tid >> 6;
     const int bsh = 4 * (r >> 4) + kp;  // this thread's 16x16 block in a tile's mask
     double* ls = rowls[tid >> 6];
     const T* pool = reinterpret_cast<const T*>(a.pool);
-    const int ntask = (a.nbr + 1) / 2;
+    const int ntask = (a.nbr + 1) / 2 * a.nrhs;
     const int rowoff = r * TS + kp * 16;
     for (;;) {
         if (tid == 0) {
@@ -190,7 +180,10 @@ __global__ __launch_bounds__(NTP) void k_trsv_persistent(SolveArgs a) {
         __syncthreads();
         const int q = __builtin_amdgcn_readfirstlane(s_row);  // wave-uniform loop control
         if (q >= ntask) break;
-        const int p = a.forward ? q : ntask - 1 - q;
+        const int qp = q / a.nrhs, c = q - qp * a.nrhs;
+        const int p = a.forward ? qp : (a.nbr + 1) / 2 - 1 - qp;
+        const double* in = a.in + (int64_t)c * a.ld;
+        double* out = a.out + (int64_t)c * a.ld;
         const int I0 = 2 * p, I1 = 2 * p + 1 < a.nbr ? 2 * p + 1 : -1;
         const int IA = a.forward || I1 < 0 ? I0 : I1;
         const int IB = I1 < 0 ? -1 : (a.forward ? I1 : I0);
@@ -202,6 +195,14 @@ __global__ __launch_bounds__(NTP) void k_trsv_persistent(SolveArgs a) {
         const bool hcb = cpl >= 0;
         seg16(pool + (size_t)a.dinv[I >= 0 ? I : IA] * TE + rowoff, dg);
         seg16(pool + (size_t)(hcb ? cpl : a.dinv[IA]) * TE + rowoff, cb);
+        if constexpr (KEEP) {  // each thread its own
+#pragma unroll
+            for (int k = 0; k < 16; k++) kept_d[w][k / VE][lane * VE + k % VE] = dg[k];
+            if (g == 1) {
+#pragma unroll
+                for (int k = 0; k < 16; k++) kept_c[w - NT / 64][k / VE][lane * VE + k % VE] = cb[k];
+            }
+        }
         const int e0 = I >= 0 ? a.rowptr[I] : 0, e1 = I >= 0 ? a.rowptr[I + 1] : 0;
         // entries in dependency order: forward e0, e0+1, ..; backward e1-1, e1-2, ..; row
         // B's last one (column IA: forward the largest column, backward the smallest) is
@@ -209,311 +210,437 @@ __global__ __launch_bounds__(NTP) void k_trsv_persistent(SolveArgs a) {
         int n = e1 - e0;
         if (g == 1 && n > 0 && a.col[a.forward ? e1 - 1 : e0] == IA) n--;
         const int64_t rowI = (int64_t)(I >= 0 ? I : 0) * TS;
-        for (int c0 = 0; c0 < a.nrhs; c0 += CW) {
-            const int cw = min(CW, a.nrhs - c0);
-            double acc[CW];
-#pragma unroll
-            for (int c = 0; c < CW; c++)
-                acc[c] = (I >= 0 && kp == 0 && c < cw) ? a.in[rowI + r + (int64_t)(c0 + c) * a.ld] : 0.0;
-            for (int base = 0; base < n; base += 64) {  // group-uniform
-                const int m = min(64, n - base);
-                int Jv = 0, sv = 0;
-                uint32_t mv = 0;
-                if (lane < m) {
-                    const int e = a.forward ? e0 + base + lane : e1 - 1 - base - lane;
-                    Jv = a.col[e];
-                    sv = a.slot[e];
-                    mv = a.mask[sv];
+        double acc = (I >= 0 && kp == 0) ? in[rowI + r] : 0.0;
+        for (int base = 0; base < n; base += 64) {  // group-uniform
+            const int m = min(64, n - base);
+            int Jv = 0, sv = 0;
+            uint32_t mv = 0;
+            if (lane < m) {
+                const int e = a.forward ? e0 + base + lane : e1 - 1 - base - lane;
+                Jv = a.col[e];
+                sv = a.slot[e];
+                mv = a.mask[sv];
+            }
+            uint64_t rem = __ballot(mv != 0u);  // entries with a nonzero tile, in order
+            if (!rem) continue;
+            // one step: entry J (tile t0), or J and J1 stored by one pair task (t1),
+            // their columns polled in one spin, then the tiles' products
+            auto consume = [&](const double* xj, int64_t off, bool poll, bool both, bool b0, bool b1, const T* u0,
+                               const T* u1) {
+                if (poll) {
+                    if (both)  // the whole wave
+                        load_row_stored<2>(xj, ls, lane, a, off);
+                    else
+                        load_row_stored<1>(xj, ls, lane, a);
                 }
-                uint64_t rem = __ballot(mv != 0u);  // entries with a nonzero tile, in order
-                if (!rem) continue;
-                // one step: entry J (tile t0), or J and J1 stored by one pair task (t1),
-                // their columns polled in one spin, then the tiles' products
-                auto consume = [&](int J, int J1, bool both, bool b0, bool b1, const T* u0, const T* u1) {
-                    const double* xj = a.out + (int64_t)J * TS;
+                // the column into registers first (one batch of LDS reads),
+                // then one branch per tile
+                double xc[16], s = 0;
 #pragma unroll
-                    for (int c = 0; c < CW; c++) {
-                        if (c < cw) {
-                            if (both)  // the whole wave
-                                load_row_stored<2>(xj + (int64_t)(c0 + c) * a.ld, ls, lane, a, (int64_t)(J1 - J) * TS);
-                            else
-                                load_row_stored<1>(xj + (int64_t)(c0 + c) * a.ld, ls, lane, a);
-                            // the column into registers first (one batch of LDS reads),
-                            // then one branch per tile
-                            double xc[16], s = 0;
+                for (int k = 0; k < 16; k++) xc[k] = ls[kp * 16 + k];
+                if (b0) {
 #pragma unroll
-                            for (int k = 0; k < 16; k++) xc[k] = ls[kp * 16 + k];
-                            if (b0) {
+                    for (int k = 0; k < 16; k++) s += (double)u0[k] * xc[k];
+                }
+                if (both) {
 #pragma unroll
-                                for (int k = 0; k < 16; k++) s += (double)u0[k] * xc[k];
-                            }
-                            if (both) {
+                    for (int k = 0; k < 16; k++) xc[k] = ls[TS + kp * 16 + k];
+                    if (b1) {
 #pragma unroll
-                                for (int k = 0; k < 16; k++) xc[k] = ls[TS + kp * 16 + k];
-                                if (b1) {
-#pragma unroll
-                                    for (int k = 0; k < 16; k++) s += (double)u1[k] * xc[k];
-                                }
-                            }
-                            __builtin_amdgcn_wave_barrier();  // ls is rewritten for the next column
-                            acc[c] -= s;
-                        }
+                        for (int k = 0; k < 16; k++) s += (double)u1[k] * xc[k];
                     }
+                }
+                __builtin_amdgcn_wave_barrier();  // ls is rewritten for the next column
+                acc -= s;
+            };
+            auto on = [&](int j) { return (__builtin_amdgcn_readlane(mv, j) >> bsh) & 1u; };
+            auto tile = [&](int j) { return pool + (size_t)__builtin_amdgcn_readlane(sv, j) * TE + rowoff; };
+            if constexpr (KEEP) {
+                struct Step {
+                    T t0[16], t1[16];  // (an element of a zero block: anything)
+                    const double* xj;
+                    int64_t off;       // of the second entry's row from the first's
+                    unsigned long long u[2];
+                    bool both, on0, on1;
                 };
-                auto on = [&](int j) { return (__builtin_amdgcn_readlane(mv, j) >> bsh) & 1u; };
-                auto tile = [&](int j) { return pool + (size_t)__builtin_amdgcn_readlane(sv, j) * TE + rowoff; };
-                if constexpr (sizeof(T) == 4) {
-                    // FP32 tiles: whole steps, the next step's tiles loaded while the
-                    // current step's columns are polled (a step that takes two entries
-                    // leaves no tile of its own to load during its wait)
-                    auto next_step = [&](uint64_t& r, int& ja, int& jb) {
-                        if (!r) return false;
-                        ja = __builtin_ctzll(r);
-                        r &= r - 1;
-                        jb = -1;
-                        if (r) {
-                            const int c = __builtin_ctzll(r);
-                            if ((__builtin_amdgcn_readlane(Jv, c) >> 1) == (__builtin_amdgcn_readlane(Jv, ja) >> 1)) {
-                                jb = c;
-                                r &= r - 1;
-                            }
-                        }
-                        return true;
-                    };
-                    T t0[16], t1[16], n0[16], n1[16];  // loaded only where the block is nonzero
-                    int ja, jb;
-                    next_step(rem, ja, jb);
-                    if (on(ja)) seg16(tile(ja), t0);
-                    if (jb >= 0 && on(jb)) seg16(tile(jb), t1);
-                    for (;;) {
-                        int na = 0, nb = -1;
-                        const bool more = next_step(rem, na, nb);
-                        if (more && on(na)) seg16(tile(na), n0);
-                        if (more && nb >= 0 && on(nb)) seg16(tile(nb), n1);
-                        const bool both = jb >= 0;
-                        const int J = __builtin_amdgcn_readlane(Jv, ja);
-                        const int J1 = __builtin_amdgcn_readlane(Jv, both ? jb : ja);
-                        consume(J, J1, both, on(ja), both && on(jb), t0, t1);
-                        if (!more) break;
-                        ja = na;
-                        jb = nb;
-#pragma unroll
-                        for (int k = 0; k < 16; k++) {
-                            t0[k] = n0[k];
-                            t1[k] = n1[k];
-                        }
-                    }
-                } else {
-                    // FP64 tiles (no registers for a second step): the next entry's tile
-                    // is loaded while the current one's column is polled
-                    int j = __builtin_ctzll(rem);
+                // Every path issues the same loads (a zero block's threads read `idle`, which
+                // is in the cache): behind a branch the compiler cannot count them, and waits
+                // for them before the step before.
+                const T* idle = pool + (size_t)a.dinv[IA] * TE + rowoff;
+                auto fetch = [&](Step& s) {
+                    const int ja = __builtin_ctzll(rem);
                     rem &= rem - 1;
-                    T t0[16], t1[16];
-                    if (on(j)) seg16(tile(j), t0);
-                    for (;;) {
-                        const int J = __builtin_amdgcn_readlane(Jv, j);
-                        const bool has1 = rem != 0;
-                        const int j1 = has1 ? __builtin_ctzll(rem) : 0;
-                        const int J1 = __builtin_amdgcn_readlane(Jv, j1);
-                        const bool on1 = has1 && on(j1);
-                        if (on1) seg16(tile(j1), t1);  // the next tile, loaded while J's column is polled
-                        const bool both = has1 && (J1 >> 1) == (J >> 1);  // stored by one pair task
-                        consume(J, J1, both, on(j), both && on1, t0, t1);
-                        if (!has1) break;
-                        rem &= rem - 1;
-                        if (both) {  // both consumed: the one after is loaded now
-                            if (!rem) break;
-                            j = __builtin_ctzll(rem);
+                    int jb = ja;
+                    s.both = false;
+                    if (rem) {
+                        const int j = __builtin_ctzll(rem);
+                        if ((__builtin_amdgcn_readlane(Jv, j) >> 1) == (__builtin_amdgcn_readlane(Jv, ja) >> 1)) {
+                            jb = j;
+                            s.both = true;
                             rem &= rem - 1;
-                            if (on(j)) seg16(tile(j), t0);
-                        } else {
-                            j = j1;
-#pragma unroll
-                            for (int k = 0; k < 16; k++) t0[k] = t1[k];
                         }
+                    }
+                    s.on0 = on(ja);
+                    s.on1 = s.both && on(jb);
+                    seg16(s.on0 ? tile(ja) : idle, s.t0);
+                    seg16(s.on1 ? tile(jb) : idle, s.t1);
+                    const int J = __builtin_amdgcn_readlane(Jv, ja), J1 = __builtin_amdgcn_readlane(Jv, jb);
+                    s.xj = out + (int64_t)J * TS;
+                    s.off = (int64_t)(J1 - J) * TS;
+                    const unsigned long long* x = reinterpret_cast<const unsigned long long*>(s.xj) + lane;
+                    s.u[0] = __hip_atomic_load(x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    s.u[1] = __hip_atomic_load(x + s.off, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                };
+                auto use = [&](Step& s) {
+                    const bool there = !__ballot(s.u[0] == SOLVE_PENDING || s.u[1] == SOLVE_PENDING);
+                    if (there) {
+                        ls[lane] = __longlong_as_double((long long)s.u[0]);
+                        ls[TS + lane] = __longlong_as_double((long long)s.u[1]);
+                        __builtin_amdgcn_wave_barrier();
+                    }
+                    consume(s.xj, s.off, !there, s.both, s.on0, s.on1, s.t0, s.t1);
+                };
+                Step b0, b1;
+                fetch(b0);
+                for (;;) {
+                    if (!rem) {
+                        use(b0);
+                        break;
+                    }
+                    fetch(b1);
+                    use(b0);
+                    if (!rem) {
+                        use(b1);
+                        break;
+                    }
+                    fetch(b0);
+                    use(b1);
+                }
+            } else if constexpr (sizeof(T) == 4) {
+                // FP32 tiles: whole steps, the next step's tiles loaded while the
+                // current step's columns are polled (a step that takes two entries
+                // leaves no tile of its own to load during its wait)
+                auto next_step = [&](uint64_t& r, int& ja, int& jb) {
+                    if (!r) return false;
+                    ja = __builtin_ctzll(r);
+                    r &= r - 1;
+                    jb = -1;
+                    if (r) {
+                        const int c = __builtin_ctzll(r);
+                        if ((__builtin_amdgcn_readlane(Jv, c) >> 1) == (__builtin_amdgcn_readlane(Jv, ja) >> 1)) {
+                            jb = c;
+                            r &= r - 1;
+                        }
+                    }
+                    return true;
+                };
+                T t0[16], t1[16], n0[16], n1[16];  // loaded only where the block is nonzero
+                int ja, jb;
+                next_step(rem, ja, jb);
+                if (on(ja)) seg16(tile(ja), t0);
+                if (jb >= 0 && on(jb)) seg16(tile(jb), t1);
+                for (;;) {
+                    int na = 0, nb = -1;
+                    const bool more = next_step(rem, na, nb);
+                    if (more && on(na)) seg16(tile(na), n0);
+                    if (more && nb >= 0 && on(nb)) seg16(tile(nb), n1);
+                    const bool both = jb >= 0;
+                    const int J = __builtin_amdgcn_readlane(Jv, ja);
+                    const int J1 = __builtin_amdgcn_readlane(Jv, both ? jb : ja);
+                    consume(out + (int64_t)J * TS, (int64_t)(J1 - J) * TS, true, both, on(ja), both && on(jb), t0, t1);
+                    if (!more) break;
+                    ja = na;
+                    jb = nb;
+#pragma unroll
+                    for (int k = 0; k < 16; k++) {
+                        t0[k] = n0[k];
+                        t1[k] = n1[k];
+                    }
+                }
+            } else {
+                // FP64 tiles (no registers for a second step): the next entry's tile
+                // is loaded while the current one's column is polled
+                int j = __builtin_ctzll(rem);
+                rem &= rem - 1;
+                T t0[16], t1[16];
+                if (on(j)) seg16(tile(j), t0);
+                for (;;) {
+                    const int J = __builtin_amdgcn_readlane(Jv, j);
+                    const bool has1 = rem != 0;
+                    const int j1 = has1 ? __builtin_ctzll(rem) : 0;
+                    const int J1 = __builtin_amdgcn_readlane(Jv, j1);
+                    const bool on1 = has1 && on(j1);
+                    if (on1) seg16(tile(j1), t1);  // the next tile, loaded while J's column is polled
+                    const bool both = has1 && (J1 >> 1) == (J >> 1);  // stored by one pair task
+                    consume(out + (int64_t)J * TS, (int64_t)(J1 - J) * TS, true, both, on(j), both && on1, t0, t1);
+                    if (!has1) break;
+                    rem &= rem - 1;
+                    if (both) {  // both consumed: the one after is loaded now
+                        if (!rem) break;
+                        j = __builtin_ctzll(rem);
+                        rem &= rem - 1;
+                        if (on(j)) seg16(tile(j), t0);
+                    } else {
+                        j = j1;
+#pragma unroll
+                        for (int k = 0; k < 16; k++) t0[k] = t1[k];
                     }
                 }
             }
-#pragma unroll
-            for (int c = 0; c < CW; c++) acc[c] = quad_sum(acc[c]);
-            if (kp == 0) {
-#pragma unroll
-                for (int c = 0; c < CW; c++) vec[g][r * CW + c] = acc[c];
-            }
-            __syncthreads();
-            double o[CW];
-#pragma unroll
-            for (int c = 0; c < CW; c++) {
-                double v[16], s = 0;
-#pragma unroll
-                for (int k = 0; k < 16; k++) v[k] = vec[g][(kp * 16 + k) * CW + c];
-#pragma unroll
-                for (int k = 0; k < 16; k++) s += (double)dg[k] * v[k];
-                if (g == 1 && hcb) {
-#pragma unroll
-                    for (int k = 0; k < 16; k++) v[k] = vec[0][(kp * 16 + k) * CW + c];
-#pragma unroll
-                    for (int k = 0; k < 16; k++) s += (double)cb[k] * v[k];
-                }
-                o[c] = s;
-            }
-#pragma unroll
-            for (int c = 0; c < CW; c++) o[c] = quad_sum(o[c]);
-            if (kp == 0 && I >= 0) {
-                for (int c = 0; c < cw; c++)
-                    __hip_atomic_store(reinterpret_cast<unsigned long long*>(a.out) + rowI + r + (int64_t)(c0 + c) * a.ld,
-                                       (unsigned long long)__double_as_longlong(o[c]), __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-            }
-            __syncthreads();  // vec is reused by the next chunk
         }
-    }
-}
-
-// Many right-hand sides: the same block-row schedule with the sums on MFMA.  Row I's
-// right-hand sides go in panels of 64 columns; for each panel the workgroup keeps
-// R = B_I - sum_J L_IJ X_J as a 64x64 accumulator (wave w: quadrant (w/2, w%2) as 2x2
-// v_mfma_f64_16x16x4 blocks), each product staged through LDS like the factor's
-// GEMM (tiles of any storage precision widened to FP64), then X_I = Linv_II R.
-// Columns past nrhs read as zero and are not stored.
-template <typename T>
-__device__ inline void tile_to_lds_f64(const T* __restrict__ g, double* __restrict__ s, int ld, int tid,
-                                       uint32_t m = MASK_ALL) {
-    const int r = tid >> 2, c0 = (tid & 3) * 16;
-    const bool on = (m >> (4 * (r >> 4) + (tid & 3))) & 1u;  // zero blocks are written, not read
+        acc = quad_sum(acc);
+        if (kp == 0) vec[g][r] = acc;
+        __syncthreads();
+        double v[16], s = 0;
 #pragma unroll
-    for (int q = 0; q < 16; q++) s[r * ld + c0 + q] = on ? (double)g[r * TS + c0 + q] : 0.0;
-}
-
-// rows row0 .. row0+63 of the column-major vector block v (column stride ld),
-// columns col0 .. col0+63 (zero past ncol), into LDS row-major
-__device__ inline void panel_to_lds(const double* __restrict__ v, int64_t ld, int64_t row0, int col0, int ncol,
-                                    double* __restrict__ s, int lds_ld, int tid) {
-    const int r = tid & 63, cq = tid >> 6;  // lanes walk rows: coalesced within a column
-#pragma unroll 4
-    for (int k = 0; k < 16; k++) {
-        const int cc = cq * 16 + k;
-        const int col = col0 + cc;
-        s[r * lds_ld + cc] = col < ncol ? v[row0 + r + (int64_t)col * ld] : 0.0;
+        for (int k = 0; k < 16; k++) v[k] = vec[g][kp * 16 + k];
+#pragma unroll
+        for (int k = 0; k < 16; k++) s += (double)(KEEP ? kept_d[w][k / VE][lane * VE + k % VE] : dg[k]) * v[k];
+        if (g == 1 && hcb) {
+#pragma unroll
+            for (int k = 0; k < 16; k++) v[k] = vec[0][kp * 16 + k];
+#pragma unroll
+            for (int k = 0; k < 16; k++) s += (double)(KEEP ? kept_c[w - NT / 64][k / VE][lane * VE + k % VE] : cb[k]) * v[k];
+        }
+        s = quad_sum(s);
+        if (kp == 0 && I >= 0)
+            __hip_atomic_store(reinterpret_cast<unsigned long long*>(out) + rowI + r,
+                               (unsigned long long)__double_as_longlong(s), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();  // vec is reused by the next task
     }
 }
 
-template <typename T, int NP>
-__global__ __launch_bounds__(NT, 2) void k_trsm_persistent(SolveArgs a) {
-    constexpr int LDA = lda<double>();
-    __shared__ __attribute__((aligned(16))) double la[TS * LDA];
-    __shared__ __attribute__((aligned(16))) double lb[TS * LDB];
-    __shared__ int s_row, s_abort;
+// Many right-hand sides (16 and more): the same pair tasks with the sums on MFMA, one task
+// per pair and panel of 16 columns (panels are chains of their own: 128 columns are 8
+// chains, which fill the chip where one chain of block rows leaves it idle).  Waves 0-3 sum
+// row A, waves 4-7 row B, wave w rows 16 (w % 4) .. + 15 of it: the products are formed
+// transposed (X^T L^T), so that a lane holds one row and its loads of the right-hand sides
+// and stores of x are whole lines.  A step takes two block columns 2P, 2P+1, which one pair
+// task stores, and the up to four tiles there (pcol, pslot).  Its x (128 x 16) is read, and
+// polled where still pending, once per workgroup, a quarter KB per wave and eighth, and goes
+// through LDS; polled by every wave for itself it was 8 times the traffic, and the polls
+// of the waiting tasks held up the chain (3D 31^3, 16 columns: 8.0 ms a solve).  The
+// tiles' elements come from memory straight into registers: contraction step 4 j + i takes
+// k = 16 j + 4 (lane / 16) + i, so that a lane's operands are runs of four consecutive
+// elements.  The next step's tiles and x are loaded before the current one is waited for; x
+// by ordinary loads (a line cached while pending is seen to be pending and polled; the
+// caches are invalidated at the kernel's start, so no older pass's values are read).
+constexpr int PC = 16;          // columns of a panel
+constexpr int XLD = 2 * TS + 2; // LDS strides of a column: 16-byte reads of 16 columns on distinct banks
+constexpr int PLD = TS + 2;
+
+template <typename T>
+__global__ __launch_bounds__(NTP) void k_trsm_persistent(SolveArgs a) {
+    constexpr int VE = 16 / sizeof(T);  // elements of a 16-byte vector
+    __shared__ __attribute__((aligned(16))) double xs[2][PC * XLD];
+    __shared__ __attribute__((aligned(16))) double vec[2][PC * PLD];
+    __shared__ __attribute__((aligned(16))) T kept_d[NTP / 64][16 / VE][64 * VE];
+    __shared__ __attribute__((aligned(16))) T kept_c[NT / 64][16 / VE][64 * VE];  // group 1
+    __shared__ int s_row;
     typedef MfmaOp<double> M;
     typedef M::acc_t acc_t;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wr = (w >> 1) * 32, wc = (w & 1) * 32, li = lane & 15, lk = lane >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6), g = w >> 2, rb = w & 3;
     const T* pool = reinterpret_cast<const T*>(a.pool);
-    auto mma_lds = [&](acc_t (&acc)[2][2], double sg) {
-#pragma unroll 4
-        for (int kk = 0; kk < TS / 4; kk++) {
-            const int k = 4 * kk + lk;
-            double af[2], bf[2];
+    const int strip = (rb * 16 + li) * TS + 4 * lk;  // this lane's row of a tile
+    const int npan = (a.nrhs + PC - 1) / PC, npair = (a.nbr + 1) / 2;
+    auto load_strip = [&](const T* t, T* v) {
 #pragma unroll
-            for (int m = 0; m < 2; m++) af[m] = sg * la[(wr + m * 16 + li) * LDA + k];
+        for (int j = 0; j < 4; j++)
 #pragma unroll
-            for (int n = 0; n < 2; n++) bf[n] = lb[k * LDB + wc + n * 16 + li];
-#pragma unroll
-            for (int m = 0; m < 2; m++)
-#pragma unroll
-                for (int n = 0; n < 2; n++) acc[m][n] = M::mma(af[m], bf[n], acc[m][n]);
-        }
+            for (int i = 0; i < 4; i++) v[4 * j + i] = t[strip + 16 * j + i];
     };
+    const int xc = tid >> 5, xr = 4 * (tid & 31);  // this thread's part of a step's x
+    struct Step {
+        T t0[16], t1[16];  // the strips of the row's tiles in block columns 2P, 2P+1
+        double x[4];
+        const double* xp;
+        uint32_t b0, b1;   // their nonzero 16x16 blocks
+    };
+    acquire_agent();  // every wave: lines left from earlier passes
     for (;;) {
         if (tid == 0) {
-            s_abort = __hip_atomic_load(a.ctrl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            s_row = s_abort ? a.nbr : atomicAdd(a.ctrl, 1);
+            const int abort = __hip_atomic_load(a.ctrl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            s_row = abort ? npair * npan : atomicAdd(a.ctrl, 1);
         }
         __syncthreads();
         const int q = __builtin_amdgcn_readfirstlane(s_row);  // wave-uniform loop control
-        if (q >= a.nbr) break;
-        const int I = a.forward ? q : a.nbr - 1 - q;
-        const int e0 = a.rowptr[I], e1 = a.rowptr[I + 1], cnt = e1 - e0;
-        const int64_t rowI = (int64_t)I * TS;
-        // R = B_I for every panel of 64 columns (NP panels cover nrhs)
-        acc_t acc[NP][2][2];
+        if (q >= npair * npan) break;
+        const int qp = q / npan, c0 = (q - qp * npan) * PC;
+        const int p = a.forward ? qp : npair - 1 - qp;
+        const int I0 = 2 * p, I1 = 2 * p + 1 < a.nbr ? 2 * p + 1 : -1;
+        const int IA = a.forward || I1 < 0 ? I0 : I1;
+        const int IB = I1 < 0 ? -1 : (a.forward ? I1 : I0);
+        const int I = g == 0 ? IA : IB;  // this group's row, -1: none
+        const int cpl = g == 1 && IB >= 0 ? a.pairinv[p] : -1;
+        const int idle = a.dinv[IA];  // read in the place of an absent tile
+        // the strips of the diagonal inverse and of row B's coupling block, loaded before the
+        // waits and kept in LDS, each lane its own
+        {
+            T dg[16], cb[16];
+            load_strip(pool + (size_t)a.dinv[I >= 0 ? I : IA] * TE, dg);
+            if (cpl >= 0) load_strip(pool + (size_t)cpl * TE, cb);
 #pragma unroll
-        for (int p = 0; p < NP; p++)
+            for (int k = 0; k < 16; k++) kept_d[w][k / VE][lane * VE + k % VE] = dg[k];
+            if (cpl >= 0) {
 #pragma unroll
-            for (int m = 0; m < 2; m++)
-#pragma unroll
-                for (int n = 0; n < 2; n++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const int row = wr + m * 16 + M::row(li, lk, r), col = p * TS + wc + n * 16 + li;
-                        acc[p][m][n][r] = col < a.nrhs ? a.in[rowI + row + (int64_t)col * a.ld] : 0.0;
-                    }
-        // dependencies oldest first; each L tile is staged once for all panels
-        for (int i = 0; i < cnt; i++) {
-            const int e = a.forward ? e0 + i : e1 - 1 - i;
-            const int J = a.col[e];
-            const uint32_t tm = a.mask[a.slot[e]];
-            if (tm == 0) continue;  // a zero tile: no product, no wait for row J
-            if (tid == 0) {
-                spin_row(a, J);
-                acquire_agent();
-            }
-            __syncthreads();  // also: the previous products are done with la / lb
-            tile_to_lds_f64(pool + (size_t)a.slot[e] * TE, la, LDA, tid, tm);
-#pragma unroll
-            for (int p = 0; p < NP; p++) {
-                if (p) __syncthreads();  // the previous panel's product is done with lb
-                panel_to_lds(a.out, a.ld, (int64_t)J * TS, p * TS, a.nrhs, lb, LDB, tid);
-                __syncthreads();
-                mma_lds(acc[p], -1.0);
+                for (int k = 0; k < 16; k++) kept_c[w - NT / 64][k / VE][lane * VE + k % VE] = cb[k];
             }
         }
-        // X_I = Dinv_II R, panel by panel: R goes through LDS as the right operand
-        __syncthreads();
-        tile_to_lds_f64(pool + (size_t)a.dinv[I] * TE, la, LDA, tid);
+        const int e0 = a.prow[p], n = a.prow[p + 1] - e0;
+        const int64_t rowI = (int64_t)(I >= 0 ? I : 0) * TS + rb * 16 + li;
+        // the right-hand sides wait in the lane's own places of vec
 #pragma unroll
-        for (int p = 0; p < NP; p++) {
-            if (p) __syncthreads();
+        for (int r = 0; r < 4; r++) {
+            const int c = c0 + M::row(li, lk, r);
+            vec[g][M::row(li, lk, r) * PLD + rb * 16 + li] = c < a.nrhs ? a.in[rowI + (int64_t)c * a.ld] : 0.0;
+        }
+        // a column past nrhs repeats the last one and is not stored
+        const double* xcol = a.out + (int64_t)min(c0 + xc, a.nrhs - 1) * a.ld;
+        acc_t s0 = {0, 0, 0, 0}, s1 = {0, 0, 0, 0};
+        // the pair's steps in dependency order, 64 at a time, one per lane; every wave walks
+        // the same ones (a step whose tiles are all zero is skipped, with no wait)
+        int base = -64, Pv = 0, sv0 = 0, sv1 = 0;
+        uint32_t mv0 = 0, mv1 = 0;
+        uint64_t rem = 0;
+        auto more = [&]() {
+            while (!rem) {
+                base += 64;
+                if (base >= n) return false;
+                bool any = false;
+                if (lane < n - base) {
+                    const int e = a.forward ? e0 + base + lane : e0 + n - 1 - base - lane;
+                    Pv = a.pcol[e];
+                    const int4 s = a.pslot[e];
+                    const uint32_t m0 = s.x >= 0 ? a.mask[s.x] : 0, m1 = s.y >= 0 ? a.mask[s.y] : 0;
+                    const uint32_t m2 = s.z >= 0 ? a.mask[s.z] : 0, m3 = s.w >= 0 ? a.mask[s.w] : 0;
+                    any = (m0 | m1 | m2 | m3) != 0;
+                    const bool odd = (I & 1) != 0;
+                    sv0 = odd ? s.z : s.x;
+                    sv1 = odd ? s.w : s.y;
+                    mv0 = I < 0 ? 0 : (odd ? m2 : m0) >> (4 * rb);
+                    mv1 = I < 0 ? 0 : (odd ? m3 : m1) >> (4 * rb);
+                }
+                rem = __ballot(any);
+            }
+            return true;
+        };
+        // every path issues the same loads, so that waits can count them
+        auto fetch = [&](Step& s) {
+            const int j = __builtin_ctzll(rem);
+            rem &= rem - 1;
+            s.b0 = __builtin_amdgcn_readlane(mv0, j) & 0xFu;
+            s.b1 = __builtin_amdgcn_readlane(mv1, j) & 0xFu;
+            const int P = __builtin_amdgcn_readlane(Pv, j);
+            const int t0 = __builtin_amdgcn_readlane(sv0, j), t1 = __builtin_amdgcn_readlane(sv1, j);
+            load_strip(pool + (size_t)(s.b0 ? t0 : idle) * TE, s.t0);
+            load_strip(pool + (size_t)(s.b1 ? t1 : idle) * TE, s.t1);
+            // (an odd last block row has no second: its own is read in its place)
+            s.xp = xcol + (int64_t)2 * P * TS + (2 * P + 1 < a.nbr ? xr : xr & (TS - 1));
 #pragma unroll
-            for (int m = 0; m < 2; m++)
+            for (int i = 0; i < 4; i++) s.x[i] = s.xp[i];
+        };
+        auto pending = [&](const Step& s) {
+            bool pend = false;
 #pragma unroll
-                for (int n = 0; n < 2; n++)
+            for (int i = 0; i < 4; i++) pend |= (unsigned long long)__double_as_longlong(s.x[i]) == SOLVE_PENDING;
+            return __ballot(pend) != 0;
+        };
+        int buf = 0;
+        auto consume = [&](Step& s) {
+            if (pending(s)) {
+                const unsigned long long* u = reinterpret_cast<const unsigned long long*>(s.xp);
+                const long long t0 = wall_clock64();
+                for (int spin = 1;; spin++) {
 #pragma unroll
-                    for (int r = 0; r < 4; r++)
-                        lb[(wr + m * 16 + M::row(li, lk, r)) * LDB + wc + n * 16 + li] = acc[p][m][n][r];
+                    for (int i = 0; i < 4; i++)
+                        s.x[i] = __longlong_as_double(
+                            (long long)__hip_atomic_load(u + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+                    if (!pending(s)) break;
+                    if (spin % SOLVE_SPIN_CHECK == 0 &&
+                        (__hip_atomic_load(a.ctrl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ||
+                         wall_clock64() - t0 > SOLVE_SPIN_LIMIT)) {
+                        __hip_atomic_store(a.ctrl + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) s.x[i] = 0.0;
+                        break;
+                    }
+                    __builtin_amdgcn_s_sleep(1);
+                }
+            }
+            // two buffers: every wave has read this one two steps ago, before the last barrier
+            double* xb = xs[buf];
+            buf ^= 1;
+#pragma unroll
+            for (int i = 0; i < 4; i++) xb[xc * XLD + xr + i] = s.x[i];
             __syncthreads();
-            acc_t o[2][2];
+            auto mul = [&](const T* t, uint32_t bits, const double* x) {
 #pragma unroll
-            for (int m = 0; m < 2; m++)
+                for (int j = 0; j < 4; j++) {
+                    if (!((bits >> j) & 1u)) continue;  // a zero block
+                    double v[4];
 #pragma unroll
-                for (int n = 0; n < 2; n++) o[m][n] = acc_t{0, 0, 0, 0};
-            mma_lds(o, 1.0);
-#pragma unroll
-            for (int m = 0; m < 2; m++)
-#pragma unroll
-                for (int n = 0; n < 2; n++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const int row = wr + m * 16 + M::row(li, lk, r), col = p * TS + wc + n * 16 + li;
-                        if (col < a.nrhs) a.out[rowI + row + (int64_t)col * a.ld] = o[m][n][r];
-                    }
+                    for (int i = 0; i < 4; i++) v[i] = x[li * XLD + 16 * j + 4 * lk + i];
+                    s0 = M::mma(v[0], (double)t[4 * j], s0);
+                    s1 = M::mma(v[1], (double)t[4 * j + 1], s1);
+                    s0 = M::mma(v[2], (double)t[4 * j + 2], s0);
+                    s1 = M::mma(v[3], (double)t[4 * j + 3], s1);
+                }
+            };
+            mul(s.t0, s.b0, xb);
+            mul(s.t1, s.b1, xb + TS);
+        };
+        Step b0, b1;
+        if (more()) {
+            fetch(b0);
+            for (;;) {
+                if (!more()) {
+                    consume(b0);
+                    break;
+                }
+                fetch(b1);
+                consume(b0);
+                if (!more()) {
+                    consume(b1);
+                    break;
+                }
+                fetch(b0);
+                consume(b1);
+            }
         }
-        __syncthreads();  // every wave's stores are complete (workgroup release)
-        if (tid == 0) {   // one device-scope release for the workgroup, then the flag
-            release_agent();
-            __hip_atomic_store(a.ready + I, a.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // r = b - sum, in LDS by columns for the diagonal products
+#pragma unroll
+        for (int r = 0; r < 4; r++) vec[g][M::row(li, lk, r) * PLD + rb * 16 + li] -= s0[r] + s1[r];
+        __syncthreads();
+        s0 = acc_t{0, 0, 0, 0};
+        s1 = acc_t{0, 0, 0, 0};
+        auto diag = [&](const double* v, const T* kept) {
+#pragma unroll
+            for (int k = 0; k < 16; k++) {
+                const double x = v[li * PLD + 4 * lk + 16 * (k / 4) + k % 4];
+                const double d = (double)kept[(k / VE) * 64 * VE + lane * VE + k % VE];
+                if (k % 2) s1 = M::mma(x, d, s1);
+                else s0 = M::mma(x, d, s0);
+            }
+        };
+        diag(vec[g], &kept_d[w][0][0]);
+        if (cpl >= 0) diag(vec[0], &kept_c[w - NT / 64][0][0]);  // wave-uniform
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int c = c0 + M::row(li, lk, r);
+            // a NaN is stored quiet: never the pending marker
+            if (I >= 0 && c < a.nrhs)
+                __hip_atomic_store(reinterpret_cast<unsigned long long*>(a.out) + rowI + (int64_t)c * a.ld,
+                                   (unsigned long long)__double_as_longlong(__builtin_canonicalize(s0[r] + s1[r])),
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        __syncthreads();  // separates the publish branch from the next fetch branch
+        __syncthreads();  // vec and xs are reused by the next task
     }
 }
 
 __global__ void k_solve_ctrl_reset(int* ctrl) {
     if (threadIdx.x < 4) ctrl[threadIdx.x] = 0;
-}
-
-__global__ void k_zero_i32(int* p, int n) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0;
 }
 
 // out = diag(L) y over the padded rows, every column: the forward result as the
@@ -538,17 +665,15 @@ namespace {
     } while (0)
 
 // Buffers of one solve beyond its input and output: the forward result y (padded n x
-// nrhs), the per-block-row ready flags of the MFMA form (they hold the epoch of the pass
-// that stored the row, so a fresh set must start at zero) and the control words.
+// nrhs) and the control words.
 struct SolveWork {
     double* y;
-    int* ready;
     int* ctrl;
-    int32_t* epoch;  // last pass's epoch of these flags; each pass takes the next one
 };
 
 template <typename T>
-int launch_pass(Context* c, Factor* f, const SolveWork& w, bool forward, const double* in, double* out, int nrhs) {
+int launch_pass(Context* c, Factor* f, const SolveWork& w, bool mfma, bool forward, const double* in, double* out,
+                int nrhs) {
     SolveArgs a{};
     a.pool = f->pool.p;
     a.rowptr = (const int32_t*)(forward ? f->l_rowptr.p : f->u_rowptr.p);
@@ -561,39 +686,26 @@ int launch_pass(Context* c, Factor* f, const SolveWork& w, bool forward, const d
     a.nrhs = nrhs;
     a.nbr = f->block_rows;
     a.forward = forward ? 1 : 0;
-    a.epoch = ++*w.epoch;
-    a.ready = w.ready;
     a.ctrl = w.ctrl;
     a.mask = (const uint32_t*)f->mask_d.p;
+    a.prow = (const int32_t*)(forward ? f->lstep_ptr.p : f->ustep_ptr.p);
+    a.pcol = (const int32_t*)(forward ? f->lstep_col.p : f->ustep_col.p);
+    a.pslot = (const int4*)(forward ? f->lstep_slot.p : f->ustep_slot.p);
     a.pairinv = (const int32_t*)(forward ? f->pairx_d.p : f->pairy_d.p);
     hipLaunchKernelGGL(k_solve_ctrl_reset, dim3(1), dim3(64), 0, c->stream, a.ctrl);
+    // the rows of out are pending until their task stores them
+    const int64_t n = a.ld * nrhs;
+    const unsigned fg = (unsigned)std::min<int64_t>((n + 255) / 256, 2048);
+    hipLaunchKernelGGL(k_fill_pending, dim3(fg), dim3(256), 0, c->stream, out, n);
+    const int64_t ntask = (int64_t)((a.nbr + 1) / 2) * (mfma ? (nrhs + PC - 1) / PC : nrhs);
+    auto kern = mfma ? k_trsm_persistent<T> : k_trsv_persistent<T, false>;
+    if constexpr (sizeof(T) == 8)
+        if (!mfma && f->solve_entries >= (int64_t)KEEP_ENTRIES * 2 * a.nbr) kern = k_trsv_persistent<T, true>;
     int per_cu = 0;
-    const bool mfma = nrhs >= TRSM_MIN_RHS;
-    if (!mfma) {  // the rows of out are pending until their task stores them
-        const int64_t n = a.ld * nrhs;
-        const unsigned fg = (unsigned)std::min<int64_t>((n + 255) / 256, 2048);
-        hipLaunchKernelGGL(k_fill_pending, dim3(fg), dim3(256), 0, c->stream, out, a.ld, a.ld, nrhs);
-    }
-    const int np = (nrhs + TS - 1) / TS;  // panels of 64 columns (at most TRSM_MAX_RHS / 64)
-    const void* kern = !mfma ? (nrhs == 1 ? (const void*)k_trsv_persistent<T, 1> : (const void*)k_trsv_persistent<T, 8>)
-                       : np == 1 ? (const void*)k_trsm_persistent<T, 1>
-                       : np == 2 ? (const void*)k_trsm_persistent<T, 2>
-                       : np == 3 ? (const void*)k_trsm_persistent<T, 3> : (const void*)k_trsm_persistent<T, 4>;
-    HIP_TRY(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, mfma ? NT : NTP, 0));
+    HIP_TRY(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, NTP, 0));
     if (per_cu < 1) per_cu = 1;
-    const int grid = std::max(1, std::min(mfma ? a.nbr : (a.nbr + 1) / 2, c->num_cu * per_cu));
-    if (!mfma) {
-        if (nrhs == 1) hipLaunchKernelGGL((k_trsv_persistent<T, 1>), dim3(grid), dim3(NTP), 0, c->stream, a);
-        else hipLaunchKernelGGL((k_trsv_persistent<T, 8>), dim3(grid), dim3(NTP), 0, c->stream, a);
-    } else if (np == 1) {
-        hipLaunchKernelGGL((k_trsm_persistent<T, 1>), dim3(grid), dim3(NT), 0, c->stream, a);
-    } else if (np == 2) {
-        hipLaunchKernelGGL((k_trsm_persistent<T, 2>), dim3(grid), dim3(NT), 0, c->stream, a);
-    } else if (np == 3) {
-        hipLaunchKernelGGL((k_trsm_persistent<T, 3>), dim3(grid), dim3(NT), 0, c->stream, a);
-    } else {
-        hipLaunchKernelGGL((k_trsm_persistent<T, 4>), dim3(grid), dim3(NT), 0, c->stream, a);
-    }
+    const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(ntask, (int64_t)c->num_cu * per_cu));
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(NTP), 0, c->stream, a);
     HIP_TRY(c, hipGetLastError());
     return SOGL_OK;
 }
@@ -606,15 +718,16 @@ int solve_core(Context* c, Factor* f, const SolveWork& w, const double* d_b, dou
     int rc;
     HIP_TRY(c, hipEventRecord(c->ev0, c->stream));
     const int64_t ld = (int64_t)R * TS;
-    for (int c0 = 0; c0 < nrhs; c0 += TRSM_MAX_RHS) {  // column groups of one MFMA solve launch
-        const int m = std::min(TRSM_MAX_RHS, nrhs - c0);
+    const bool mfma = nrhs >= TRSM_MIN_RHS;
+    for (int c0 = 0; c0 < nrhs; c0 += MAX_RHS) {
+        const int m = std::min(MAX_RHS, nrhs - c0);
         const int64_t off = (int64_t)c0 * ld;
         if (f->elem == 8) {
-            if ((rc = launch_pass<double>(c, f, w, true, d_b + off, w.y + off, m))) return rc;
-            if ((rc = launch_pass<double>(c, f, w, false, w.y + off, d_x + off, m))) return rc;
+            if ((rc = launch_pass<double>(c, f, w, mfma, true, d_b + off, w.y + off, m))) return rc;
+            if ((rc = launch_pass<double>(c, f, w, mfma, false, w.y + off, d_x + off, m))) return rc;
         } else {
-            if ((rc = launch_pass<float>(c, f, w, true, d_b + off, w.y + off, m))) return rc;
-            if ((rc = launch_pass<float>(c, f, w, false, w.y + off, d_x + off, m))) return rc;
+            if ((rc = launch_pass<float>(c, f, w, mfma, true, d_b + off, w.y + off, m))) return rc;
+            if ((rc = launch_pass<float>(c, f, w, mfma, false, w.y + off, d_x + off, m))) return rc;
         }
     }
     HIP_TRY(c, hipEventRecord(c->ev1, c->stream));
@@ -628,18 +741,11 @@ int solve_core(Context* c, Factor* f, const SolveWork& w, const double* d_b, dou
     return SOGL_OK;
 }
 
-// The factor's own work buffers (allocated on first use; the flags are zeroed once and
-// then ordered by the factor's epoch counter).
+// With the factor's own control words (allocated on first use).
 int solve_device(Context* c, Factor* f, const double* d_b, double* d_x, double* d_y, int nrhs) {
-    const int R = f->block_rows;
     int rc;
-    if ((rc = dev_alloc(c, f->solve_ready, (size_t)R * 4, "solve flags"))) return rc;
     if ((rc = dev_alloc(c, f->solve_ctrl, 16, "solve control"))) return rc;
-    if (f->solve_epoch == 0) {
-        hipLaunchKernelGGL(k_zero_i32, dim3(64), dim3(256), 0, c->stream, (int*)f->solve_ready.p, R);
-        HIP_TRY(c, hipGetLastError());
-    }
-    const SolveWork w{d_y, (int*)f->solve_ready.p, (int*)f->solve_ctrl.p, &f->solve_epoch};
+    const SolveWork w{d_y, (int*)f->solve_ctrl.p};
     return solve_core(c, f, w, d_b, d_x, nrhs);
 }
 
@@ -707,7 +813,7 @@ extern "C" int sogl_solve_device(sogl_ctx* x, int32_t factor_id, const double* d
 }
 
 // ------------------------------------------------------------------ solve without allocation
-// The solve's work buffers (y, flags, control) in one fixed array per GPU, for callers
+// The solve's work buffers (y, control) in one fixed array per GPU, for callers
 // that cannot allocate device memory.  In host code `scratch` names a host-side stand-in
 // for the array, never its device address: the address each GPU gives its own copy is
 // looked up once per device, when the first context on it is created, and only that
@@ -725,15 +831,15 @@ bool g_scratch_done[SCRATCH_MAX_DEVICES];
 
 constexpr size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// Layout inside the array: control words, the flags of `rows` block rows, then y.
+// Layout inside the array: control words, 4 bytes per block row that sogl.h counts in (not
+// used any more; what fits stays the same), then y.
 struct ScratchLayout {
-    size_t ctrl, ready, y, end;
+    size_t ctrl, y, end;
 };
 ScratchLayout scratch_layout(int32_t rows, int32_t nrhs) {
     ScratchLayout l;
     l.ctrl = 0;
-    l.ready = 256;
-    l.y = l.ready + align256((size_t)rows * 4);
+    l.y = 256 + align256((size_t)rows * 4);
     l.end = l.y + (size_t)rows * TS * (size_t)nrhs * 8;
     return l;
 }
@@ -785,11 +891,6 @@ extern "C" int sogl_solve_device_noalloc(sogl_ctx* x, int32_t factor_id, const d
                                               std::to_string((size_t)SOGL_NOALLOC_SCRATCH_BYTES));
     HIP_TRY(c, hipSetDevice(dev));
     char* s = (char*)base;
-    // the flags start at zero for every call (earlier calls, of any factor, left their
-    // epochs in them); a fill kernel, so the call stays capturable
-    hipLaunchKernelGGL(k_zero_i32, dim3(64), dim3(256), 0, c->stream, (int*)(s + l.ready), f->block_rows);
-    HIP_TRY(c, hipGetLastError());
-    int32_t epoch = 0;
-    const SolveWork w{(double*)(s + l.y), (int*)(s + l.ready), (int*)(s + l.ctrl), &epoch};
+    const SolveWork w{(double*)(s + l.y), (int*)(s + l.ctrl)};
     return solve_core(c, f, w, d_bp, d_xp, nrhs);
 }
