@@ -185,6 +185,8 @@ struct Context {
     bool after_links = false;              // for the factors loaded from now on (sogl_ctx_set_task_links)
     bool absorb_panels = true;             // for the factors loaded from now on (sogl_ctx_set_task_links)
     size_t free_mem = 0, total_mem = 0;    // device HBM when the context was made
+    double* norms_h = nullptr;             // pinned: the residual kernel's result (of the call that holds mu)
+    size_t norms_cap = 0;                  // doubles
     std::string err;
     std::map<int32_t, Factor*> factors;
     int32_t next_id = 1;
@@ -197,7 +199,18 @@ int check_hip(Context* c, hipError_t e, const char* what);
 int dev_alloc(Context* c, DevBuf& b, size_t bytes, const char* what);
 void dev_free(DevBuf& b);
 Factor* find_factor(Context* c, int32_t id);
-// implemented in solve.hip: looks up the device address of the no-allocation solve's
+// implemented in solve.hip.  Buffers of one solve beyond its input and output: the forward
+// result y (padded n x nrhs) and the control words (four of each pass).
+constexpr int SOLVE_CTRL_WORDS = 8;
+struct SolveWork {
+    double* y;
+    int* ctrl;
+};
+int solve_work(Context* c, Factor* f, SolveWork& w);
+int solve_launch(Context* c, Factor* f, const SolveWork& w, const double* d_b, double* d_x, int nrhs);
+int solve_timeout(Context* c);
+int ensure_vectors(Context* c, Factor* f, int nrhs);
+// looks up the device address of the no-allocation solve's
 // scratch array on `device` (current), once per device
 void noalloc_scratch_init(int device);
 

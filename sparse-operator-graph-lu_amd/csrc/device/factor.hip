@@ -2610,6 +2610,7 @@ extern "C" void sogl_ctx_destroy(sogl_ctx* x) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     for (auto& kv : c->factors) free_factor(kv.second);
     c->factors.clear();
+    if (c->norms_h) (void)hipHostFree(c->norms_h);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->ex0) (void)hipEventDestroy(c->ex0);

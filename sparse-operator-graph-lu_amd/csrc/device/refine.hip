@@ -22,11 +22,6 @@
 #include "device.h"
 #include "tile_ops.h"
 
-namespace sogl_dev {
-int solve_device(Context* c, Factor* f, const double* d_b, double* d_x, double* d_y, int nrhs);
-int ensure_vectors(Context* c, Factor* f, int nrhs);
-}  // namespace sogl_dev
-
 using namespace sogl_dev;
 
 namespace {
@@ -37,35 +32,18 @@ namespace {
         if (_rc != SOGL_OK) return _rc;                          \
     } while (0)
 
-constexpr int RED_BLOCKS = 256;
+constexpr int RED_BLOCKS = 256;  // blocks of a column group in the residual kernel
 
-// r = b - A x on the permuted padded system, one row per thread, every rhs column
-__global__ void k_residual(const int64_t* ptr, const int32_t* col, const double* val,
-                           const double* b, const double* x, double* r, int64_t N, int nrhs) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    for (int c = 0; c < nrhs; c++) {
-        const double* xc = x + (int64_t)c * N;
-        double s = 0;
-        for (int64_t e = ptr[i]; e < ptr[i + 1]; e++) s = fma(val[e], xc[col[e]], s);
-        r[i + (int64_t)c * N] = b[i + (int64_t)c * N] - s;
-    }
-}
-
-// bp[i] = b[new_order[i]] for i < n, 1 on the padding rows (solver.cpp:155-161 + GPSOrder.cpp:433-447)
+// bp[i] = b[new_order[i]] for i < n, 1 on the padding rows (solver.cpp:155-161 + GPSOrder.cpp:433-447);
+// also zeroes the residual kernel's block counters
 __global__ void k_permute_in(const double* b, const int32_t* new_order, double* bp, int32_t n, int64_t N,
-                             int nrhs) {
+                             int nrhs, int* count, int ncount) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (blockIdx.y == 0)
+        for (int64_t k = i; k < ncount; k += (int64_t)gridDim.x * blockDim.x) count[k] = 0;
     if (i >= N) return;
-    for (int c = 0; c < nrhs; c++) bp[i + c * N] = i < n ? b[new_order[i] + (int64_t)c * n] : 1.0;
-}
-
-// x[new_order[i]] = xp[i] (GOrder::reOrderResult, GPSOrder.cpp:41-53)
-__global__ void k_permute_out(const double* xp, const int32_t* new_order, double* x, int32_t n, int64_t N,
-                              int nrhs) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    for (int c = 0; c < nrhs; c++) x[new_order[i] + (int64_t)c * n] = xp[i + c * N];
+    const int64_t o = i < n ? new_order[i] : 0;
+    for (int c = blockIdx.y; c < nrhs; c += gridDim.y) bp[i + c * N] = i < n ? b[o + (int64_t)c * n] : 1.0;
 }
 
 __global__ void k_axpy(double* x, const double* d, int64_t n) {
@@ -73,53 +51,128 @@ __global__ void k_axpy(double* x, const double* d, int64_t n) {
     if (i < n) x[i] += d[i];
 }
 
-// Per column and block, over the first n rows: the sums of squares of r and x and
-// their largest magnitudes, at out[(c*4 + {0,1,2,3}) * RED_BLOCKS + block].  A NaN
-// reaches the maxima through the sums (fmax drops NaN; the host checks the sums).
-constexpr int RED_VALUES = 4;
-__global__ void k_norms(const double* r, const double* x, int64_t n, int64_t N, double* out) {
-    __shared__ double sr[256], sx[256], mr[256], mx[256];
-    const int c = blockIdx.y;
-    double ar = 0, ax = 0, br = 0, bx = 0;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const double a = r[i + c * N], b = x[i + c * N];
-        ar += a * a;
-        ax += b * b;
-        br = fmax(br, fabs(a));
-        bx = fmax(bx, fabs(b));
+// All that follows a solve, in one launch: r = b - A x on the permuted padded system; x in
+// the caller's order, xo[new_order[i]] = x[i] (GOrder::reOrderResult, GPSOrder.cpp:41-53);
+// per column, over the first n rows, {||r||_2^2, ||x||_2^2, ||b||_2^2, ||r||_inf, ||x||_inf,
+// ||b||_inf} and, after the columns, whether a pass of the solve was aborted, to pinned host
+// memory `norms`, so that the host's one wait brings everything it decides by.  (As a
+// residual, norm, copy and output kernel with a copy of the control words and three waits,
+// and with every column in turn in one thread per row, it was half of a resident solve:
+// random band 4,099 x 100 columns 3.1 of 3.6 ms, 2D 64^2 0.13 of 0.24.)
+// A block takes CW columns (the matrix entries are read once for them); its sums go to
+// part[(column * NORM_VALUES + v) * blocks + block], and the last block of a column group
+// adds them up in block order, so a result does not depend on the blocks' timing.  A NaN
+// reaches the maxima's reader through the sums (fmax drops NaN; the host checks the sums).
+constexpr int NORM_VALUES = 6;
+constexpr int RES_CW = 4;  // columns of a group (one column: 1)
+constexpr int RES_NT = 256;
+
+template <bool MAX>
+__device__ inline double wave_reduce(double v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const double u = __shfl_xor(v, o);
+        v = MAX ? fmax(v, u) : v + u;
     }
-    sr[threadIdx.x] = ar;
-    sx[threadIdx.x] = ax;
-    mr[threadIdx.x] = br;
-    mx[threadIdx.x] = bx;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (threadIdx.x < o) {
-            sr[threadIdx.x] += sr[threadIdx.x + o];
-            sx[threadIdx.x] += sx[threadIdx.x + o];
-            mr[threadIdx.x] = fmax(mr[threadIdx.x], mr[threadIdx.x + o]);
-            mx[threadIdx.x] = fmax(mx[threadIdx.x], mx[threadIdx.x + o]);
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        out[(c * RED_VALUES + 0) * RED_BLOCKS + blockIdx.x] = sr[0];
-        out[(c * RED_VALUES + 1) * RED_BLOCKS + blockIdx.x] = sx[0];
-        out[(c * RED_VALUES + 2) * RED_BLOCKS + blockIdx.x] = mr[0];
-        out[(c * RED_VALUES + 3) * RED_BLOCKS + blockIdx.x] = mx[0];
-    }
+    return v;
 }
 
-// Column c's reduced norms from the per-block partials: {||r||_2^2, ||x||_2^2,
-// ||r||_inf, ||x||_inf}.
-void reduce_norms(const std::vector<double>& part, int c, double out[RED_VALUES]) {
-    for (int v = 0; v < RED_VALUES; v++) {
-        double a = 0;
-        for (int q = 0; q < RED_BLOCKS; q++) {
-            const double p = part[(size_t)((c * RED_VALUES + v) * RED_BLOCKS + q)];
-            a = v < 2 ? a + p : std::max(a, p);
+template <int CW>
+__global__ __launch_bounds__(RES_NT) void k_residual(const int64_t* ptr, const int32_t* col, const double* val,
+                                                     const double* b, const double* x, double* r, double* xo,
+                                                     const int32_t* new_order, int32_t n, int64_t N, int nrhs,
+                                                     double* part, int* count, const int* ctrl, double* norms) {
+    __shared__ double s_w[RES_NT / 64][CW * NORM_VALUES];
+    __shared__ int s_last;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, nb = gridDim.x;
+    const int c0 = blockIdx.y * CW, cw = min(CW, nrhs - c0);
+    const double* xc[CW];  // a column past the last repeats it and is not stored
+#pragma unroll
+    for (int c = 0; c < CW; c++) xc[c] = x + (int64_t)(c0 + min(c, cw - 1)) * N;
+    double acc[CW][NORM_VALUES];
+#pragma unroll
+    for (int c = 0; c < CW; c++)
+#pragma unroll
+        for (int v = 0; v < NORM_VALUES; v++) acc[c][v] = 0;
+    for (int64_t i = (int64_t)blockIdx.x * RES_NT + tid; i < N; i += (int64_t)nb * RES_NT) {
+        double s[CW];
+#pragma unroll
+        for (int c = 0; c < CW; c++) s[c] = 0;
+        int64_t e = ptr[i];
+        const int64_t e1 = ptr[i + 1];
+        for (; e + 4 <= e1; e += 4) {  // four entries' loads in flight
+            double v[4], xv[4][CW];
+            int32_t j[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) j[k] = col[e + k];
+#pragma unroll
+            for (int k = 0; k < 4; k++) v[k] = val[e + k];
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+#pragma unroll
+                for (int c = 0; c < CW; c++) xv[k][c] = xc[c][j[k]];
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+#pragma unroll
+                for (int c = 0; c < CW; c++) s[c] = fma(v[k], xv[k][c], s[c]);
         }
-        out[v] = a;
+        for (; e < e1; e++) {
+            const double v = val[e];
+            const int32_t j = col[e];
+#pragma unroll
+            for (int c = 0; c < CW; c++) s[c] = fma(v, xc[c][j], s[c]);
+        }
+        const int64_t o = i < n ? new_order[i] : 0;
+#pragma unroll
+        for (int c = 0; c < CW; c++) {
+            if (c >= cw) continue;
+            const double bv = b[i + (int64_t)(c0 + c) * N], xv = xc[c][i], rv = bv - s[c];
+            r[i + (int64_t)(c0 + c) * N] = rv;
+            if (i < n) {
+                xo[o + (int64_t)(c0 + c) * n] = xv;
+                acc[c][0] += rv * rv;
+                acc[c][1] += xv * xv;
+                acc[c][2] += bv * bv;
+                acc[c][3] = fmax(acc[c][3], fabs(rv));
+                acc[c][4] = fmax(acc[c][4], fabs(xv));
+                acc[c][5] = fmax(acc[c][5], fabs(bv));
+            }
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < CW; c++)
+#pragma unroll
+        for (int v = 0; v < NORM_VALUES; v++) {
+            const double t = v < 3 ? wave_reduce<false>(acc[c][v]) : wave_reduce<true>(acc[c][v]);
+            if (lane == 0) s_w[w][c * NORM_VALUES + v] = t;
+        }
+    __syncthreads();
+    if (tid < cw * NORM_VALUES) {
+        double t = s_w[0][tid];
+        for (int k = 1; k < RES_NT / 64; k++) t = tid % NORM_VALUES < 3 ? t + s_w[k][tid] : fmax(t, s_w[k][tid]);
+        __hip_atomic_store(part + ((int64_t)c0 * NORM_VALUES + tid) * nb + blockIdx.x, t, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    }
+    wave_stores_done();  // the partials are at the coherence point before the count
+    __syncthreads();
+    if (tid == 0)
+        s_last = __hip_atomic_fetch_add(count + blockIdx.y, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nb - 1;
+    __syncthreads();
+    if (!s_last) return;
+    if (tid == 0) {
+        count[blockIdx.y] = 0;  // for the next launch
+        if (blockIdx.y == 0) norms[(int64_t)nrhs * NORM_VALUES] = ctrl[1] || ctrl[5] ? 1.0 : 0.0;
+    }
+    for (int v = w; v < cw * NORM_VALUES; v += RES_NT / 64) {
+        const double* q = part + ((int64_t)c0 * NORM_VALUES + v) * nb;
+        const bool sum = v % NORM_VALUES < 3;
+        double t = 0;  // (maxima of magnitudes start at 0 too)
+        for (int k = lane; k < nb; k += 64) {
+            const double u = __hip_atomic_load(q + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            t = sum ? t + u : fmax(t, u);
+        }
+        t = sum ? wave_reduce<false>(t) : wave_reduce<true>(t);
+        if (lane == 0) norms[(int64_t)c0 * NORM_VALUES + v] = t;
     }
 }
 
@@ -204,67 +257,66 @@ static int refined_core(Context* c, Factor* f, const double* d_b, double* d_x, i
     const int32_t n = f->n;
     const int64_t N = (int64_t)f->block_rows * TS;
     int rc;
-    if ((rc = ensure_vectors(c, f, nrhs))) return rc;
+    const int cw = nrhs == 1 ? 1 : RES_CW, groups = (nrhs + cw - 1) / cw;
+    const int nb = (int)std::min<int64_t>((N + RES_NT - 1) / RES_NT, RED_BLOCKS);
+    const size_t part_bytes = (size_t)nrhs * NORM_VALUES * RED_BLOCKS * 8, norms = (size_t)nrhs * NORM_VALUES + 1;
+    SolveWork w;
+    if ((rc = ensure_vectors(c, f, nrhs)) || (rc = solve_work(c, f, w))) return rc;
     if ((rc = dev_alloc(c, f->vec_r, (size_t)N * nrhs * 8, "residual")) ||
         (rc = dev_alloc(c, f->vec_d, (size_t)N * nrhs * 8, "correction")) ||
-        (rc = dev_alloc(c, f->red, (size_t)nrhs * RED_VALUES * RED_BLOCKS * 8, "norms")))
+        (rc = dev_alloc(c, f->red, part_bytes + (size_t)groups * sizeof(int), "norms")))
         return rc;
+    if (c->norms_cap < norms) {
+        if (c->norms_h) (void)hipHostFree(c->norms_h);
+        c->norms_h = nullptr;
+        c->norms_cap = 0;
+        HIP_TRY(c, hipHostMalloc((void**)&c->norms_h, norms * 8, hipHostMallocDefault));
+        c->norms_cap = norms;
+    }
+    double* d_norms = nullptr;
+    HIP_TRY(c, hipHostGetDevicePointer((void**)&d_norms, c->norms_h, 0));
     double* db = (double*)f->vec_b.p;
     double* dx = (double*)f->vec_x.p;
     double* dr = (double*)f->vec_r.p;
     double* dd = (double*)f->vec_d.p;
+    int* count = (int*)((char*)f->red.p + part_bytes);
     const unsigned gN = (unsigned)((N + 255) / 256);
     const unsigned gA = (unsigned)((N * nrhs + 255) / 256);
-    hipLaunchKernelGGL(k_permute_in, dim3(gN), dim3(256), 0, c->stream, d_b, (const int32_t*)f->perm_d.p, db, n, N,
-                       nrhs);
+    hipLaunchKernelGGL(k_permute_in, dim3(gN, (unsigned)std::min(nrhs, 65535)), dim3(256), 0, c->stream, d_b,
+                       (const int32_t*)f->perm_d.p, db, n, N, nrhs, count, groups);
     HIP_TRY(c, hipGetLastError());
-    std::vector<double> part((size_t)nrhs * RED_VALUES * RED_BLOCKS);
-    // ||b||_2 and ||b||_inf over the real rows, once
-    hipLaunchKernelGGL(k_norms, dim3(RED_BLOCKS, nrhs), dim3(256), 0, c->stream, db, db, (int64_t)n, N,
-                       (double*)f->red.p);
-    HIP_TRY(c, hipMemcpyAsync(part.data(), f->red.p, part.size() * 8, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
-    std::vector<double> bnorm((size_t)nrhs, 0.0), bmax((size_t)nrhs, 0.0);
-    for (int32_t r = 0; r < nrhs; r++) {
-        double v[RED_VALUES];
-        reduce_norms(part, r, v);
-        bnorm[(size_t)r] = std::sqrt(v[0]);
-        bmax[(size_t)r] = v[2];
-    }
-    if ((rc = solve_device(c, f, db, dx, (double*)f->vec_y.p, nrhs))) return rc;
-    double solve_ms = f->solve_ms;
+    if ((rc = solve_launch(c, f, w, db, dx, nrhs))) return rc;
+    double solve_ms = 0;
     int it = 0;
     double worst = 0;
     for (;;) {
-        hipLaunchKernelGGL(k_residual, dim3(gN), dim3(256), 0, c->stream, (const int64_t*)f->csr_ptr.p,
-                           (const int32_t*)f->csr_col.p, (const double*)f->csr_val.p, db, dx, dr, N, nrhs);
-        hipLaunchKernelGGL(k_norms, dim3(RED_BLOCKS, nrhs), dim3(256), 0, c->stream, dr, dx, (int64_t)n, N,
-                           (double*)f->red.p);
+        auto kern = cw == 1 ? k_residual<1> : k_residual<RES_CW>;
+        hipLaunchKernelGGL(kern, dim3(nb, groups), dim3(RES_NT), 0, c->stream, (const int64_t*)f->csr_ptr.p,
+                           (const int32_t*)f->csr_col.p, (const double*)f->csr_val.p, (const double*)db,
+                           (const double*)dx, dr, d_x, (const int32_t*)f->perm_d.p, n, N, nrhs, (double*)f->red.p, count,
+                           (const int*)w.ctrl, d_norms);
         HIP_TRY(c, hipGetLastError());
-        HIP_TRY(c, hipMemcpyAsync(part.data(), f->red.p, part.size() * 8, hipMemcpyDeviceToHost, c->stream));
         HIP_TRY(c, hipStreamSynchronize(c->stream));
+        float ms = 0;
+        HIP_TRY(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
+        solve_ms += ms;
+        if (c->norms_h[norms - 1] != 0) return solve_timeout(c);
         worst = 0;
         for (int32_t r = 0; r < nrhs; r++) {
-            double v[RED_VALUES];
-            reduce_norms(part, r, v);
-            const double den2 = f->a_fro * std::sqrt(v[1]) + bnorm[(size_t)r];
+            const double* v = c->norms_h + (size_t)r * NORM_VALUES;
+            const double den2 = f->a_fro * std::sqrt(v[1]) + std::sqrt(v[2]);
             const double rel2 = den2 > 0 ? std::sqrt(v[0]) / den2 : std::sqrt(v[0]);
-            const double deni = f->a_inf * v[3] + bmax[(size_t)r];
-            const double reli = deni > 0 ? v[2] / deni : v[2];
+            const double deni = f->a_inf * v[4] + v[5];
+            const double reli = deni > 0 ? v[3] / deni : v[3];
             const double rel = std::isnan(rel2) ? rel2 : std::max(rel2, reli);
             if (!(rel <= worst)) worst = rel;  // NaN propagates
         }
         if (worst <= tol || it >= max_iter || std::isnan(worst)) break;
-        if ((rc = solve_device(c, f, dr, dd, (double*)f->vec_y.p, nrhs))) return rc;
-        solve_ms += f->solve_ms;
+        if ((rc = solve_launch(c, f, w, dr, dd, nrhs))) return rc;
         hipLaunchKernelGGL(k_axpy, dim3(gA), dim3(256), 0, c->stream, dx, (const double*)dd, N * nrhs);
         HIP_TRY(c, hipGetLastError());
         it++;
     }
-    hipLaunchKernelGGL(k_permute_out, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, (const double*)dx,
-                       (const int32_t*)f->perm_d.p, d_x, n, N, nrhs);
-    HIP_TRY(c, hipGetLastError());
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
     f->solve_ms = solve_ms;
     if (iters) *iters = it;
     if (resid) *resid = worst;

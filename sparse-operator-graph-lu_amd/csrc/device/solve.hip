@@ -45,7 +45,7 @@ struct SolveArgs {
     int32_t nrhs;
     int32_t nbr;
     int32_t forward;
-    int* ctrl;            // [0] task counter, [1] abort
+    int* ctrl;            // the pass's: [0] task counter, [1] abort
     const uint32_t* mask; // per slot: the factor's 16x16 block masks (a zero tile is skipped)
     const int32_t* prow;     // the many-RHS form's steps (pair_steps): per row pair, its steps'
     const int32_t* pcol;     // block column pairs
@@ -59,15 +59,20 @@ struct SolveArgs {
 constexpr int SOLVE_SPIN_CHECK = 64;
 
 // Rows of the output that a pass has not stored yet hold this signalling NaN, written by
-// k_fill_pending before the pass.  FP arithmetic never produces a signalling NaN (a NaN
+// k_solve_begin before the pass.  FP arithmetic never produces a signalling NaN (a NaN
 // result is quiet), so a stored value is never mistaken for it.  A task polls the values it
 // reads themselves, with agent-scope atomic loads, until none is the marker, and stores its
 // rows with agent-scope atomic stores, which reach the coherence point without a release.
 constexpr unsigned long long SOLVE_PENDING = 0x7FF4C0DE5EED0001ull;
 
-__global__ void k_fill_pending(double* out, int64_t n) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        reinterpret_cast<unsigned long long*>(out)[i] = SOLVE_PENDING;
+// Before the two passes: the outputs of both pending, the task counters of both (ctrl[0],
+// ctrl[4]) at zero and, before the first columns, their abort words (ctrl[1], ctrl[5]).
+__global__ void k_solve_begin(int* ctrl, int first, double* y, double* x, int64_t n) {
+    if (blockIdx.x == 0 && threadIdx.x < SOLVE_CTRL_WORDS && (first || threadIdx.x % 4 == 0)) ctrl[threadIdx.x] = 0;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+        reinterpret_cast<unsigned long long*>(y)[i] = SOLVE_PENDING;
+        reinterpret_cast<unsigned long long*>(x)[i] = SOLVE_PENDING;
+    }
 }
 
 // The 64 values of one column of row J, which another task stores, into this wave's
@@ -639,10 +644,6 @@ __global__ __launch_bounds__(NTP) void k_trsm_persistent(SolveArgs a) {
     }
 }
 
-__global__ void k_solve_ctrl_reset(int* ctrl) {
-    if (threadIdx.x < 4) ctrl[threadIdx.x] = 0;
-}
-
 // out = diag(L) y over the padded rows, every column: the forward result as the
 // reference's lowerSolver leaves it in its right-hand side, b_i = l_ii y_i (for a
 // unit-diagonal L that is y itself).
@@ -664,13 +665,6 @@ namespace {
         if (_rc != SOGL_OK) return _rc;                          \
     } while (0)
 
-// Buffers of one solve beyond its input and output: the forward result y (padded n x
-// nrhs) and the control words.
-struct SolveWork {
-    double* y;
-    int* ctrl;
-};
-
 template <typename T>
 int launch_pass(Context* c, Factor* f, const SolveWork& w, bool mfma, bool forward, const double* in, double* out,
                 int nrhs) {
@@ -686,17 +680,12 @@ int launch_pass(Context* c, Factor* f, const SolveWork& w, bool mfma, bool forwa
     a.nrhs = nrhs;
     a.nbr = f->block_rows;
     a.forward = forward ? 1 : 0;
-    a.ctrl = w.ctrl;
+    a.ctrl = w.ctrl + (forward ? 0 : 4);
     a.mask = (const uint32_t*)f->mask_d.p;
     a.prow = (const int32_t*)(forward ? f->lstep_ptr.p : f->ustep_ptr.p);
     a.pcol = (const int32_t*)(forward ? f->lstep_col.p : f->ustep_col.p);
     a.pslot = (const int4*)(forward ? f->lstep_slot.p : f->ustep_slot.p);
     a.pairinv = (const int32_t*)(forward ? f->pairx_d.p : f->pairy_d.p);
-    hipLaunchKernelGGL(k_solve_ctrl_reset, dim3(1), dim3(64), 0, c->stream, a.ctrl);
-    // the rows of out are pending until their task stores them
-    const int64_t n = a.ld * nrhs;
-    const unsigned fg = (unsigned)std::min<int64_t>((n + 255) / 256, 2048);
-    hipLaunchKernelGGL(k_fill_pending, dim3(fg), dim3(256), 0, c->stream, out, n);
     const int64_t ntask = (int64_t)((a.nbr + 1) / 2) * (mfma ? (nrhs + PC - 1) / PC : nrhs);
     auto kern = mfma ? k_trsm_persistent<T> : k_trsv_persistent<T, false>;
     if constexpr (sizeof(T) == 8)
@@ -712,8 +701,9 @@ int launch_pass(Context* c, Factor* f, const SolveWork& w, bool mfma, bool forwa
 
 }  // namespace
 
-// Both passes over nrhs columns on the context stream, timed; d_x may not alias d_b.
-int solve_core(Context* c, Factor* f, const SolveWork& w, const double* d_b, double* d_x, int nrhs) {
+// Both passes over nrhs columns, enqueued on the context stream between the events ev0 and
+// ev1; d_x may not alias d_b.  solve_finish waits and looks at the outcome.
+int solve_launch(Context* c, Factor* f, const SolveWork& w, const double* d_b, double* d_x, int nrhs) {
     const int R = f->block_rows;
     int rc;
     HIP_TRY(c, hipEventRecord(c->ev0, c->stream));
@@ -721,7 +711,9 @@ int solve_core(Context* c, Factor* f, const SolveWork& w, const double* d_b, dou
     const bool mfma = nrhs >= TRSM_MIN_RHS;
     for (int c0 = 0; c0 < nrhs; c0 += MAX_RHS) {
         const int m = std::min(MAX_RHS, nrhs - c0);
-        const int64_t off = (int64_t)c0 * ld;
+        const int64_t off = (int64_t)c0 * ld, n = ld * m;
+        const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 2048));
+        hipLaunchKernelGGL(k_solve_begin, dim3(grid), dim3(256), 0, c->stream, w.ctrl, c0 == 0, w.y + off, d_x + off, n);
         if (f->elem == 8) {
             if ((rc = launch_pass<double>(c, f, w, mfma, true, d_b + off, w.y + off, m))) return rc;
             if ((rc = launch_pass<double>(c, f, w, mfma, false, w.y + off, d_x + off, m))) return rc;
@@ -731,21 +723,40 @@ int solve_core(Context* c, Factor* f, const SolveWork& w, const double* d_b, dou
         }
     }
     HIP_TRY(c, hipEventRecord(c->ev1, c->stream));
+    return SOGL_OK;
+}
+
+int solve_timeout(Context* c) {
+    return set_error(c, SOGL_ERR_TIMEOUT, "solve: a dependency wait exceeded its bound");
+}
+
+int solve_finish(Context* c, Factor* f, const SolveWork& w) {
     HIP_TRY(c, hipEventSynchronize(c->ev1));
     float ms = 0;
     HIP_TRY(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
     f->solve_ms = ms;
-    int ctrl[4];
+    int ctrl[SOLVE_CTRL_WORDS];
     HIP_TRY(c, hipMemcpy(ctrl, w.ctrl, sizeof(ctrl), hipMemcpyDeviceToHost));
-    if (ctrl[1]) return set_error(c, SOGL_ERR_TIMEOUT, "solve: a dependency wait exceeded its bound");
+    return ctrl[1] || ctrl[5] ? solve_timeout(c) : SOGL_OK;
+}
+
+int solve_core(Context* c, Factor* f, const SolveWork& w, const double* d_b, double* d_x, int nrhs) {
+    const int rc = solve_launch(c, f, w, d_b, d_x, nrhs);
+    return rc ? rc : solve_finish(c, f, w);
+}
+
+// With the factor's own control words (allocated on first use) and y.
+int solve_work(Context* c, Factor* f, SolveWork& w) {
+    int rc;
+    if ((rc = dev_alloc(c, f->solve_ctrl, SOLVE_CTRL_WORDS * sizeof(int), "solve control"))) return rc;
+    w = SolveWork{(double*)f->vec_y.p, (int*)f->solve_ctrl.p};
     return SOGL_OK;
 }
 
-// With the factor's own control words (allocated on first use).
-int solve_device(Context* c, Factor* f, const double* d_b, double* d_x, double* d_y, int nrhs) {
+int solve_device(Context* c, Factor* f, const double* d_b, double* d_x, int nrhs) {
+    SolveWork w;
     int rc;
-    if ((rc = dev_alloc(c, f->solve_ctrl, 16, "solve control"))) return rc;
-    const SolveWork w{d_y, (int*)f->solve_ctrl.p};
+    if ((rc = solve_work(c, f, w))) return rc;
     return solve_core(c, f, w, d_b, d_x, nrhs);
 }
 
@@ -776,7 +787,7 @@ extern "C" int sogl_solve(sogl_ctx* x, int32_t factor_id, const double* bp, doub
     if ((rc = ensure_vectors(c, f, nrhs))) return rc;
     const size_t bytes = (size_t)f->block_rows * TS * nrhs * 8;
     HIP_TRY(c, hipMemcpyAsync(f->vec_b.p, bp, bytes, hipMemcpyHostToDevice, c->stream));
-    if ((rc = solve_device(c, f, (const double*)f->vec_b.p, (double*)f->vec_x.p, (double*)f->vec_y.p, nrhs)))
+    if ((rc = solve_device(c, f, (const double*)f->vec_b.p, (double*)f->vec_x.p, nrhs)))
         return rc;
     HIP_TRY(c, hipMemcpyAsync(xp, f->vec_x.p, bytes, hipMemcpyDeviceToHost, c->stream));
     if (y && f->llt) {
@@ -809,7 +820,7 @@ extern "C" int sogl_solve_device(sogl_ctx* x, int32_t factor_id, const double* d
     HIP_TRY(c, hipSetDevice(c->device));
     int rc;
     if ((rc = ensure_vectors(c, f, nrhs))) return rc;
-    return solve_device(c, f, d_bp, d_xp, (double*)f->vec_y.p, nrhs);
+    return solve_device(c, f, d_bp, d_xp, nrhs);
 }
 
 // ------------------------------------------------------------------ solve without allocation

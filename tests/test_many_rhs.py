@@ -6,6 +6,7 @@ import pytest
 import scipy.linalg as sl
 
 import sogl
+import workloads as W
 
 pytestmark = pytest.mark.gpu
 
@@ -85,3 +86,27 @@ def test_more_columns_than_a_launch(dev):
     dev.release(fid)
     want = sl.solve_triangular(Uf, sl.solve_triangular(Lf, b, lower=True), lower=False)
     assert np.abs(x - want).max() / np.abs(want).max() < 1e-12
+
+
+@pytest.mark.parametrize("nrhs", [1, 3, 4, 5])
+def test_residual_columns(dev, nrhs):
+    """The refinement's residual and norms by column groups of four: an FP32 factor's first solve,
+    its reported backward error (the largest over the columns) against the formula in numpy.
+    The residual is about 1e-7 of |A||x|, so FP64 rounding changes it by about 1e-8."""
+    p = W.convdiff2d(37)
+    b = W.uniform_pm1(3, p.n * nrhs).reshape(nrhs, p.n).T.copy() * 10.0 ** np.arange(nrhs)
+    plan = sogl.Plan(p.n, p.row, p.col, p.val, b[:, 0])
+    fid = dev.load(plan, sogl.FP32)
+    dev.factor(fid)
+    dev.attach_refine(fid, plan)
+    x, it, resid, rc = dev.solve_refined(fid, b, tol=1.0, max_iter=5)
+    dev.release(fid)
+    x = np.asarray(x).reshape(p.n, nrhs)
+    assert rc == 0 and it == 0
+    row_sums = np.bincount(p.row, weights=np.abs(p.val), minlength=p.n)
+    want = 0.0
+    for c in range(nrhs):
+        r = b[:, c] - np.bincount(p.row, weights=p.val * x[p.col, c], minlength=p.n)
+        want = max(want, np.linalg.norm(r) / (np.linalg.norm(p.val) * np.linalg.norm(x[:, c]) + np.linalg.norm(b[:, c])),
+                   np.abs(r).max() / (row_sums.max() * np.abs(x[:, c]).max() + np.abs(b[:, c]).max()))
+    assert 0 < want < 1e-5 and abs(resid - want) < 1e-6 * want
