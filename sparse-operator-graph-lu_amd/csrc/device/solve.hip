@@ -75,6 +75,13 @@ __global__ void k_solve_begin(int* ctrl, int first, double* y, double* x, int64_
     }
 }
 
+// A wait has exceeded its bound: every task ends.  A release, so that whoever sees the word
+// sees all that this wave stored before it.
+__device__ inline void raise_abort(const SolveArgs& a) {
+    release_agent();
+    __hip_atomic_store(a.ctrl + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // The 64 values of one column of row J, which another task stores, into this wave's
 // LDS slot ls once all are stored: lane l polls value l (one coalesced load per spin
 // for the wave), the wave's ballot says when none is pending.  NC = 2 polls the same
@@ -101,7 +108,7 @@ __device__ inline void load_row_stored(const double* col, double* ls, int lane, 
         } else if (spin % SOLVE_SPIN_CHECK == 0 &&
                    (__hip_atomic_load(a.ctrl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ||
                     wall_clock64() - t0 > SOLVE_SPIN_LIMIT)) {
-            __hip_atomic_store(a.ctrl + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            raise_abort(a);
 #pragma unroll
             for (int i = 0; i < NC; i++) u[i] = 0;  // the bit pattern of 0.0
             break;
@@ -566,7 +573,7 @@ __global__ __launch_bounds__(NTP) void k_trsm_persistent(SolveArgs a) {
                     if (spin % SOLVE_SPIN_CHECK == 0 &&
                         (__hip_atomic_load(a.ctrl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ||
                          wall_clock64() - t0 > SOLVE_SPIN_LIMIT)) {
-                        __hip_atomic_store(a.ctrl + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        raise_abort(a);
 #pragma unroll
                         for (int i = 0; i < 4; i++) s.x[i] = 0.0;
                         break;
