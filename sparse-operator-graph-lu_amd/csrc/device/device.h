@@ -74,12 +74,28 @@ struct DevTask {
     // (a GEMM on the critical path that reads an output of this one; it waits for its
     // other operands like a queued task and is not handed out by the queue), or -1
     int32_t after = -1;
-    // lu (FP32 LU factors, persistent executor): the panel GEMMs this task runs inside
+    // lu (FP32 and FP64 LU factors, persistent executor): the panel GEMMs this task runs inside
     // itself, before publishing, from the inverses it keeps in LDS: pan_l = A U^-1 (its
     // U^-1 the second operand), pan_u = L^-1 A (its L^-1 the first); -1: none
     int32_t pan_l = -1, pan_u = -1;
-    int32_t pad[3] = {0, 0, 0};
+    // lu (persistent executor, with both panels): the GEMM of the next diagonal tile's last
+    // update, pan_l's tile times pan_u's, whose lu (its `next`) the same workgroup goes on
+    // with (diagonal chains); -1: none
+    int32_t dia = -1;
+    int32_t rec = -1;  // and its DiagRec; -1: none
+    int32_t pad[1] = {0};
 };
+
+// All that a diagonal chain's step needs beyond its lu's task, in one line (slots, and the
+// value ids that index the flags): the tiles its two panels and the update read (S_l, S_u,
+// P), those they make, the lu that follows, and the tasks' indices.
+struct DiagRec {
+    int32_t s_l, f_sl, s_u, f_su, p, f_p;
+    int32_t o_l, f_ol, o_u, f_ou, o_d, next;
+    int32_t neg;  // bit 0 / 1: panel l / u negated, 2: the product, 3: P
+    int32_t pan_l, pan_u, dia;
+};
+static_assert(sizeof(DiagRec) == 64, "one cache line half");
 
 // One check entry of a task's chain candidates: candidate `task` (index `cand` in the
 // list) reads `slot` at operand position `pos` (0-3: pair lanes, 4: the added tile);
@@ -123,12 +139,14 @@ struct Factor {
     int64_t n_chained = 0;      // lu / llt tasks run by the workgroup that made their source
     int64_t n_pair_tasks = 0;   // GEMM tasks making the solve's two-row blocks X_p / Y_p
     // device arrays
-    DevBuf pool, tasks_d, pairs_d, deps_d, ready_d, ctrl_d, op_tasks_d, op_pairs_d, inputs_d, queue_d, chk_d;
+    DevBuf pool, tasks_d, pairs_d, deps_d, ready_d, ctrl_d, op_tasks_d, op_pairs_d, inputs_d, queue_d, chk_d, diag_d;
     std::vector<ChainChk> chk;             // chain candidates' check entries (see DevTask)
     int64_t n_chain_cands = 0;             // tasks that are some task's chain candidate
     bool after_links = false;              // build after-links (set from the context at load)
     bool absorb_panels = false;            // let lu tasks absorb a panel GEMM (set from the context)
     int64_t n_absorbed = 0;                // panel GEMMs absorbed by their lu task
+    std::vector<DiagRec> diag;             // diagonal chains' steps (device copy: diag_d)
+    int32_t n_diag_chains = 0;             // diagonal chains (build_diag_chains)
     int64_t n_after = 0;                   // after-links (tasks run by their producer's workgroup)
     bool tile_order = false;               // the op list is in tile-column order (tile_order.h)
     std::vector<int32_t> chain_head;       // per task: the queued task whose workgroup runs it

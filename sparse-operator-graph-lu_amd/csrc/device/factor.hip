@@ -25,6 +25,7 @@
 #include <deque>
 #include <map>
 #include <new>
+#include <set>
 #include <string>
 #include <vector>
 
@@ -177,6 +178,7 @@ struct Args {
     uint32_t* mask;       // per slot: 16x16 block mask of the tile (see tile_ops.h)
     const ChainChk* chk;  // persistent executor: chain candidates' check entries
     int32_t chain;        // claims per finished task at most (0: no dynamic chaining)
+    const DiagRec* diag;
     const int32_t* war;   // value ids whose readers a reused result slot waits for (DevTask)
 };
 
@@ -406,7 +408,7 @@ struct PairWait {
 // slot's first value in the run (no cache holds an earlier one), and this CU's own
 // caches have its stores, which coherent loads could pass (the chain does not wait for
 // them).
-// xcopy / zcopy (FP32 LU kernels of the persistent executor): LDS for the copies of the
+// xcopy / zcopy (LU kernels of the persistent executor): LDS for the copies of the
 // inverses an lu task with absorbed panels keeps.  Returns an lu task's growth (1
 // otherwise).
 template <typename T, bool BF16, bool ACC, bool LLT, bool MASKS, bool ONE = false, bool COH = false, typename Wait>
@@ -442,7 +444,7 @@ __device__ __attribute__((always_inline)) double run_task(const DevTask& t, cons
                     }
                 } else {
                     g = lu_task<T>(pool, t.a, t.out0, t.out1, t.out2, t.out3, lds, a.growth_limit, a.ctrl + 2,
-                                   COH && !chained, nullptr, nullptr, LDS_HANDOFF && chained);
+                                   COH && !chained, xcopy, zcopy, LDS_HANDOFF && chained);
                 }
             }
             break;
@@ -518,6 +520,172 @@ __device__ __attribute__((always_inline)) void absorbed_panel(const Args& a, con
     }
 }
 
+// One step of a diagonal chain, inside the lu task of block column k, after its elimination:
+//     L_{k+1,k} = S_{k+1,k} U_kk^-1,   U_{k,k+1} = L_kk^-1 S_{k,k+1}   (its panels pl, pu)
+//     S_{k+1,k+1} = P - L_{k+1,k} U_{k,k+1}                            (its update pd)
+// from the inverses' copies and through LDS, where the lu of k + 1 that this workgroup runs
+// next takes the sum.  The chain through the diagonal, which bounds narrow graphs, is then
+// lu, two panels and a product per block row with no publish, hand-off or operand load from
+// another workgroup between them but the loads of S (sums made elsewhere meanwhile).
+// The lu's own tiles are published as soon as those loads are in (the same wait), the panels
+// after the product; the sum is read by nobody else.  Products, signs and masks are the
+// GEMM tasks' own, so the bits are.  A block row of C5 FP32 takes 14.8 us (18 before): the lu
+// 8.4, the flags of S 0.4, this step 4.8 (S's loads 1.3; the products 2.0 at the FP32 matrix
+// rate), the way to the next lu 1.1; of 2D 64^2 FP64 25 (26.4): 15.2, 0.4, 8.3, 1.4.
+template <typename T, bool MASKS, bool COH>
+__device__ __attribute__((always_inline)) void diag_step(const Args& a, const DevTask& lu, const DiagRec& d, char* lds,
+                                                         T* xcopy, T* zcopy, bool refactored,
+                                                         uint32_t (*s_pmask)[NT / 64], uint32_t* s_words,
+                                                         unsigned long long want, long long* t_wait) {
+    typedef typename MfmaOp<T>::acc_t acc_t;
+    T* pool = reinterpret_cast<T*>(a.pool);
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wr = (w >> 1) * 32, wc = (w & 1) * 32, li = lane & 15, lk = lane >> 4;
+    constexpr int LDA = lda<T>();
+    T* la = reinterpret_cast<T*>(lds);
+    T* lb = la + TS * LDA;
+    if (tid < 3) s_words[tid] = (uint32_t)spin_ready(a, tid == 0 ? d.f_sl : tid == 1 ? d.f_su : d.f_p) & MASK_ALL;
+    if (refactored) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the inverses are read back below
+    __syncthreads();
+    if (a.trace && tid == 0) *t_wait = wall_clock64();
+    const uint32_t ml = __builtin_amdgcn_readfirstlane(s_words[0]), mu = __builtin_amdgcn_readfirstlane(s_words[1]);
+    {
+        Seg<T> gl, gu;
+        seg_load<COH>(pool + (size_t)d.s_l * TE, gl, tid, !MASKS || seg_on<T>(ml, tid));
+        seg_load<COH>(pool + (size_t)d.s_u * TE, gu, tid, !MASKS || seg_on<T>(mu, tid));
+        seg_store(gl, la, LDA, tid, !MASKS || seg_on<T>(ml, tid), d.neg & 1);
+        seg_store(gu, lb, LDB, tid, !MASKS || seg_on<T>(mu, tid), (d.neg >> 1) & 1);
+    }
+    if (refactored) {
+        tile_to_lds<true>(pool + (size_t)lu.out3 * TE, zcopy, LDB, tid);
+        tile_to_lds<true>(pool + (size_t)lu.out2 * TE, xcopy, LDA, tid);
+    }
+    wave_stores_done();  // the lu's
+    __syncthreads();
+    if (tid == 0) {
+        const unsigned long long fv = want | MASK_ALL;
+        for (int32_t fl : {lu.f0, lu.f1, lu.f2, lu.f3})
+            if (fl >= 0) __hip_atomic_store(a.ready + fl, fv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    // the next lu's task and record into this XCD's L2 meanwhile (from HBM on a long factor)
+    int warm = 0;
+    if (w == 3 && lane < 3)
+        warm = lane < 2 ? reinterpret_cast<const int32_t*>(a.tasks + d.next)[lane * (sizeof(DevTask) / 4 - 1)]
+                        : a.diag[lu.rec + 1].s_l;  // (the array ends with one more)
+    acc_t acc[2][2], xr[2][2];
+    auto zero = [&]() {
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int n = 0; n < 2; n++) acc[m][n] = acc_t{0, 0, 0, 0};
+    };
+    // A panel: A U^-1 (UPPER: column block J of the product needs the k blocks up to J) or
+    // L^-1 A (row block I the k blocks up to I).  Waves take blocks {0, 3} or {1, 2} of the
+    // triangle's side, five of its eight block products each, and two neighbours of the
+    // other.  (The products left out are with the inverse's zero blocks.)
+    auto panel = [&](auto upper, const T* A, const T* B, uint32_t mo, int32_t out, T* dst, int ld, bool neg,
+                     uint32_t* out_mask) {
+        constexpr bool UPPER = decltype(upper)::value;
+        const int tri[2] = {w & 1, 3 - (w & 1)}, oth[2] = {2 * (w >> 1), 2 * (w >> 1) + 1};
+        const int* I = UPPER ? oth : tri;
+        const int* J = UPPER ? tri : oth;
+        zero();
+        // the k blocks in which the other operand's blocks are not all zero
+        uint32_t use = 0xFu;
+        if constexpr (MASKS) {
+            const uint32_t x = UPPER ? mo : mask_transpose(mo);
+            use = mask_row(x, oth[0]) | mask_row(x, oth[1]);
+        }
+#pragma unroll
+        for (int K = 0; K < 4; K++) {
+            if (K > tri[1] || !((use >> K) & 1u)) continue;  // wave-uniform
+            const int k0 = 16 * K + 4 * lk;
+            T av[2][4], bv[2][4];
+#pragma unroll
+            for (int m = 0; m < 2; m++) read4(A + (16 * I[m] + li) * LDA + k0, av[m]);
+#pragma unroll
+            for (int n = 0; n < 2; n++)
+#pragma unroll
+                for (int k4 = 0; k4 < 4; k4++) bv[n][k4] = B[(k0 + k4) * LDB + 16 * J[n] + li];
+            const bool both = K <= tri[0];  // wave-uniform
+#pragma unroll
+            for (int k4 = 0; k4 < 4; k4++)
+#pragma unroll
+                for (int m = 0; m < 2; m++)
+#pragma unroll
+                    for (int n = 0; n < 2; n++)
+                        if (both || (UPPER ? n : m) == 1) acc[m][n] = MfmaOp<T>::mma(av[m][k4], bv[n][k4], acc[m][n]);
+        }
+        T* C = pool + (size_t)out * TE;
+        uint32_t bits = 0;
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int n = 0; n < 2; n++) {
+                acc_store_global(acc[m][n], C, 16 * I[m], 16 * J[n], li, lk);
+                if constexpr (MASKS)
+                    if (__ballot(acc_nonzero(acc[m][n], MASK_TINY)) != 0) bits |= 1u << (4 * I[m] + J[n]);
+            }
+        if constexpr (MASKS)
+            if (lane == 0) out_mask[w] = bits;
+        __syncthreads();  // every wave is done reading the tile
+        // (a block that counts as zero is zero for its readers)
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int n = 0; n < 2; n++) {
+                if (MASKS && !((bits >> (4 * I[m] + J[n])) & 1u)) acc[m][n] = acc_t{0, 0, 0, 0};
+                acc_store<T>(neg ? -acc[m][n] : acc[m][n], dst + 16 * I[m] * ld + 16 * J[n], ld, li, lk);
+            }
+    };
+    auto keep = [&](T* d, int ld, bool neg) {  // the accumulators into LDS
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int n = 0; n < 2; n++)
+                acc_store<T>(neg ? -acc[m][n] : acc[m][n], d + (wr + m * 16) * ld + wc + n * 16, ld, li, lk);
+    };
+#pragma unroll
+    for (int m = 0; m < 2; m++)
+#pragma unroll
+        for (int n = 0; n < 2; n++) xr[m][n] = acc_load_global<COH>(pool + (size_t)d.p * TE, wr + m * 16, wc + n * 16, li, lk);
+    panel(std::true_type{}, la, zcopy, ml, d.o_l, la, LDA, (d.neg >> 2) & 1, s_pmask[0]);
+    panel(std::false_type{}, xcopy, lb, mu, d.o_u, lb, LDB, false, s_pmask[1]);
+    __syncthreads();
+    uint32_t ma = MASK_ALL, mb = MASK_ALL;
+    if constexpr (MASKS) {
+        ma = __builtin_amdgcn_readfirstlane(s_pmask[0][0] | s_pmask[0][1] | s_pmask[0][2] | s_pmask[0][3]);
+        mb = __builtin_amdgcn_readfirstlane(s_pmask[1][0] | s_pmask[1][1] | s_pmask[1][2] | s_pmask[1][3]);
+    }
+    zero();
+    if (!MASKS || (ma != 0 && mb != 0)) {
+        uint32_t kuse = 0xFu;
+        if constexpr (MASKS) kuse = k_blocks_used(ma, mb, wr >> 4, wc >> 4);
+        gemm_lds<T, false, true>(acc, la, lb, wr, wc, li, lk, kuse);
+    }
+#pragma unroll
+    for (int m = 0; m < 2; m++)
+#pragma unroll
+        for (int n = 0; n < 2; n++) acc[m][n] += (d.neg >> 3) & 1 ? -xr[m][n] : xr[m][n];
+    asm volatile("" ::"v"(warm));
+    wave_stores_done();  // the panels'
+    __syncthreads();     // and every wave is done reading la and lb
+    if (tid == 0) {
+        __hip_atomic_store(a.ready + d.f_ol, want | ma, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(a.ready + d.f_ou, want | mb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        gst(&a.mask[d.o_l], ma);
+        gst(&a.mask[d.o_u], mb);
+        gst(&a.mask[d.o_d], MASK_ALL);
+    }
+    keep(la, LDA, false);
+    // (an FP64 refactorisation of the next lu reads the sum from memory)
+#pragma unroll
+    for (int m = 0; m < 2; m++)
+#pragma unroll
+        for (int n = 0; n < 2; n++)
+            acc_store_global(acc[m][n], pool + (size_t)d.o_d * TE, wr + m * 16, wc + n * 16, li, lk);
+}
+
 // Block mask of a finished task's outputs (thread 0, after the task's last barrier):
 // GEMM, sub and transpose tasks leave their waves' bits in s_mask; the tiles of lu /
 // llt and the inverses, and everything when masks are off, count as full.
@@ -549,11 +717,11 @@ constexpr int CHAIN_MAX_CANDS = 16;    // claim bits 16..31 of a ready flag
 constexpr int CHAIN_MAX_CHECKS = 64;   // check entries per task: one lane of wave 0 each
 template <typename T, bool BF16, bool LLT, bool MASKS, bool ONE, bool COH>
 __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
-    // FP32 LU kernels built for one workgroup per CU: lu tasks run their panel GEMMs
+    // LU kernels built for one workgroup per CU: lu tasks run their panel GEMMs
     // (DevTask::pan_l / pan_u) inside themselves, keeping copies of the inverses in LDS
     // beyond what any task kind uses.  The kernels built for two (no registers to spare)
     // run them as after-links instead: right after the lu, in the same workgroup.
-    constexpr bool ABSORB = sizeof(T) == 4 && !BF16 && !LLT && ONE;
+    constexpr bool ABSORB = !BF16 && !LLT && ONE;
     constexpr int XCOPY_BYTES = ABSORB ? TS * lda<T>() * (int)sizeof(T) : 0;
     constexpr int ZCOPY_BYTES = ABSORB ? TS * LDB * (int)sizeof(T) : 0;
     __shared__ __attribute__((aligned(16))) char lds[lds_bytes<T>() + XCOPY_BYTES + ZCOPY_BYTES];
@@ -561,7 +729,10 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
     T* const zcopy = ABSORB ? reinterpret_cast<T*>(lds + lds_bytes<T>() + XCOPY_BYTES) : nullptr;
     __shared__ uint32_t s_pmask[2][NT / 64];
     __shared__ uint32_t s_word;
-    __shared__ int s_pend;  // an absorbed panel still to run as an after-link (kernels without the copies)
+    // an absorbed panel, and the next diagonal tile's update, still to run as after-links
+    // (kernels without the copies)
+    __shared__ int s_pend, s_pend_d;
+    __shared__ uint32_t s_words[3];
     __shared__ int s_task;
     __shared__ int s_abort;
     __shared__ int s_lost;
@@ -582,7 +753,7 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
             s_abort = __hip_atomic_load(a.ctrl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             s_task = s_abort ? a.nqueue : atomicAdd(a.ctrl, a.chunk);
             s_ring_head = s_ring_n = 0;
-            s_pend = -1;
+            s_pend = s_pend_d = -1;
         }
         __syncthreads();
         // wave-uniform loop control: the exit branch must not depend on the lane
@@ -603,7 +774,7 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
         for (;;) {
         const DevTask t = const_load(a.tasks + ti);
         const int nxt = __builtin_amdgcn_readfirstlane(t.next);
-        long long t_taken = 0, t_ready = 0, t_wait = 0;
+        long long t_taken = 0, t_ready = 0, t_wait = 0, t_done = 0;
         if (a.trace && tid == 0) t_taken = wall_clock64();
         if (t.kind != TK_GEMM && (mode == 0 || mode == 3)) {
             if (tid == 0) {
@@ -637,7 +808,9 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
         // (with dynamic chaining on, panels run as after-links, whose outputs' candidates
         // can be claimed)
         const bool absorbs = ABSORB && !a.chain && t.kind == TK_LU && (t.pan_l >= 0 || t.pan_u >= 0);
-        const bool has_l = absorbs && t.pan_l >= 0, has_u = absorbs && t.pan_u >= 0;
+        const bool has_d = absorbs && t.rec >= 0;
+        const bool has_l = absorbs && !has_d && t.pan_l >= 0, has_u = absorbs && !has_d && t.pan_u >= 0;
+        const DiagRec dr = const_load(a.diag + (has_d ? t.rec : 0));
         const DevTask pdl = const_load(a.tasks + (has_l ? t.pan_l : ti));
         const DevTask pdu = const_load(a.tasks + (has_u ? t.pan_u : ti));
         // the task this workgroup runs next (the static chain): touch its descriptor now,
@@ -654,12 +827,15 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
             t, a, lds, s_mask,
             PairWait{&a, &t_wait, s_pm, mode == 2 ? s_pre : nullptr, mode == 0 ? t.ctag : 0, &s_lost, t.war_begin,
                      t.war_count},
-            mode == 1, has_u ? xcopy : nullptr, has_l ? zcopy : nullptr, nxt >= 0);
+            mode == 1, has_u || has_d ? xcopy : nullptr, has_l || has_d ? zcopy : nullptr, nxt >= 0);
         if (nxt >= 0) asm volatile("" ::"s"(pf0), "s"(pf1), "s"(pf2));
         if constexpr (ABSORB) {
             if (absorbs) {
                 __syncthreads();  // the lu's LDS (the inverses' copies included) is complete
                 const bool refactored = !(growth <= a.growth_limit);
+                if (a.trace && tid == 0) t_done = wall_clock64();
+                if (has_d)
+                    diag_step<T, MASKS, COH>(a, t, dr, lds, xcopy, zcopy, refactored, s_pmask, s_words, want, &t_wait);
                 if (has_l) absorbed_panel<T, MASKS, COH>(a, t, pdl, true, lds, zcopy, refactored, s_pmask[0], &s_word);
                 if (has_l && has_u) __syncthreads();  // the first panel's operands leave LDS
                 if (has_u) absorbed_panel<T, MASKS, COH>(a, t, pdu, false, lds, xcopy, refactored, s_pmask[1], &s_word);
@@ -675,7 +851,8 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
         // claims of this workgroup.  A sum that goes to the chained task is read by nobody
         // else: no wait, no flag (the chained task runs on this CU and reads it after the
         // barrier).
-        if (nxt < 0) wave_stores_done();
+        // (A diagonal chain's step has published its lu and panels and goes on the same way.)
+        if (nxt < 0 && !has_d) wave_stores_done();
         __syncthreads();
         if (a.trace && tid == 0) t_ready = wall_clock64();  // work done, publish starts
         uint32_t claims = 0;
@@ -703,7 +880,7 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
         }
         if (tid == 0) {
             const uint32_t m = task_mask<MASKS>(t, s_mask);
-            if (nxt < 0) {
+            if (nxt < 0 && !has_d) {
                 const unsigned long long fv = want | ((unsigned long long)claims << 16) | m;
                 __hip_atomic_store(a.ready + t.f0, fv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 if (t.f1 >= 0)
@@ -722,12 +899,24 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
                 write_masks(pd, a, mp);
                 if (a.trace) {
                     long long* tr = a.trace + (size_t)(q == 0 ? t.pan_l : t.pan_u) * 4;
-                    gst(&tr[0], t_taken);
+                    gst(&tr[0], t_done);
                     gst(&tr[1], t_ready);
                     gst(&tr[2], (long long)wall_clock64());
                     gst(&tr[3], t_wait | (3ll << 60));
                 }
                 n_ran++;
+            }
+            if (has_d) {  // a diagonal chain's step, published in it
+                if (a.trace) {
+                    for (int32_t q : {dr.pan_l, dr.pan_u, dr.dia}) {
+                        long long* tr = a.trace + (size_t)q * 4;
+                        gst(&tr[0], t_done);
+                        gst(&tr[1], t_ready);
+                        gst(&tr[2], (long long)wall_clock64());
+                        gst(&tr[3], t_wait | (3ll << 60));
+                    }
+                }
+                n_ran += 3;
             }
             // consumers in this run read the masks from the flags; the mask array serves
             // the solve and the other executors, after the kernel
@@ -751,9 +940,13 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
             if (nxt >= 0) {
                 s_next_ti = nxt;
                 s_next_mode = 1;
+            } else if (has_d) {
+                s_next_ti = dr.next;
+                s_next_mode = 1;
             } else if (pl >= 0 || pu >= 0) {
                 s_next_ti = pl >= 0 ? pl : pu;
                 s_pend = pl >= 0 ? pu : -1;
+                s_pend_d = t.dia;
                 s_next_mode = 3;
             } else if (t.after >= 0) {
                 s_next_ti = t.after;
@@ -761,6 +954,10 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
             } else if (s_pend >= 0) {
                 s_next_ti = s_pend;
                 s_pend = -1;
+                s_next_mode = 3;
+            } else if (s_pend_d >= 0) {
+                s_next_ti = s_pend_d;
+                s_pend_d = -1;
                 s_next_mode = 3;
             } else if (s_ring_n > 0) {
                 const int h = s_ring_head;
@@ -950,7 +1147,7 @@ void build_chains(Factor* f, HostGraph& hg) {
     // after-links keep their chains in their heads' workgroups: neither end is claimed
     std::vector<char> linked(T, 0);
     for (size_t t = 0; t < T; t++)
-        for (int32_t u : {f->tasks[t].after, f->tasks[t].pan_l, f->tasks[t].pan_u})
+        for (int32_t u : {f->tasks[t].after, f->tasks[t].pan_l, f->tasks[t].pan_u, f->tasks[t].dia})
             if (u >= 0) linked[(size_t)u] = linked[t] = 1;
     for (size_t u = 0; u < T; u++) {
         const DevTask& k = f->tasks[u];
@@ -1139,6 +1336,84 @@ void build_after_links(Factor* f, const HostGraph& hg, std::vector<char>& linked
         f->n_after++;
     }
     f->chain_head = head;
+}
+
+// Diagonal chains (LU factors in FP32 and FP64).  Where the lu of block column k makes, through
+// its two panels next to the diagonal, the last update of the next diagonal tile
+// (S_{k+1,k+1} = P - L_{k+1,k} U_{k,k+1}, tile_order.h), its workgroup runs all three and the
+// next lu after them: the diagonal of a banded factor is one workgroup's work (diag_step).
+// Deadlock freedom: every wait in such a chain, and every other wait, is for a task of lower
+// index than the waiting one's (checked here for the panels, which run with the lu, by the
+// dependency levels else), and the queue hands tasks out by index.  Of the unfinished tasks
+// the lowest, m, waits for nothing.  Every queue entry before it is finished, so the
+// workgroups not on m are on chains whose heads come before it; with fewer such chains
+// than workgroups (launch_factor checks it) one is free to take m.  So there are at most
+// DIAG_CHAINS of them; a factor with more (many disconnected pieces) gets absorbed panels as
+// above.  Factor alone, absorbed panels -> chains: C5 FP32 281 -> 228 ms, C2 FP32 34.9 -> 28.8;
+// FP64, which had no absorbed panels: C2 51.3 -> 50.4, 2D 64^2 1.69 -> 1.62.
+constexpr int DIAG_CHAINS = 16;
+
+bool build_diag_chains(Factor* f, const HostGraph& hg, std::vector<char>& linked) {
+    const size_t T = f->tasks.size();
+    std::vector<int32_t> slot_task((size_t)f->n_slots, -1);
+    for (size_t t = 0; t < T; t++)
+        for (int32_t o : {f->tasks[t].out0, f->tasks[t].out1, f->tasks[t].out2, f->tasks[t].out3})
+            if (o >= 0) slot_task[(size_t)o] = (int32_t)t;
+    auto maker = [&](int32_t s) { return s >= 0 ? slot_task[(size_t)s] : -1; };
+    auto panel = [&](int32_t p, int32_t& lu, int which) {  // is p a panel (0: A U^-1, 1: L^-1 A) of some lu?
+        if (p < 0) return false;
+        const DevTask& k = f->tasks[(size_t)p];
+        if (k.kind != TK_GEMM || k.b != 1 || k.add >= 0 || k.next >= 0 || linked[(size_t)p]) return false;
+        const Pair& pr = hg.pairs[(size_t)k.a];
+        if (pr.a < 0) return false;
+        lu = maker(which == 0 ? pair_b(pr) : pair_a(pr));
+        if (lu < 0 || f->tasks[(size_t)lu].kind != TK_LU) return false;
+        const DevTask& kl = f->tasks[(size_t)lu];
+        if ((which == 0 ? pair_b(pr) != kl.out3 : pair_a(pr) != kl.out2)) return false;
+        return maker(which == 0 ? pair_a(pr) : pair_b(pr)) < lu;
+    };
+    struct Link {
+        int32_t lu, pl, pu, d;
+    };
+    std::vector<Link> links;
+    std::vector<char> used(T, 0);
+    for (size_t t = 0; t < T; t++) {
+        const DevTask& k = f->tasks[t];
+        if (k.kind != TK_GEMM || k.b != 1 || k.add < 0 || k.next < 0 || linked[t]) continue;
+        const Pair& pr = hg.pairs[(size_t)k.a];
+        if (pr.a < 0) continue;
+        const int32_t pl = maker(pair_a(pr)), pu = maker(pair_b(pr));
+        int32_t l0 = -1, l1 = -1;
+        if (pl == pu || !panel(pl, l0, 0) || !panel(pu, l1, 1) || l0 != l1 || used[(size_t)l0]) continue;
+        used[(size_t)l0] = 1;
+        links.push_back({l0, pl, pu, (int32_t)t});
+    }
+    if (links.empty()) return false;
+    std::vector<int32_t> pred(T, -1), head(T, -1);
+    for (size_t t = 0; t < T; t++)
+        if (f->tasks[t].next >= 0) pred[(size_t)f->tasks[t].next] = (int32_t)t;
+    for (const Link& l : links) pred[(size_t)l.pl] = pred[(size_t)l.pu] = pred[(size_t)l.d] = l.lu;
+    std::vector<char> chain(T, 0);
+    for (size_t t = 0; t < T; t++) {
+        if (pred[t] >= (int32_t)t) return false;
+        head[t] = pred[t] < 0 ? (int32_t)t : head[(size_t)pred[t]];
+    }
+    int32_t n = 0;
+    for (const Link& l : links)
+        if (!chain[(size_t)head[(size_t)l.lu]]) chain[(size_t)head[(size_t)l.lu]] = 1, n++;
+    if (n > DIAG_CHAINS) return false;
+    for (const Link& l : links) {
+        DevTask& k = f->tasks[(size_t)l.lu];
+        k.pan_l = l.pl;
+        k.pan_u = l.pu;
+        k.dia = l.d;
+        linked[(size_t)l.pl] = linked[(size_t)l.pu] = linked[(size_t)l.d] = 1;
+    }
+    f->n_absorbed = 2 * (int64_t)links.size();
+    f->n_after = 0;
+    f->n_diag_chains = n;
+    f->chain_head = head;
+    return true;
 }
 
 // The task graph of a factor description, on the host only (no device calls).
@@ -1621,7 +1896,7 @@ int build_host_graph(Context* c, const sogl_factor_desc* d, Factor* f, HostGraph
             chained[u] = 1;
             f->n_chained++;
         }
-        for (DevTask& k : f->tasks) k.after = k.pan_l = k.pan_u = -1;
+        for (DevTask& k : f->tasks) k.after = k.pan_l = k.pan_u = k.dia = k.rec = -1;
         // queue order: the task order (by dependency level).  Handing the GEMMs whose lu
         // follows them out last in their level lets more panels pass the head order
         // below (C5: 23k instead of 8k) but delays the diagonal chain (C5 FP32 factor
@@ -1630,7 +1905,9 @@ int build_host_graph(Context* c, const sogl_factor_desc* d, Factor* f, HostGraph
         std::vector<int64_t> rank(f->tasks.size());
         for (size_t u = 0; u < f->tasks.size(); u++) rank[u] = (int64_t)u;
         const bool absorb = f->absorb_panels && f->precision == SOGL_FP32 && !llt;
-        if (f->after_links || absorb) build_after_links(f, hg, chained, f->after_links, absorb, rank);
+        f->n_diag_chains = 0;
+        if (f->absorb_panels && !f->after_links && f->precision != SOGL_BF16 && !llt && build_diag_chains(f, hg, chained)) {
+        } else if (f->after_links || absorb) build_after_links(f, hg, chained, f->after_links, absorb, rank);
         else f->chain_head.clear();
         f->queue.clear();
         for (size_t u = 0; u < f->tasks.size(); u++)
@@ -1800,7 +2077,7 @@ int validate_graph(Context* c, const sogl_factor_desc* d, const Factor* f, const
             for (int which = 0; which < 2; which++) {  // an lu running one-pair panel GEMMs on its inverses
                 const int32_t p = which == 0 ? k.pan_l : k.pan_u;
                 if (p < 0) continue;
-                if (k.kind != TK_LU || f->precision != SOGL_FP32 || (size_t)p >= T || seen[(size_t)p])
+                if (k.kind != TK_LU || f->precision == SOGL_BF16 || (size_t)p >= T || seen[(size_t)p])
                     return bad("absorbed panel of task " + std::to_string(t));
                 const DevTask& u = f->tasks[(size_t)p];
                 if (u.kind != TK_GEMM || u.level <= k.level || u.b != 1 || u.add >= 0 || u.next >= 0 || u.after >= 0 ||
@@ -1813,6 +2090,21 @@ int validate_graph(Context* c, const sogl_factor_desc* d, const Factor* f, const
                 pred[(size_t)p] = (int32_t)t;
             }
         }
+        int32_t chains = 0;  // diagonal chains: the lu's panels, then their product and its lu
+        for (size_t t = 0; t < T; t++) {
+            const DevTask& k = f->tasks[t];
+            if (k.dia < 0) continue;
+            if (k.pan_l < 0 || k.pan_u < 0 || (size_t)k.dia >= T || seen[(size_t)k.dia])
+                return bad("diagonal chain of task " + std::to_string(t));
+            const DevTask& u = f->tasks[(size_t)k.dia];
+            if (u.kind != TK_GEMM || u.level <= k.level || u.b != 1 || u.add < 0 || u.next < 0 || u.after >= 0)
+                return bad("diagonal chain of task " + std::to_string(t));
+            const Pair& pr = hg.pairs[(size_t)u.a];
+            if (pr.a < 0 || pair_a(pr) != f->tasks[(size_t)k.pan_l].out0 || pair_b(pr) != f->tasks[(size_t)k.pan_u].out0)
+                return bad("diagonal chain of task " + std::to_string(t));
+            seen[(size_t)k.dia] = 1;
+            pred[(size_t)k.dia] = (int32_t)t;
+        }
         for (size_t t = 0; t < T; t++)
             if (!seen[t]) return bad("task " + std::to_string(t) + " is neither queued nor chained");
         // heads: links go to later levels, so a task's predecessor has a lower index
@@ -1820,6 +2112,7 @@ int validate_graph(Context* c, const sogl_factor_desc* d, const Factor* f, const
             if (pred[t] >= 0 && (size_t)pred[t] >= t) return bad("link order at task " + std::to_string(t));
             head[t] = pred[t] < 0 ? (int32_t)t : head[(size_t)pred[t]];
         }
+        std::set<int32_t> in_chain;
         std::vector<int32_t> producer((size_t)n, -1);
         for (size_t t = 0; t < T; t++)
             for (int32_t o : {f->tasks[t].out0, f->tasks[t].out1, f->tasks[t].out2, f->tasks[t].out3})
@@ -1827,6 +2120,17 @@ int validate_graph(Context* c, const sogl_factor_desc* d, const Factor* f, const
         for (size_t t = 0; t < T; t++) {
             const DevTask& k = f->tasks[t];
             if (pred[t] < 0 || k.kind != TK_GEMM || f->tasks[(size_t)pred[t]].next == (int32_t)t) continue;
+            if (f->tasks[(size_t)pred[t]].dia >= 0) {  // a diagonal chain's waits are for lower indices
+                const size_t at = f->tasks[(size_t)pred[t]].dia == (int32_t)t ? t : (size_t)pred[t];
+                for (int32_t q = k.dep_begin; q < k.dep_begin + k.dep_count; q++) {
+                    const int32_t p = producer[(size_t)hg.deps[(size_t)q]];
+                    if (p >= 0 && p != pred[t] && (size_t)p >= at)
+                        return bad("task " + std::to_string(t) + " of a diagonal chain waits for a later task");
+                }
+                if (in_chain.insert(head[t]).second && ++chains > DIAG_CHAINS) return bad("too many diagonal chains");
+                continue;
+            }
+            if (f->n_diag_chains) return bad("task " + std::to_string(t) + " is linked beside diagonal chains");
             for (int32_t q = k.dep_begin; q < k.dep_begin + k.dep_count; q++) {
                 const int32_t p = producer[(size_t)hg.deps[(size_t)q]];
                 if (p < 0) continue;
@@ -2260,6 +2564,21 @@ PairSteps pair_steps(const std::vector<int32_t>& rp, const std::vector<int32_t>&
     return s;
 }
 
+// The records of the diagonal chains' steps, in the order of their lus, after the slots are
+// assigned.
+void make_diag_records(Factor* f, const HostGraph& hg) {
+    f->diag.clear();
+    for (DevTask& k : f->tasks) {
+        if (k.dia < 0) continue;
+        const DevTask &l = f->tasks[(size_t)k.pan_l], &u = f->tasks[(size_t)k.pan_u], &d = f->tasks[(size_t)k.dia];
+        const Pair &pl = hg.pairs[(size_t)l.a], &pu = hg.pairs[(size_t)u.a], &pd = hg.pairs[(size_t)d.a];
+        k.rec = (int32_t)f->diag.size();
+        f->diag.push_back(DiagRec{pair_a(pl), pl.fa, pair_b(pu), pu.fb, d.add, d.fadd, l.out0, l.f0, u.out0, u.f0, d.out0,
+                                  d.next, (pl.b < 0) | (pu.b < 0) << 1 | (pd.b < 0) << 2 | (d.add_neg ? 8 : 0), k.pan_l,
+                                  k.pan_u, k.dia});
+    }
+}
+
 // Device arrays of a checked graph: pool, tasks, pairs, dependencies, flags, solve
 // structure, and the input tiles copied in.
 int upload_graph(Context* c, const sogl_factor_desc* d, const InputCells* cells, Factor* f,
@@ -2285,6 +2604,11 @@ int upload_graph(Context* c, const sogl_factor_desc* d, const InputCells* cells,
     if ((rc = dev_alloc(c, f->war_d, std::max<size_t>(f->war.size(), 1) * 4, "write-after-read flags")) != SOGL_OK)
         return rc;
     if (!f->war.empty()) HIP_TRY(c, hipMemcpy(f->war_d.p, f->war.data(), f->war.size() * 4, hipMemcpyHostToDevice));
+    // (one record more: a kernel reads record 0 where a task has none, and one ahead)
+    if ((rc = dev_alloc(c, f->diag_d, (f->diag.size() + 1) * sizeof(DiagRec), "diagonal chains")) != SOGL_OK)
+        return rc;
+    if (!f->diag.empty())
+        HIP_TRY(c, hipMemcpy(f->diag_d.p, f->diag.data(), f->diag.size() * sizeof(DiagRec), hipMemcpyHostToDevice));
     auto up_i32 = [&](DevBuf& b, const std::vector<int32_t>& v, const char* what) -> int {
         int r2 = dev_alloc(c, b, std::max<size_t>(v.size(), 1) * 4, what);
         if (r2 != SOGL_OK) return r2;
@@ -2428,6 +2752,7 @@ int build_graph(Context* c, const sogl_factor_desc* d, const InputCells* cells, 
                            (c->pool_reuse == SOGL_REUSE_AUTO && value_bytes > 0.25 * (double)c->total_mem);
         assign_slots(f, hg, reuse, cells != nullptr);
         rc = validate_slots(c, f, hg);
+        make_diag_records(f, hg);
     }
     if (rc == SOGL_OK) rc = upload_graph(c, d, cells, f, hg);
     return rc;
@@ -2436,7 +2761,7 @@ int build_graph(Context* c, const sogl_factor_desc* d, const InputCells* cells, 
 void free_factor(Factor* f) {
     if (f->graph_exec) (void)hipGraphExecDestroy(f->graph_exec);
     if (f->graph) (void)hipGraphDestroy(f->graph);
-    for (DevBuf* b : {&f->pool, &f->mask_d, &f->queue_d, &f->war_d, &f->uinv_chk_d, &f->pairx_d, &f->pairy_d, &f->cell_begin, &f->cell_pos, &f->cell_val, &f->chk_d, &f->tasks_d, &f->pairs_d, &f->deps_d, &f->ready_d, &f->ctrl_d,
+    for (DevBuf* b : {&f->pool, &f->mask_d, &f->queue_d, &f->diag_d, &f->war_d, &f->uinv_chk_d, &f->pairx_d, &f->pairy_d, &f->cell_begin, &f->cell_pos, &f->cell_val, &f->chk_d, &f->tasks_d, &f->pairs_d, &f->deps_d, &f->ready_d, &f->ctrl_d,
                       &f->op_tasks_d, &f->op_pairs_d, &f->inputs_d, &f->l_rowptr, &f->l_col,
                       &f->l_slot, &f->u_rowptr, &f->u_col, &f->u_slot, &f->l_diag_d, &f->u_diag_d,
                       &f->linv_d, &f->uinv_d, &f->lstep_ptr, &f->lstep_col, &f->lstep_slot, &f->ustep_ptr, &f->ustep_col,
@@ -2461,6 +2786,7 @@ int launch_factor(Context* c, Factor* f, int mode, int chunk, int wg_per_cu) {
     a.trace = (mode == SOGL_EXEC_PERSISTENT && f->trace_on) ? (long long*)f->trace_d.p : nullptr;
     a.chk = (const ChainChk*)f->chk_d.p;
     a.war = (const int32_t*)f->war_d.p;
+    a.diag = (const DiagRec*)f->diag_d.p;
     a.chain = (mode == SOGL_EXEC_PERSISTENT && !f->chk.empty()) ? f->chain_claims : 0;
     auto launch_levels = [&]() {
         a.tasks = (const DevTask*)f->tasks_d.p;
@@ -2524,6 +2850,11 @@ int launch_factor(Context* c, Factor* f, int mode, int chunk, int wg_per_cu) {
         if (per_cu < 1) per_cu = 1;
         if (wg_per_cu > 0) per_cu = std::min(per_cu, wg_per_cu);  // never more than fit: all must be resident
         int grid = std::max(1, std::min<int>(a.nqueue, c->num_cu * per_cu));
+        if (f->n_diag_chains) {  // see build_diag_chains; a chunk's entry behind a chain would wait for it
+            a.chunk = 1;
+            if (grid < a.nqueue && grid <= f->n_diag_chains)
+                return set_error(c, SOGL_ERR_UNSUPPORTED, "factor: fewer workgroups than diagonal chains");
+        }
         if (a.nqueue > 0) hipLaunchKernelGGL(kern, dim3(grid), dim3(NT), 0, st, a);
     } else if (mode == SOGL_EXEC_LEVELS) {
         launch_levels();
@@ -2705,6 +3036,20 @@ int graph_check(const sogl_factor_desc* d, bool cells, int64_t* info) {
         info[9] = f.n_pair_tasks;
         info[10] = f.n_after;
         info[11] = f.n_absorbed;
+    }
+    if (rc != SOGL_OK) return rc;
+    // and as factors are loaded, with diagonal chains where they apply
+    Factor g;
+    g.precision = f.precision;
+    g.elem = f.elem;
+    g.n_inputs = f.n_inputs;
+    g.absorb_panels = true;
+    HostGraph hd;
+    rc = build_host_graph(nullptr, d, &g, hd);
+    if (rc == SOGL_OK) rc = validate_graph(nullptr, d, &g, hd);
+    if (rc == SOGL_OK) {
+        assign_slots(&g, hd, true, cells);
+        rc = validate_slots(nullptr, &g, hd);
     }
     return rc;
 }

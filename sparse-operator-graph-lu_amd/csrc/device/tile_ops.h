@@ -1624,9 +1624,9 @@ __device__ inline void lu_inv_fp64_lds(T* __restrict__ pool, int src, int outl, 
 template <typename T>
 __device__ __attribute__((always_inline)) double lu_task(T* __restrict__ pool, int src, int outl, int outu, int outli, int outui,
                           char* lds_raw, double growth_limit, int* n_fp64, bool coh = false,
-                          float* xcopy = nullptr, float* zcopy = nullptr, bool in_lds = false) {
+                          T* xcopy = nullptr, T* zcopy = nullptr, bool in_lds = false) {
     if constexpr (sizeof(T) == 8) {
-        lu_inv_blocked<T>(pool, src, outl, outu, outli, outui, lds_raw, nullptr, nullptr, coh, nullptr, nullptr, in_lds);
+        lu_inv_blocked<T>(pool, src, outl, outu, outli, outui, lds_raw, nullptr, nullptr, coh, xcopy, zcopy, in_lds);
         return 1.0;
     } else {
         float amax = 0, umax = 0;

@@ -128,7 +128,9 @@ inline bool tile_order_ops(const sogl_factor_desc* d, const int32_t* in_bi, cons
             else if (lr[p].first > uc[q].first) q++;
             else {
                 const int32_t j = lr[p].first;
-                if (acc && (i + k + j) % SUM_PAIRS == 0) close();
+                // an LU's diagonal's last update, by the block column before it, is a part of
+                // its own: the lu of that column runs it (diagonal chains in factor.hip)
+                if (acc && ((i + k + j) % SUM_PAIRS == 0 || (!llt && i == k && j == k - 1))) close();
                 if (!acc) acc = next++;
                 emit(llt ? SOGL_OP_MULT : SOGL_OP_MUL, lr[p].second, uc[q].second, acc, 0, st);
                 found++;
@@ -143,8 +145,8 @@ inline bool tile_order_ops(const sogl_factor_desc* d, const int32_t* in_bi, cons
         const auto& lc = lcol[(size_t)k];
         const auto& ur = urow[(size_t)k];
         std::vector<int32_t> s_l(lc.size(), -1), s_u(ur.size(), -1);
-        // at most size / SUM_PAIRS + 2 parts in any sum of this step
-        const int32_t done = stage + (int32_t)(std::max(lrow[(size_t)k].size(), ucol[(size_t)k].size()) / SUM_PAIRS) + 3;
+        // at most size / SUM_PAIRS + 3 parts in any sum of this step
+        const int32_t done = stage + (int32_t)(std::max(lrow[(size_t)k].size(), ucol[(size_t)k].size()) / SUM_PAIRS) + 4;
         const int32_t x = next++, z = llt ? 0 : next++;
         bool ok = true;
         auto panel_l = [&](size_t q) {
