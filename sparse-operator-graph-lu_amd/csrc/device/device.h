@@ -78,8 +78,8 @@ struct DevTask {
     // itself, before publishing, from the inverses it keeps in LDS: pan_l = A U^-1 (its
     // U^-1 the second operand), pan_u = L^-1 A (its L^-1 the first); -1: none
     int32_t pan_l = -1, pan_u = -1;
-    // lu (persistent executor, with both panels): the GEMM of the next diagonal tile's last
-    // update, pan_l's tile times pan_u's, whose lu (its `next`) the same workgroup goes on
+    // lu (persistent executor, with both panels; an llt with its one, pan_l): the GEMM of the next diagonal tile's last
+    // update, pan_l's tile times pan_u's (an llt's: its own transpose), whose lu (its `next`) the same workgroup goes on
     // with (diagonal chains); -1: none
     int32_t dia = -1;
     int32_t rec = -1;  // and its DiagRec; -1: none
@@ -88,7 +88,7 @@ struct DevTask {
 
 // All that a diagonal chain's step needs beyond its lu's task, in one line (slots, and the
 // value ids that index the flags): the tiles its two panels and the update read (S_l, S_u,
-// P), those they make, the lu that follows, and the tasks' indices.
+// P), those they make, the lu that follows, and the tasks' indices (an llt has no panel u).
 struct DiagRec {
     int32_t s_l, f_sl, s_u, f_su, p, f_p;
     int32_t o_l, f_ol, o_u, f_ou, o_d, next;

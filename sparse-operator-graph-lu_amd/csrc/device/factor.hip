@@ -686,6 +686,130 @@ __device__ __attribute__((always_inline)) void diag_step(const Args& a, const De
             acc_store_global(acc[m][n], pool + (size_t)d.o_d * TE, wr + m * 16, wc + n * 16, li, lk);
 }
 
+// The same for an L L^T factor: L_{k+1,k} = S_{k+1,k} L_kk^-T and S_{k+1,k+1} = P - L_{k+1,k}
+// L_{k+1,k}^T.  The inverse is read back from the llt's stores, which have to be complete to
+// publish it.
+template <typename T, bool MASKS, bool COH>
+__device__ __attribute__((always_inline)) void diag_step_llt(const Args& a, const DevTask& lu, const DiagRec& d, char* lds,
+                                                             T* xcopy, uint32_t (*s_pmask)[NT / 64], uint32_t* s_words,
+                                                             unsigned long long want, long long* t_wait) {
+    typedef typename MfmaOp<T>::acc_t acc_t;
+    T* pool = reinterpret_cast<T*>(a.pool);
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wr = (w >> 1) * 32, wc = (w & 1) * 32, li = lane & 15, lk = lane >> 4;
+    constexpr int LDA = lda<T>();
+    T* la = reinterpret_cast<T*>(lds);
+    if (tid < 2) s_words[tid] = (uint32_t)spin_ready(a, tid == 0 ? d.f_sl : d.f_p) & MASK_ALL;
+    wave_stores_done();  // the llt's
+    __syncthreads();
+    if (tid == 0) {
+        if (a.trace) *t_wait = wall_clock64();
+        const unsigned long long fv = want | MASK_ALL;
+        for (int32_t fl : {lu.f0, lu.f1, lu.f2, lu.f3})
+            if (fl >= 0) __hip_atomic_store(a.ready + fl, fv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    const uint32_t ml = __builtin_amdgcn_readfirstlane(s_words[0]);
+    {
+        Seg<T> gs, gx;
+        seg_load<true>(pool + (size_t)lu.out2 * TE, gx, tid, true);
+        seg_load<COH>(pool + (size_t)d.s_l * TE, gs, tid, !MASKS || seg_on<T>(ml, tid));
+        seg_store(gx, xcopy, LDA, tid, true, false);
+        seg_store(gs, la, LDA, tid, !MASKS || seg_on<T>(ml, tid), d.neg & 1);
+    }
+    acc_t acc[2][2], xr[2][2];
+    auto zero = [&]() {
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int n = 0; n < 2; n++) acc[m][n] = acc_t{0, 0, 0, 0};
+    };
+#pragma unroll
+    for (int m = 0; m < 2; m++)
+#pragma unroll
+        for (int n = 0; n < 2; n++) xr[m][n] = acc_load_global<COH>(pool + (size_t)d.p * TE, wr + m * 16, wc + n * 16, li, lk);
+    int warm = 0;  // as in diag_step
+    if (w == 3 && lane < 3)
+        warm = lane < 2 ? reinterpret_cast<const int32_t*>(a.tasks + d.next)[lane * (sizeof(DevTask) / 4 - 1)]
+                        : a.diag[lu.rec + 1].s_l;
+    __syncthreads();
+    // the panel, as diag_step's A U^-1 (L^-T is upper triangular)
+    uint32_t bits = 0;
+    {
+        const int J[2] = {w & 1, 3 - (w & 1)}, I0 = 2 * (w >> 1);
+        zero();
+        uint32_t use = 0xFu;
+        if constexpr (MASKS) use = mask_row(ml, I0) | mask_row(ml, I0 + 1);
+#pragma unroll
+        for (int K = 0; K < 4; K++) {
+            if (K > J[1] || !((use >> K) & 1u)) continue;  // wave-uniform
+            const int k0 = 16 * K + 4 * lk;
+            T av[2][4], bv[2][4];
+#pragma unroll
+            for (int m = 0; m < 2; m++) read4(la + (16 * (I0 + m) + li) * LDA + k0, av[m]);
+#pragma unroll
+            for (int n = 0; n < 2; n++) read4(xcopy + (16 * J[n] + li) * LDA + k0, bv[n]);
+            const bool both = K <= J[0];  // wave-uniform
+#pragma unroll
+            for (int k4 = 0; k4 < 4; k4++)
+#pragma unroll
+                for (int m = 0; m < 2; m++)
+#pragma unroll
+                    for (int n = 0; n < 2; n++)
+                        if (both || n == 1) acc[m][n] = MfmaOp<T>::mma(av[m][k4], bv[n][k4], acc[m][n]);
+        }
+        T* C = pool + (size_t)d.o_l * TE;
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int n = 0; n < 2; n++) {
+                acc_store_global(acc[m][n], C, 16 * (I0 + m), 16 * J[n], li, lk);
+                if constexpr (MASKS)
+                    if (__ballot(acc_nonzero(acc[m][n], MASK_TINY)) != 0) bits |= 1u << (4 * (I0 + m) + J[n]);
+            }
+        if constexpr (MASKS)
+            if (lane == 0) s_pmask[0][w] = bits;
+        __syncthreads();  // every wave is done reading S
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int n = 0; n < 2; n++) {
+                if (MASKS && !((bits >> (4 * (I0 + m) + J[n])) & 1u)) acc[m][n] = acc_t{0, 0, 0, 0};
+                acc_store<T>(acc[m][n], la + 16 * (I0 + m) * LDA + 16 * J[n], LDA, li, lk);
+            }
+    }
+    __syncthreads();
+    uint32_t ma = MASK_ALL;
+    if constexpr (MASKS) ma = __builtin_amdgcn_readfirstlane(s_pmask[0][0] | s_pmask[0][1] | s_pmask[0][2] | s_pmask[0][3]);
+    zero();
+    if (!MASKS || ma != 0) {
+        uint32_t kuse = 0xFu;
+        if constexpr (MASKS) kuse = k_blocks_used(ma, mask_transpose(ma), wr >> 4, wc >> 4);
+        gemm_lds<T, true, true>(acc, la, la, wr, wc, li, lk, kuse);
+    }
+#pragma unroll
+    for (int m = 0; m < 2; m++)
+#pragma unroll
+        for (int n = 0; n < 2; n++) {
+            if ((d.neg >> 2) & 1) acc[m][n] = acc_t{0, 0, 0, 0} - acc[m][n];
+            acc[m][n] += (d.neg >> 3) & 1 ? -xr[m][n] : xr[m][n];
+        }
+    asm volatile("" ::"v"(warm));
+    wave_stores_done();  // the panel's
+    __syncthreads();     // and every wave is done reading la
+    if (tid == 0) {
+        __hip_atomic_store(a.ready + d.f_ol, want | ma, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        gst(&a.mask[d.o_l], ma);
+        gst(&a.mask[d.o_d], MASK_ALL);
+    }
+#pragma unroll
+    for (int m = 0; m < 2; m++)
+#pragma unroll
+        for (int n = 0; n < 2; n++) {
+            acc_store<T>(acc[m][n], la + (wr + m * 16) * LDA + wc + n * 16, LDA, li, lk);
+            acc_store_global(acc[m][n], pool + (size_t)d.o_d * TE, wr + m * 16, wc + n * 16, li, lk);
+        }
+}
+
 // Block mask of a finished task's outputs (thread 0, after the task's last barrier):
 // GEMM, sub and transpose tasks leave their waves' bits in s_mask; the tiles of lu /
 // llt and the inverses, and everything when masks are off, count as full.
@@ -722,10 +846,11 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
     // beyond what any task kind uses.  The kernels built for two (no registers to spare)
     // run them as after-links instead: right after the lu, in the same workgroup.
     constexpr bool ABSORB = !BF16 && !LLT && ONE;
-    constexpr int XCOPY_BYTES = ABSORB ? TS * lda<T>() * (int)sizeof(T) : 0;
+    constexpr bool CHAINS = !BF16 && ONE;  // and lu / llt tasks run diagonal chains' steps
+    constexpr int XCOPY_BYTES = CHAINS ? TS * lda<T>() * (int)sizeof(T) : 0;
     constexpr int ZCOPY_BYTES = ABSORB ? TS * LDB * (int)sizeof(T) : 0;
     __shared__ __attribute__((aligned(16))) char lds[lds_bytes<T>() + XCOPY_BYTES + ZCOPY_BYTES];
-    T* const xcopy = ABSORB ? reinterpret_cast<T*>(lds + lds_bytes<T>()) : nullptr;
+    T* const xcopy = CHAINS ? reinterpret_cast<T*>(lds + lds_bytes<T>()) : nullptr;
     T* const zcopy = ABSORB ? reinterpret_cast<T*>(lds + lds_bytes<T>() + XCOPY_BYTES) : nullptr;
     __shared__ uint32_t s_pmask[2][NT / 64];
     __shared__ uint32_t s_word;
@@ -807,7 +932,7 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
         // an lu with absorbed panels (wave-uniform task fields): the panels' descriptors
         // (with dynamic chaining on, panels run as after-links, whose outputs' candidates
         // can be claimed)
-        const bool absorbs = ABSORB && !a.chain && t.kind == TK_LU && (t.pan_l >= 0 || t.pan_u >= 0);
+        const bool absorbs = CHAINS && !a.chain && t.kind == (LLT ? TK_LLT : TK_LU) && (t.pan_l >= 0 || t.pan_u >= 0);
         const bool has_d = absorbs && t.rec >= 0;
         const bool has_l = absorbs && !has_d && t.pan_l >= 0, has_u = absorbs && !has_d && t.pan_u >= 0;
         const DiagRec dr = const_load(a.diag + (has_d ? t.rec : 0));
@@ -829,6 +954,13 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
                      t.war_count},
             mode == 1, has_u || has_d ? xcopy : nullptr, has_l || has_d ? zcopy : nullptr, nxt >= 0);
         if (nxt >= 0) asm volatile("" ::"s"(pf0), "s"(pf1), "s"(pf2));
+        if constexpr (CHAINS && LLT) {
+            if (has_d) {
+                __syncthreads();
+                if (a.trace && tid == 0) t_done = wall_clock64();
+                diag_step_llt<T, MASKS, COH>(a, t, dr, lds, xcopy, s_pmask, s_words, want, &t_wait);
+            }
+        }
         if constexpr (ABSORB) {
             if (absorbs) {
                 __syncthreads();  // the lu's LDS (the inverses' copies included) is complete
@@ -909,6 +1041,7 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
             if (has_d) {  // a diagonal chain's step, published in it
                 if (a.trace) {
                     for (int32_t q : {dr.pan_l, dr.pan_u, dr.dia}) {
+                        if (q < 0) continue;
                         long long* tr = a.trace + (size_t)q * 4;
                         gst(&tr[0], t_done);
                         gst(&tr[1], t_ready);
@@ -916,7 +1049,7 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
                         gst(&tr[3], t_wait | (3ll << 60));
                     }
                 }
-                n_ran += 3;
+                n_ran += LLT ? 2 : 3;
             }
             // consumers in this run read the masks from the flags; the mask array serves
             // the solve and the other executors, after the kernel
@@ -935,8 +1068,8 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
             // barrier): the static chain's next task, else the after-link, else the
             // ring's head with its masks
             // (kernels without the inverses' copies run an lu's panels as after-links)
-            const int pl = !absorbs && t.kind == TK_LU ? t.pan_l : -1;
-            const int pu = !absorbs && t.kind == TK_LU ? t.pan_u : -1;
+            const int pl = !absorbs ? t.pan_l : -1;
+            const int pu = !absorbs ? t.pan_u : -1;
             if (nxt >= 0) {
                 s_next_ti = nxt;
                 s_next_mode = 1;
@@ -1338,7 +1471,7 @@ void build_after_links(Factor* f, const HostGraph& hg, std::vector<char>& linked
     f->chain_head = head;
 }
 
-// Diagonal chains (LU factors in FP32 and FP64).  Where the lu of block column k makes, through
+// Diagonal chains (FP32 and FP64 factors; L L^T ones with one panel, diag_step_llt).  Where the lu of block column k makes, through
 // its two panels next to the diagonal, the last update of the next diagonal tile
 // (S_{k+1,k+1} = P - L_{k+1,k} U_{k,k+1}, tile_order.h), its workgroup runs all three and the
 // next lu after them: the diagonal of a banded factor is one workgroup's work (diag_step).
@@ -1350,7 +1483,8 @@ void build_after_links(Factor* f, const HostGraph& hg, std::vector<char>& linked
 // than workgroups (launch_factor checks it) one is free to take m.  So there are at most
 // DIAG_CHAINS of them; a factor with more (many disconnected pieces) gets absorbed panels as
 // above.  Factor alone, absorbed panels -> chains: C5 FP32 281 -> 228 ms, C2 FP32 34.9 -> 28.8;
-// FP64, which had no absorbed panels: C2 51.3 -> 50.4, 2D 64^2 1.69 -> 1.62.
+// FP64, which had no absorbed panels: C2 51.3 -> 50.4, 2D 64^2 1.69 -> 1.62; symmetric 3D
+// 37^3 FP64 21.4 -> 18.5.
 constexpr int DIAG_CHAINS = 16;
 
 bool build_diag_chains(Factor* f, const HostGraph& hg, std::vector<char>& linked) {
@@ -1365,7 +1499,11 @@ bool build_diag_chains(Factor* f, const HostGraph& hg, std::vector<char>& linked
         const DevTask& k = f->tasks[(size_t)p];
         if (k.kind != TK_GEMM || k.b != 1 || k.add >= 0 || k.next >= 0 || linked[(size_t)p]) return false;
         const Pair& pr = hg.pairs[(size_t)k.a];
-        if (pr.a < 0) return false;
+        if (pr.a < 0) {  // A L^-T, the one panel of an llt
+            lu = maker(pair_b(pr));
+            return lu >= 0 && f->tasks[(size_t)lu].kind == TK_LLT && pair_b(pr) == f->tasks[(size_t)lu].out2 &&
+                   maker(pair_a(pr)) < lu;
+        }
         lu = maker(which == 0 ? pair_b(pr) : pair_a(pr));
         if (lu < 0 || f->tasks[(size_t)lu].kind != TK_LU) return false;
         const DevTask& kl = f->tasks[(size_t)lu];
@@ -1381,18 +1519,25 @@ bool build_diag_chains(Factor* f, const HostGraph& hg, std::vector<char>& linked
         const DevTask& k = f->tasks[t];
         if (k.kind != TK_GEMM || k.b != 1 || k.add < 0 || k.next < 0 || linked[t]) continue;
         const Pair& pr = hg.pairs[(size_t)k.a];
-        if (pr.a < 0) continue;
         const int32_t pl = maker(pair_a(pr)), pu = maker(pair_b(pr));
         int32_t l0 = -1, l1 = -1;
-        if (pl == pu || !panel(pl, l0, 0) || !panel(pu, l1, 1) || l0 != l1 || used[(size_t)l0]) continue;
+        if (!panel(pl, l0, 0) || !panel(pu, l1, 1) || l0 != l1 || used[(size_t)l0]) continue;
+        const bool llt = f->tasks[(size_t)l0].kind == TK_LLT;
+        if ((pr.a < 0) != llt || (pl == pu) != llt) continue;
         used[(size_t)l0] = 1;
+        if (llt) {
+            links.push_back({l0, pl, -1, (int32_t)t});
+            continue;
+        }
         links.push_back({l0, pl, pu, (int32_t)t});
     }
     if (links.empty()) return false;
     std::vector<int32_t> pred(T, -1), head(T, -1);
     for (size_t t = 0; t < T; t++)
         if (f->tasks[t].next >= 0) pred[(size_t)f->tasks[t].next] = (int32_t)t;
-    for (const Link& l : links) pred[(size_t)l.pl] = pred[(size_t)l.pu] = pred[(size_t)l.d] = l.lu;
+    for (const Link& l : links)
+        for (int32_t u : {l.pl, l.pu, l.d})
+            if (u >= 0) pred[(size_t)u] = l.lu;
     std::vector<char> chain(T, 0);
     for (size_t t = 0; t < T; t++) {
         if (pred[t] >= (int32_t)t) return false;
@@ -1402,14 +1547,16 @@ bool build_diag_chains(Factor* f, const HostGraph& hg, std::vector<char>& linked
     for (const Link& l : links)
         if (!chain[(size_t)head[(size_t)l.lu]]) chain[(size_t)head[(size_t)l.lu]] = 1, n++;
     if (n > DIAG_CHAINS) return false;
+    f->n_absorbed = 0;
     for (const Link& l : links) {
         DevTask& k = f->tasks[(size_t)l.lu];
         k.pan_l = l.pl;
         k.pan_u = l.pu;
         k.dia = l.d;
-        linked[(size_t)l.pl] = linked[(size_t)l.pu] = linked[(size_t)l.d] = 1;
+        f->n_absorbed += l.pu < 0 ? 1 : 2;
+        for (int32_t u : {l.pl, l.pu, l.d})
+            if (u >= 0) linked[(size_t)u] = 1;
     }
-    f->n_absorbed = 2 * (int64_t)links.size();
     f->n_after = 0;
     f->n_diag_chains = n;
     f->chain_head = head;
@@ -1906,7 +2053,7 @@ int build_host_graph(Context* c, const sogl_factor_desc* d, Factor* f, HostGraph
         for (size_t u = 0; u < f->tasks.size(); u++) rank[u] = (int64_t)u;
         const bool absorb = f->absorb_panels && f->precision == SOGL_FP32 && !llt;
         f->n_diag_chains = 0;
-        if (f->absorb_panels && !f->after_links && f->precision != SOGL_BF16 && !llt && build_diag_chains(f, hg, chained)) {
+        if (f->absorb_panels && !f->after_links && f->precision != SOGL_BF16 && build_diag_chains(f, hg, chained)) {
         } else if (f->after_links || absorb) build_after_links(f, hg, chained, f->after_links, absorb, rank);
         else f->chain_head.clear();
         f->queue.clear();
@@ -2077,14 +2224,16 @@ int validate_graph(Context* c, const sogl_factor_desc* d, const Factor* f, const
             for (int which = 0; which < 2; which++) {  // an lu running one-pair panel GEMMs on its inverses
                 const int32_t p = which == 0 ? k.pan_l : k.pan_u;
                 if (p < 0) continue;
-                if (k.kind != TK_LU || f->precision == SOGL_BF16 || (size_t)p >= T || seen[(size_t)p])
+                const bool chol = k.kind == TK_LLT && which == 0 && k.dia >= 0;
+                if ((k.kind != TK_LU && !chol) || f->precision == SOGL_BF16 || (size_t)p >= T || seen[(size_t)p])
                     return bad("absorbed panel of task " + std::to_string(t));
                 const DevTask& u = f->tasks[(size_t)p];
                 if (u.kind != TK_GEMM || u.level <= k.level || u.b != 1 || u.add >= 0 || u.next >= 0 || u.after >= 0 ||
                     u.pan_l >= 0 || u.pan_u >= 0 || u.a < 0 || (size_t)u.a >= hg.pairs.size())
                     return bad("absorbed panel of task " + std::to_string(t));
                 const Pair& pr = hg.pairs[(size_t)u.a];
-                if (pr.a < 0 || (which == 0 ? pair_b(pr) != k.out3 : pair_a(pr) != k.out2))
+                if (chol ? pr.a >= 0 || pair_b(pr) != k.out2
+                         : pr.a < 0 || (which == 0 ? pair_b(pr) != k.out3 : pair_a(pr) != k.out2))
                     return bad("absorbed panel of task " + std::to_string(t));
                 seen[(size_t)p] = 1;
                 pred[(size_t)p] = (int32_t)t;
@@ -2094,13 +2243,15 @@ int validate_graph(Context* c, const sogl_factor_desc* d, const Factor* f, const
         for (size_t t = 0; t < T; t++) {
             const DevTask& k = f->tasks[t];
             if (k.dia < 0) continue;
-            if (k.pan_l < 0 || k.pan_u < 0 || (size_t)k.dia >= T || seen[(size_t)k.dia])
+            const bool chol = k.kind == TK_LLT;
+            if (k.pan_l < 0 || (k.pan_u < 0) != chol || (size_t)k.dia >= T || seen[(size_t)k.dia])
                 return bad("diagonal chain of task " + std::to_string(t));
             const DevTask& u = f->tasks[(size_t)k.dia];
             if (u.kind != TK_GEMM || u.level <= k.level || u.b != 1 || u.add < 0 || u.next < 0 || u.after >= 0)
                 return bad("diagonal chain of task " + std::to_string(t));
             const Pair& pr = hg.pairs[(size_t)u.a];
-            if (pr.a < 0 || pair_a(pr) != f->tasks[(size_t)k.pan_l].out0 || pair_b(pr) != f->tasks[(size_t)k.pan_u].out0)
+            if ((pr.a < 0) != chol || pair_a(pr) != f->tasks[(size_t)k.pan_l].out0 ||
+                pair_b(pr) != f->tasks[(size_t)(chol ? k.pan_l : k.pan_u)].out0)
                 return bad("diagonal chain of task " + std::to_string(t));
             seen[(size_t)k.dia] = 1;
             pred[(size_t)k.dia] = (int32_t)t;
@@ -2570,7 +2721,15 @@ void make_diag_records(Factor* f, const HostGraph& hg) {
     f->diag.clear();
     for (DevTask& k : f->tasks) {
         if (k.dia < 0) continue;
-        const DevTask &l = f->tasks[(size_t)k.pan_l], &u = f->tasks[(size_t)k.pan_u], &d = f->tasks[(size_t)k.dia];
+        const DevTask &l = f->tasks[(size_t)k.pan_l], &d = f->tasks[(size_t)k.dia];
+        if (k.pan_u < 0) {
+            const Pair &pl = hg.pairs[(size_t)l.a], &pd = hg.pairs[(size_t)d.a];
+            k.rec = (int32_t)f->diag.size();
+            f->diag.push_back(DiagRec{pair_a(pl), pl.fa, -1, -1, d.add, d.fadd, l.out0, l.f0, -1, -1, d.out0, d.next,
+                                      (pl.b < 0) | (pd.b < 0) << 2 | (d.add_neg ? 8 : 0), k.pan_l, -1, k.dia});
+            continue;
+        }
+        const DevTask& u = f->tasks[(size_t)k.pan_u];
         const Pair &pl = hg.pairs[(size_t)l.a], &pu = hg.pairs[(size_t)u.a], &pd = hg.pairs[(size_t)d.a];
         k.rec = (int32_t)f->diag.size();
         f->diag.push_back(DiagRec{pair_a(pl), pl.fa, pair_b(pu), pu.fb, d.add, d.fadd, l.out0, l.f0, u.out0, u.f0, d.out0,

@@ -128,9 +128,9 @@ inline bool tile_order_ops(const sogl_factor_desc* d, const int32_t* in_bi, cons
             else if (lr[p].first > uc[q].first) q++;
             else {
                 const int32_t j = lr[p].first;
-                // an LU's diagonal's last update, by the block column before it, is a part of
-                // its own: the lu of that column runs it (diagonal chains in factor.hip)
-                if (acc && ((i + k + j) % SUM_PAIRS == 0 || (!llt && i == k && j == k - 1))) close();
+                // the diagonal's last update, by the block column before it, is a part of its
+                // own: the lu / llt of that column runs it (diagonal chains in factor.hip)
+                if (acc && ((i + k + j) % SUM_PAIRS == 0 || (i == k && j == k - 1))) close();
                 if (!acc) acc = next++;
                 emit(llt ? SOGL_OP_MULT : SOGL_OP_MUL, lr[p].second, uc[q].second, acc, 0, st);
                 found++;
