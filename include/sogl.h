@@ -204,9 +204,12 @@ int sogl_ctx_set_pool_reuse(sogl_ctx* ctx, int32_t mode);
 /* Task links of the persistent executor, for the factors loaded from now on (a mask of
  * SOGL_LINK_*; default SOGL_LINK_PANEL).  No reference counterpart (the reference runs
  * a stage's ops on a thread pool); results are the same bits with any mask.
- *   SOGL_LINK_PANEL: the lu task of an FP32 LU factor runs its most critical panel
- *     GEMM (A U^-1 or L^-1 A, one pair) itself, from the inverse it keeps in LDS, and
- *     publishes both tiles at once.
+ *   SOGL_LINK_PANEL: the lu / llt task of an FP32 or FP64 factor runs its panels next to
+ *     the diagonal and the next diagonal tile's last update itself, in LDS, and its
+ *     workgroup goes on with that tile's lu (diagonal chains); where there would be too
+ *     many such chains, or with SOGL_LINK_AFTER, the lu of an FP32 LU factor runs its
+ *     most critical panel GEMM (A U^-1 or L^-1 A, one pair), from the inverse it keeps in
+ *     LDS, and publishes both tiles at once.
  *   SOGL_LINK_AFTER: the workgroup that made a tile on the critical path goes on, right
  *     after publishing it, to a one-pair GEMM that reads it, instead of handing it to
  *     another workgroup (measured slower: off by default).
@@ -278,7 +281,7 @@ int sogl_factor_release(sogl_ctx* ctx, int32_t factor_id);
 /* No counterpart in the reference.  sogl_solve_device for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): the same kernels, but the solve's intermediates (the forward
- * result y, per-block-row flags and control words) live in a fixed per-GPU scratch
+ * result y and control words; the limit counts 4 bytes per block row besides) live in a fixed per-GPU scratch
  * array of SOGL_NOALLOC_SCRATCH_BYTES instead of buffers the factor allocates, and the
  * call allocates nothing.  It needs 256 + 4*block_rows (rounded up to a multiple of
  * 256) + 512*block_rows*nrhs bytes of the array; a larger solve returns SOGL_ERR_ARG.

@@ -138,7 +138,9 @@ struct Factor {
     int64_t n_folded = 0;       // copies, negations and subtractions folded into other tasks
     int64_t n_chained = 0;      // lu / llt tasks run by the workgroup that made their source
     int64_t n_pair_tasks = 0;   // GEMM tasks making the solve's two-row blocks X_p / Y_p
-    // device arrays
+    // device arrays (index_d: one allocation for the index arrays, whose DevBufs point into it
+    // and are not freed themselves: the solve's, inputs_d, war_d and diag_d)
+    DevBuf index_d;
     DevBuf pool, tasks_d, pairs_d, deps_d, ready_d, ctrl_d, op_tasks_d, op_pairs_d, inputs_d, queue_d, chk_d, diag_d;
     std::vector<ChainChk> chk;             // chain candidates' check entries (see DevTask)
     int64_t n_chain_cands = 0;             // tasks that are some task's chain candidate

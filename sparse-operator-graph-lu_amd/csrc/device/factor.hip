@@ -2760,20 +2760,6 @@ int upload_graph(Context* c, const sogl_factor_desc* d, const InputCells* cells,
     if ((rc = dev_alloc(c, f->queue_d, std::max<size_t>(f->queue.size(), 1) * 4, "task queue")) != SOGL_OK) return rc;
     if ((rc = dev_alloc(c, f->chk_d, std::max<size_t>(f->chk.size(), 1) * sizeof(ChainChk), "chain checks")) != SOGL_OK)
         return rc;
-    if ((rc = dev_alloc(c, f->war_d, std::max<size_t>(f->war.size(), 1) * 4, "write-after-read flags")) != SOGL_OK)
-        return rc;
-    if (!f->war.empty()) HIP_TRY(c, hipMemcpy(f->war_d.p, f->war.data(), f->war.size() * 4, hipMemcpyHostToDevice));
-    // (one record more: a kernel reads record 0 where a task has none, and one ahead)
-    if ((rc = dev_alloc(c, f->diag_d, (f->diag.size() + 1) * sizeof(DiagRec), "diagonal chains")) != SOGL_OK)
-        return rc;
-    if (!f->diag.empty())
-        HIP_TRY(c, hipMemcpy(f->diag_d.p, f->diag.data(), f->diag.size() * sizeof(DiagRec), hipMemcpyHostToDevice));
-    auto up_i32 = [&](DevBuf& b, const std::vector<int32_t>& v, const char* what) -> int {
-        int r2 = dev_alloc(c, b, std::max<size_t>(v.size(), 1) * 4, what);
-        if (r2 != SOGL_OK) return r2;
-        if (!v.empty()) HIP_TRY(c, hipMemcpy(b.p, v.data(), v.size() * 4, hipMemcpyHostToDevice));
-        return SOGL_OK;
-    };
     hipStream_t st = c->stream;
     if (T) HIP_TRY(c, hipMemcpy(f->tasks_d.p, f->tasks.data(), T * sizeof(DevTask), hipMemcpyHostToDevice));
     if (!pairs.empty()) HIP_TRY(c, hipMemcpy(f->pairs_d.p, pairs.data(), pairs.size() * sizeof(Pair), hipMemcpyHostToDevice));
@@ -2788,22 +2774,37 @@ int upload_graph(Context* c, const sogl_factor_desc* d, const InputCells* cells,
     if (!f->queue.empty()) HIP_TRY(c, hipMemcpy(f->queue_d.p, f->queue.data(), f->queue.size() * 4, hipMemcpyHostToDevice));
     if (!f->chk.empty())
         HIP_TRY(c, hipMemcpy(f->chk_d.p, f->chk.data(), f->chk.size() * sizeof(ChainChk), hipMemcpyHostToDevice));
-    if ((rc = up_i32(f->l_rowptr, hg.lp, "L rows")) || (rc = up_i32(f->l_col, hg.lc, "L cols")) ||
-        (rc = up_i32(f->l_slot, hg.ls, "L slots")) || (rc = up_i32(f->u_rowptr, hg.up, "U rows")) ||
-        (rc = up_i32(f->u_col, hg.uc, "U cols")) || (rc = up_i32(f->u_slot, hg.us, "U slots")) ||
-        (rc = up_i32(f->l_diag_d, f->l_diag, "L diag")) || (rc = up_i32(f->u_diag_d, f->u_diag, "U diag")) ||
-        (rc = up_i32(f->linv_d, f->linv_slot, "L inv")) || (rc = up_i32(f->uinv_d, f->uinv_slot, "U inv")) ||
-        (rc = up_i32(f->pairx_d, hg.pair_x, "row pair L blocks")) || (rc = up_i32(f->pairy_d, hg.pair_y, "row pair U blocks")) ||
-        (rc = up_i32(f->inputs_d, f->input_slots, "input slots")))
-        return rc;
+    // the index arrays: parts of one allocation, filled by one copy (an allocation and a copy
+    // each, they were a tenth of a small drop-in solve)
     f->solve_entries = (int64_t)hg.lc.size() + (int64_t)hg.uc.size();
-    for (int which = 0; which < 2; which++) {
-        const PairSteps s = which == 0 ? pair_steps(hg.lp, hg.lc, hg.ls) : pair_steps(hg.up, hg.uc, hg.us);
-        if ((rc = up_i32(which == 0 ? f->lstep_ptr : f->ustep_ptr, s.ptr, "solve steps")) ||
-            (rc = up_i32(which == 0 ? f->lstep_col : f->ustep_col, s.col, "solve step columns")) ||
-            (rc = up_i32(which == 0 ? f->lstep_slot : f->ustep_slot, s.slot, "solve step tiles")))
-            return rc;
+    const PairSteps ls = pair_steps(hg.lp, hg.lc, hg.ls), us = pair_steps(hg.up, hg.uc, hg.us);
+    struct Part {
+        DevBuf* b;
+        const void* p;
+        size_t bytes, room;
+    };
+    std::vector<Part> parts;
+    auto add = [&](DevBuf& b, const std::vector<int32_t>& v) { parts.push_back({&b, v.data(), v.size() * 4, v.size() * 4}); };
+    add(f->l_rowptr, hg.lp), add(f->l_col, hg.lc), add(f->l_slot, hg.ls);
+    add(f->u_rowptr, hg.up), add(f->u_col, hg.uc), add(f->u_slot, hg.us);
+    add(f->l_diag_d, f->l_diag), add(f->u_diag_d, f->u_diag), add(f->linv_d, f->linv_slot), add(f->uinv_d, f->uinv_slot);
+    add(f->pairx_d, hg.pair_x), add(f->pairy_d, hg.pair_y), add(f->inputs_d, f->input_slots), add(f->war_d, f->war);
+    add(f->lstep_ptr, ls.ptr), add(f->lstep_col, ls.col), add(f->lstep_slot, ls.slot);
+    add(f->ustep_ptr, us.ptr), add(f->ustep_col, us.col), add(f->ustep_slot, us.slot);
+    // (one record more: a kernel reads record 0 where a task has none, and one ahead)
+    parts.push_back({&f->diag_d, f->diag.data(), f->diag.size() * sizeof(DiagRec), (f->diag.size() + 1) * sizeof(DiagRec)});
+    size_t total = 0;
+    for (Part& q : parts) {
+        q.b->p = (void*)total;  // its offset, for now
+        total += (std::max<size_t>(q.room, 4) + 255) & ~(size_t)255;
     }
+    std::vector<char> host(total);
+    for (const Part& q : parts)
+        if (q.bytes) std::memcpy(host.data() + (size_t)q.b->p, q.p, q.bytes);
+    rc = dev_alloc(c, f->index_d, total, "index arrays");
+    for (Part& q : parts) q.b->p = rc ? nullptr : (char*)f->index_d.p + (size_t)q.b->p;
+    if (rc) return rc;
+    HIP_TRY(c, hipMemcpy(f->index_d.p, host.data(), total, hipMemcpyHostToDevice));
     hipLaunchKernelGGL(k_fill<unsigned long long>, dim3(256), dim3(256), 0, st, (unsigned long long*)f->ready_d.p,
                        (size_t)f->n_slots, 0ull);
     // input tiles (slots 0..n_inputs-1) and the zero tile never change: always ready
@@ -2920,11 +2921,8 @@ int build_graph(Context* c, const sogl_factor_desc* d, const InputCells* cells, 
 void free_factor(Factor* f) {
     if (f->graph_exec) (void)hipGraphExecDestroy(f->graph_exec);
     if (f->graph) (void)hipGraphDestroy(f->graph);
-    for (DevBuf* b : {&f->pool, &f->mask_d, &f->queue_d, &f->diag_d, &f->war_d, &f->uinv_chk_d, &f->pairx_d, &f->pairy_d, &f->cell_begin, &f->cell_pos, &f->cell_val, &f->chk_d, &f->tasks_d, &f->pairs_d, &f->deps_d, &f->ready_d, &f->ctrl_d,
-                      &f->op_tasks_d, &f->op_pairs_d, &f->inputs_d, &f->l_rowptr, &f->l_col,
-                      &f->l_slot, &f->u_rowptr, &f->u_col, &f->u_slot, &f->l_diag_d, &f->u_diag_d,
-                      &f->linv_d, &f->uinv_d, &f->lstep_ptr, &f->lstep_col, &f->lstep_slot, &f->ustep_ptr, &f->ustep_col,
-                      &f->ustep_slot, &f->solve_ctrl, &f->vec_b, &f->vec_x,
+    for (DevBuf* b : {&f->pool, &f->mask_d, &f->queue_d, &f->index_d, &f->uinv_chk_d, &f->cell_begin, &f->cell_pos, &f->cell_val, &f->chk_d, &f->tasks_d, &f->pairs_d, &f->deps_d, &f->ready_d, &f->ctrl_d,
+                      &f->op_tasks_d, &f->op_pairs_d, &f->solve_ctrl, &f->vec_b, &f->vec_x,
                       &f->vec_y, &f->csr_ptr, &f->csr_col, &f->csr_val, &f->vec_r, &f->vec_d, &f->red, &f->perm_d, &f->vec_io, &f->trace_d})
         dev_free(*b);
     delete f;
