@@ -273,7 +273,8 @@ int sogl_factor_set_masks(sogl_ctx* ctx, int32_t factor_id, int32_t mode);
  * solves L y = b, then L^T x = y (upperSolverT, BlockPlanner.cpp:769-797). */
 int sogl_solve(sogl_ctx* ctx, int32_t factor_id, const double* bp, double* xp, double* y,
                int32_t nrhs);
-/* Same, on device-resident arrays (hipMalloc'd by the caller) on the ctx stream. */
+/* Same, on device-resident arrays (hipMalloc'd by the caller) on the ctx stream.  d_xp may
+ * be d_bp (x takes the place of b). */
 int sogl_solve_device(sogl_ctx* ctx, int32_t factor_id, const double* d_bp, double* d_xp,
                       int32_t nrhs);
 int sogl_factor_release(sogl_ctx* ctx, int32_t factor_id);

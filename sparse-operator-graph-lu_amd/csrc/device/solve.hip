@@ -59,21 +59,27 @@ struct SolveArgs {
 // that each poll costs one round trip to the device coherence point.
 constexpr int SOLVE_SPIN_CHECK = 64;
 
-// Rows of the output that a pass has not stored yet hold this signalling NaN, written by
-// k_solve_begin before the pass.  FP arithmetic never produces a signalling NaN (a NaN
-// result is quiet), so a stored value is never mistaken for it.  A task polls the values it
-// reads themselves, with agent-scope atomic loads, until none is the marker, and stores its
-// rows with agent-scope atomic stores, which reach the coherence point without a release.
+// Rows of the output that a pass has not stored yet hold this signalling NaN, written before
+// the pass (k_solve_begin; k_fill_pending for an x that shares memory with b).  FP arithmetic
+// never produces a signalling NaN (a NaN result is quiet), so a stored value is never mistaken
+// for it.  A task polls the values it reads themselves, with agent-scope atomic loads, until
+// none is the marker, and stores its rows with agent-scope atomic stores, which reach the
+// coherence point without a release.
 constexpr unsigned long long SOLVE_PENDING = 0x7FF4C0DE5EED0001ull;
 
-// Before the two passes: the outputs of both pending, the task counters of both (ctrl[0],
-// ctrl[4]) at zero and, before the first columns, their abort words (ctrl[1], ctrl[5]).
+// Before the two passes: the outputs of both pending (x null: y alone), the task counters of
+// both (ctrl[0], ctrl[4]) at zero and, before the first columns, their abort words (ctrl[1],
+// ctrl[5]).
 __global__ void k_solve_begin(int* ctrl, int first, double* y, double* x, int64_t n) {
     if (blockIdx.x == 0 && threadIdx.x < SOLVE_CTRL_WORDS && (first || threadIdx.x % 4 == 0)) ctrl[threadIdx.x] = 0;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
         reinterpret_cast<unsigned long long*>(y)[i] = SOLVE_PENDING;
-        reinterpret_cast<unsigned long long*>(x)[i] = SOLVE_PENDING;
+        if (x) reinterpret_cast<unsigned long long*>(x)[i] = SOLVE_PENDING;
     }
+}
+__global__ void k_fill_pending(double* x, int64_t n) {
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+        reinterpret_cast<unsigned long long*>(x)[i] = SOLVE_PENDING;
 }
 
 // A wait has exceeded its bound: every task ends.  A release, so that whoever sees the word
@@ -711,25 +717,30 @@ int launch_pass(Context* c, Factor* f, const SolveWork& w, bool mfma, bool forwa
 }  // namespace
 
 // Both passes over nrhs columns, enqueued on the context stream between the events ev0 and
-// ev1; d_x may not alias d_b.  solve_finish waits and looks at the outcome.
+// ev1.  d_x may be d_b: the forward pass reads b and writes y, and an x that shares memory
+// with b is marked pending only after it (one launch more).  solve_finish waits and looks at
+// the outcome.
 int solve_launch(Context* c, Factor* f, const SolveWork& w, const double* d_b, double* d_x, int nrhs) {
     const int R = f->block_rows;
     int rc;
     HIP_TRY(c, hipEventRecord(c->ev0, c->stream));
     const int64_t ld = (int64_t)R * TS;
     const bool mfma = nrhs >= TRSM_MIN_RHS;
+    const uintptr_t b0 = (uintptr_t)d_b, x0 = (uintptr_t)d_x, bytes = (uintptr_t)ld * (uintptr_t)nrhs * sizeof(double);
+    const bool shared = b0 < x0 + bytes && x0 < b0 + bytes;
     for (int c0 = 0; c0 < nrhs; c0 += MAX_RHS) {
         const int m = std::min(MAX_RHS, nrhs - c0);
         const int64_t off = (int64_t)c0 * ld, n = ld * m;
         const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 2048));
-        hipLaunchKernelGGL(k_solve_begin, dim3(grid), dim3(256), 0, c->stream, w.ctrl, c0 == 0, w.y + off, d_x + off, n);
-        if (f->elem == 8) {
-            if ((rc = launch_pass<double>(c, f, w, mfma, true, d_b + off, w.y + off, m))) return rc;
-            if ((rc = launch_pass<double>(c, f, w, mfma, false, w.y + off, d_x + off, m))) return rc;
-        } else {
-            if ((rc = launch_pass<float>(c, f, w, mfma, true, d_b + off, w.y + off, m))) return rc;
-            if ((rc = launch_pass<float>(c, f, w, mfma, false, w.y + off, d_x + off, m))) return rc;
-        }
+        auto pass = [&](bool forward, const double* in, double* out) {
+            return f->elem == 8 ? launch_pass<double>(c, f, w, mfma, forward, in, out, m)
+                                : launch_pass<float>(c, f, w, mfma, forward, in, out, m);
+        };
+        hipLaunchKernelGGL(k_solve_begin, dim3(grid), dim3(256), 0, c->stream, w.ctrl, c0 == 0, w.y + off,
+                           shared ? nullptr : d_x + off, n);
+        if ((rc = pass(true, d_b + off, w.y + off))) return rc;
+        if (shared) hipLaunchKernelGGL(k_fill_pending, dim3(grid), dim3(256), 0, c->stream, d_x + off, n);
+        if ((rc = pass(false, w.y + off, d_x + off))) return rc;
     }
     HIP_TRY(c, hipEventRecord(c->ev1, c->stream));
     return SOGL_OK;
