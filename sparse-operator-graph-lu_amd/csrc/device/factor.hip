@@ -1476,8 +1476,11 @@ void build_after_links(Factor* f, const HostGraph& hg, std::vector<char>& linked
 // (S_{k+1,k+1} = P - L_{k+1,k} U_{k,k+1}, tile_order.h), its workgroup runs all three and the
 // next lu after them: the diagonal of a banded factor is one workgroup's work (diag_step).
 // Deadlock freedom: every wait in such a chain, and every other wait, is for a task of lower
-// index than the waiting one's (checked here for the panels, which run with the lu, by the
-// dependency levels else), and the queue hands tasks out by index.  Of the unfinished tasks
+// index than the waiting one's, and the queue hands tasks out by index.  The dependency levels
+// give it for every task by itself; but the lu waits for what its panels and the update read
+// (S_l, S_u and P) before it publishes, so their makers have to come before the lu too: checked
+// here and by validate_graph.  (A P made later, by a long chain beside an early lu, stopped the
+// kernel: the tasks that read that lu's tiles held every workgroup.)  Of the unfinished tasks
 // the lowest, m, waits for nothing.  Every queue entry before it is finished, so the
 // workgroups not on m are on chains whose heads come before it; with fewer such chains
 // than workgroups (launch_factor checks it) one is free to take m.  So there are at most
@@ -1521,7 +1524,7 @@ bool build_diag_chains(Factor* f, const HostGraph& hg, std::vector<char>& linked
         const Pair& pr = hg.pairs[(size_t)k.a];
         const int32_t pl = maker(pair_a(pr)), pu = maker(pair_b(pr));
         int32_t l0 = -1, l1 = -1;
-        if (!panel(pl, l0, 0) || !panel(pu, l1, 1) || l0 != l1 || used[(size_t)l0]) continue;
+        if (!panel(pl, l0, 0) || !panel(pu, l1, 1) || l0 != l1 || used[(size_t)l0] || maker(k.add) > l0) continue;
         const bool llt = f->tasks[(size_t)l0].kind == TK_LLT;
         if ((pr.a < 0) != llt || (pl == pu) != llt) continue;
         used[(size_t)l0] = 1;
@@ -2271,11 +2274,13 @@ int validate_graph(Context* c, const sogl_factor_desc* d, const Factor* f, const
         for (size_t t = 0; t < T; t++) {
             const DevTask& k = f->tasks[t];
             if (pred[t] < 0 || k.kind != TK_GEMM || f->tasks[(size_t)pred[t]].next == (int32_t)t) continue;
-            if (f->tasks[(size_t)pred[t]].dia >= 0) {  // a diagonal chain's waits are for lower indices
-                const size_t at = f->tasks[(size_t)pred[t]].dia == (int32_t)t ? t : (size_t)pred[t];
-                for (int32_t q = k.dep_begin; q < k.dep_begin + k.dep_count; q++) {
-                    const int32_t p = producer[(size_t)hg.deps[(size_t)q]];
-                    if (p >= 0 && p != pred[t] && (size_t)p >= at)
+            if (f->tasks[(size_t)pred[t]].dia >= 0) {
+                // a diagonal chain's waits, made by its lu, are for tasks before the lu
+                const DevTask& l = f->tasks[(size_t)pred[t]];
+                const Pair& pr = hg.pairs[(size_t)k.a];
+                for (int32_t s2 : {pair_a(pr), pair_b(pr), k.add}) {
+                    const int32_t p = s2 >= 0 ? producer[(size_t)s2] : -1;
+                    if (p > pred[t] && !(l.dia == (int32_t)t && (p == l.pan_l || p == l.pan_u)))
                         return bad("task " + std::to_string(t) + " of a diagonal chain waits for a later task");
                 }
                 if (in_chain.insert(head[t]).second && ++chains > DIAG_CHAINS) return bad("too many diagonal chains");

@@ -1,0 +1,132 @@
+"""The order in which the persistent executor's workgroups can run a task graph with diagonal chains, on
+the CPU: host/graph_model.hip builds the graph with the executor's own code and plays the queue without
+times.  Every number of workgroups above the number of chains has to finish every task, with the chain's
+steps inside its lu (one workgroup per CU), after it (two), and with dynamic chaining."""
+import ctypes as C
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+import sogl
+import workloads as W
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+PKG = os.path.join(ROOT, "sparse-operator-graph-lu_amd")
+HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    d = tmp_path_factory.mktemp("graph_model")
+    obj, so = str(d / "model.o"), str(d / "model.so")
+    r = subprocess.run([HIPCC, "-std=c++17", "-O1", "-fPIC", "--offload-arch=gfx950", "--offload-host-only", "-fuse-cuid=none",
+                        "-I", os.path.join(ROOT, "include"), "-c", os.path.join(ROOT, "tests", "host", "graph_model.hip"),
+                        "-o", obj], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr[-2000:]
+    host = os.path.join(PKG, "build", "libsogl_host.so")
+    rocm = os.path.dirname(os.path.dirname(HIPCC)) + "/lib"
+    r = subprocess.run(["g++", "-shared", "-Wl,-Bsymbolic", "-o", so, obj, host, f"-L{rocm}", "-lamdhip64",
+                        f"-Wl,-rpath,{rocm}", f"-Wl,-rpath,{os.path.dirname(host)}"], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr[-2000:]
+    return C.CDLL(so)
+
+
+def fill(n, pairs):
+    """Block rows of L (strictly lower) of a symmetric block pattern after elimination in order."""
+    rows = [set() for _ in range(n)]
+    for i, j in pairs:
+        rows[max(i, j)].add(min(i, j))
+    cols = [set() for _ in range(n)]
+    for i in range(n):
+        for j in rows[i]:
+            cols[j].add(i)
+    for j in range(n):
+        c = sorted(cols[j])
+        for a, i in enumerate(c):
+            for k in c[a + 1:]:
+                rows[k].add(i)
+                cols[i].add(k)
+    return rows
+
+
+def leaf_beside_chain(depth, width):
+    """A tridiagonal chain of `depth` block rows, then a block coupled to none of them, then `width` rows
+    coupled to it, the first of them to the chain's end as well: that row's diagonal has an update from
+    the chain that is made long after the leaf's lu could be."""
+    leaf = depth
+    pairs = [(i, i + 1) for i in range(depth - 1)] + [(leaf, leaf + 1 + k) for k in range(width)] + [(depth - 1, leaf + 1)]
+    return depth + 1 + width, pairs
+
+
+def band(n, half):
+    return n, [(i, j) for i in range(n) for j in range(max(0, i - half), i)]
+
+
+LU, LLT = 1, 10
+
+
+def describe(n, pairs, symmetric, precision):
+    """A factor description of the block pattern (one op, which says LU or L L^T; the tile-column list takes its
+    place) and its inputs' block coordinates."""
+    at = [(i, i) for i in range(n)] + [(max(p), min(p)) for p in pairs]
+    if not symmetric:
+        at += [(j, i) for i, j in at if i != j]
+    ids = np.arange(1, len(at) + 1, dtype=np.int32)
+    nid = len(at) + 1
+    rows = fill(n, pairs)
+    lt, ut = [], []
+    for i in range(n):
+        for j in sorted(rows[i]) + [i]:
+            lt.append([i, j, nid])
+            nid += 1
+            if not symmetric:
+                ut.append([j, i, nid])
+                nid += 1
+    op = [[1, 0, LLT if symmetric else LU, lt[0][2], 0 if symmetric else ut[0][2], 1, 0, 0]]
+    d, keep = sogl.make_desc(nid, op, ids, np.zeros((1, 1)), lt, ut if ut else np.zeros((0, 3)), n, precision)
+    bi, bj = (np.array([a[k] for a in at], np.int32) for k in range(2))
+    return d, (keep, bi, bj), bi.ctypes.data_as(C.c_void_p), bj.ctypes.data_as(C.c_void_p)
+
+
+def play(lib, desc, workgroups, one, claims):
+    d, _, bi, bj = desc
+    out = np.zeros(5, np.int64)
+    assert lib.model(C.byref(d), bi, bj, workgroups, one, claims, out.ctypes.data_as(C.c_void_p)) == sogl.OK
+    return dict(zip(("tasks", "finished", "steps", "chains", "claimers"), (int(v) for v in out)))
+
+
+PATTERNS = {
+    "leaf_beside_chain": lambda: leaf_beside_chain(12, 8),
+    "wide_leaf_beside_chain": lambda: leaf_beside_chain(40, 30),
+    "band_3": lambda: band(14, 3),
+    "tridiagonal": lambda: band(20, 1),
+}
+
+
+@pytest.mark.parametrize("symmetric", [False, True])
+@pytest.mark.parametrize("name", sorted(PATTERNS))
+@pytest.mark.parametrize("one,claims", [(1, 0), (0, 0), (1, 4), (0, 4)])
+def test_every_task_finishes(lib, name, symmetric, one, claims):
+    desc = describe(*PATTERNS[name](), symmetric, sogl.FP64)
+    chains = play(lib, desc, 64, one, claims)["chains"]
+    for workgroups in range(chains + 1, chains + 8):
+        r = play(lib, desc, workgroups, one, claims)
+        assert r["finished"] == r["tasks"], (workgroups, r)
+
+
+def test_bands_are_chains(lib):
+    for half in (1, 3):  # every diagonal but the first comes from a chain's step
+        r = play(lib, describe(*band(14, half), False, sogl.FP32), 4, 1, 0)
+        assert (r["chains"], r["steps"]) == (1, 13)
+
+
+@pytest.mark.parametrize("symmetric", [False, True])
+def test_late_sum_breaks_the_chain(lib, symmetric):
+    """The leaf's step is not linked (the row's other updates come long after the leaf's lu), and a graph
+    with such a link is refused."""
+    desc = describe(*leaf_beside_chain(12, 8), symmetric, sogl.FP64)
+    assert play(lib, desc, 4, 1, 0)["steps"] == 11 + 7  # along the chain, and along the leaf's rows
+    d, _, bi, bj = describe(*band(14, 3), symmetric, sogl.FP64)
+    assert lib.plant_late_sum(C.byref(d), bi, bj) > 0
