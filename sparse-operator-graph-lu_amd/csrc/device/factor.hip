@@ -1277,11 +1277,16 @@ void build_chains(Factor* f, HostGraph& hg) {
     std::vector<std::vector<int32_t>> cand(T);
     std::vector<int32_t> nchk(T, 0);
     std::vector<int32_t> order;
-    // after-links keep their chains in their heads' workgroups: neither end is claimed
+    // after-links keep their chains in their heads' workgroups: neither end is claimed, nor the
+    // sum whose lu is one.  A workgroup runs what it has claimed when its chain ends, and with
+    // after-links no task of a chain waits for a later chain's; a diagonal chain's tasks wait
+    // for any earlier task, a claimed one included, so they claim none.
     std::vector<char> linked(T, 0);
     for (size_t t = 0; t < T; t++)
         for (int32_t u : {f->tasks[t].after, f->tasks[t].pan_l, f->tasks[t].pan_u, f->tasks[t].dia})
             if (u >= 0) linked[(size_t)u] = linked[t] = 1;
+    for (size_t t = 0; t < T; t++)
+        if (f->tasks[t].next >= 0 && linked[(size_t)f->tasks[t].next]) linked[t] = 1;
     for (size_t u = 0; u < T; u++) {
         const DevTask& k = f->tasks[u];
         if (k.kind == TK_GEMM && k.b >= 1 && k.b <= CHAIN_MAX_PAIRS && !linked[u] &&
@@ -1299,7 +1304,7 @@ void build_chains(Factor* f, HostGraph& hg) {
         bool any = false;
         for (int l = 0; l < n; l++) {
             const int32_t p = slot_task[(size_t)sl[l]];
-            if (p < 0) continue;
+            if (p < 0 || (f->n_diag_chains && linked[(size_t)p])) continue;
             auto& cl = cand[(size_t)p];
             if (std::find(cl.begin(), cl.end(), u) != cl.end()) continue;
             if ((int)cl.size() >= CHAIN_MAX_CANDS || nchk[(size_t)p] + nent > CHAIN_MAX_CHECKS) continue;
@@ -2283,6 +2288,8 @@ int validate_graph(Context* c, const sogl_factor_desc* d, const Factor* f, const
                     if (p > pred[t] && !(l.dia == (int32_t)t && (p == l.pan_l || p == l.pan_u)))
                         return bad("task " + std::to_string(t) + " of a diagonal chain waits for a later task");
                 }
+                if (k.chk_count || l.chk_count)
+                    return bad("task " + std::to_string(t) + " of a diagonal chain claims others");
                 if (in_chain.insert(head[t]).second && ++chains > DIAG_CHAINS) return bad("too many diagonal chains");
                 continue;
             }
@@ -2313,6 +2320,8 @@ int validate_graph(Context* c, const sogl_factor_desc* d, const Factor* f, const
             if (u.kind != TK_GEMM || u.b < 1 || u.b > CHAIN_MAX_PAIRS || (e.pos < 4 && e.pos >= 2 * u.b) ||
                 (e.pos == 4 && u.add < 0))
                 return bad("chain candidate " + std::to_string(e.task));
+            if (u.next >= 0 && f->tasks[(size_t)u.next].dia >= 0)
+                return bad("claimed task " + std::to_string(e.task) + " begins a diagonal chain");
             const Pair& pr = hg.pairs[(size_t)(u.a + (e.pos < 4 ? e.pos / 2 : 0))];
             const int32_t operand = e.pos == 4 ? u.add : ((e.pos & 1) ? pair_b(pr) : pair_a(pr));
             const bool own = operand == k.out0 || operand == k.out1 || operand == k.out2 || operand == k.out3;

@@ -130,3 +130,100 @@ def test_late_sum_breaks_the_chain(lib, symmetric):
     assert play(lib, desc, 4, 1, 0)["steps"] == 11 + 7  # along the chain, and along the leaf's rows
     d, _, bi, bj = describe(*band(14, 3), symmetric, sogl.FP64)
     assert lib.plant_late_sum(C.byref(d), bi, bj) > 0
+
+
+class Ops:
+    """An op list over new ids, kept by stage."""
+    LINV, UINV, SUB, MUL = 2, 3, 4, 8
+
+    def __init__(self, inputs):
+        self.inputs = {key: k + 1 for k, key in enumerate(inputs)}
+        self.n_ids = len(self.inputs) + 1
+        self.rows, self.lt, self.ut = [], [], []
+
+    def __getitem__(self, key):
+        return self.inputs[key]
+
+    def op(self, code, src, src2, stage, res=None):
+        if res is None:
+            res, self.n_ids = self.n_ids, self.n_ids + 1
+        self.rows.append([src, src2, code, res, 0, stage, 0, 0])
+        return res
+
+    def less(self, a, products, stage):
+        """a - sum of the products"""
+        acc = None
+        for x, y in products:
+            acc = self.op(self.MUL, x, y, stage, acc)
+        return self.op(self.SUB, acc, a, stage + 1)
+
+    def lu(self, k, s, stage):
+        low = self.op(LU, s, 0, stage)
+        up, self.n_ids = self.n_ids, self.n_ids + 1
+        self.rows[-1][4] = up
+        self.lt.append([k, k, low])
+        self.ut.append([k, k, up])
+        return self.op(self.LINV, low, 0, stage + 1), self.op(self.UINV, up, 0, stage + 1)
+
+    def panels(self, k, x, z, s_l, s_u, stage):
+        pl, pu = self.op(self.MUL, s_l, z, stage), self.op(self.MUL, x, s_u, stage)
+        self.lt.append([k + 1, k, pl])
+        self.ut.append([k, k + 1, pu])
+        return pl, pu
+
+    def desc(self, n):
+        rows = sorted(self.rows, key=lambda r: r[5])
+        for k, r in enumerate(rows):
+            r[6] = k
+        ids = np.arange(1, len(self.inputs) + 1, dtype=np.int32)
+        d, keep = sogl.make_desc(self.n_ids, rows, ids, np.zeros((1, 1)), self.lt, self.ut, n, sogl.FP64)
+        return d, keep, None, None
+
+
+def tridiagonal_inputs(n):
+    return [(i, i) for i in range(n)] + [(i + 1, i) for i in range(n - 1)] + [(i, i + 1) for i in range(n - 1)] + ["v"]
+
+
+def claims_inside_a_chain():
+    """The first step's panel could claim a product that the third step's panel needs (a sum of 60 products
+    follows the claimed one, so it is on the critical path)."""
+    n = 4
+    o = Ops(tridiagonal_inputs(n))
+    s, first = o[0, 0], None
+    for k in range(n):
+        st = 10 * k + 1
+        x, z = o.lu(k, s, st)
+        if k == n - 1:
+            break
+        s_l, v = o[k + 1, k], o["v"]
+        if k == 2:
+            s_l = o.less(s_l, [(o.op(o.MUL, first, v, 5), v)] + [(v, v)] * 60, 6)
+        pl, pu = o.panels(k, x, z, s_l, o[k, k + 1], st + 2)
+        first = first or pl
+        s = o.less(o[k + 1, k + 1], [(pl, pu)], st + 3)
+    return o.desc(n)
+
+
+def claims_before_a_chain():
+    """A product outside any chain could claim the sum that a chain's first lu follows, and with it another
+    that this lu's panel needs (a sum of 13 products follows that one: both are on the critical path)."""
+    o = Ops(tridiagonal_inputs(2))
+    v = o["v"]
+    p = o.op(o.MUL, v, v, 1)
+    s_l = o.less(o[1, 0], [(o.op(o.MUL, p, v, 2), v)] + [(v, v)] * 12, 3)
+    x, z = o.lu(0, o.less(o[0, 0], [(p, v)], 2), 5)
+    pl, pu = o.panels(0, x, z, s_l, o[0, 1], 7)
+    o.lu(1, o.less(o[1, 1], [(pl, pu)], 8), 10)
+    return o.desc(2)
+
+
+@pytest.mark.parametrize("make", [claims_inside_a_chain, claims_before_a_chain])
+def test_claims_beside_a_chain(lib, make):
+    """Dynamic chaining: a workgroup runs the tasks it has claimed when its chain ends, so a workgroup on a
+    diagonal chain may hold none."""
+    desc = make()
+    for claims in (0, 1, 8):
+        for workgroups in (2, 3, 8):
+            r = play(lib, desc, workgroups, 0, claims)
+            assert r["steps"] > 0 and r["finished"] == r["tasks"], (claims, workgroups, r)
+    assert r["claimers"] == 0
