@@ -783,6 +783,7 @@ int solve_device(Context* c, Factor* f, const double* d_b, double* d_x, int nrhs
 int ensure_vectors(Context* c, Factor* f, int nrhs) {
     const size_t need = (size_t)f->block_rows * TS * (size_t)nrhs;
     if (f->vec_cap >= need) return SOGL_OK;
+    f->vec_cap = 0;  // a growth that fails leaves a vector freed
     int rc;
     if ((rc = dev_alloc(c, f->vec_b, need * 8, "rhs")) || (rc = dev_alloc(c, f->vec_x, need * 8, "x")) ||
         (rc = dev_alloc(c, f->vec_y, need * 8, "y")))

@@ -3,34 +3,17 @@ the CPU: host/graph_model.hip builds the graph with the executor's own code and 
 times.  Every number of workgroups above the number of chains has to finish every task, with the chain's
 steps inside its lu (one workgroup per CU), after it (two), and with dynamic chaining."""
 import ctypes as C
-import os
-import subprocess
 
 import numpy as np
 import pytest
 
+import host_lib
 import sogl
-import workloads as W
-
-ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-PKG = os.path.join(ROOT, "sparse-operator-graph-lu_amd")
-HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 
 @pytest.fixture(scope="module")
 def lib(tmp_path_factory):
-    d = tmp_path_factory.mktemp("graph_model")
-    obj, so = str(d / "model.o"), str(d / "model.so")
-    r = subprocess.run([HIPCC, "-std=c++17", "-O1", "-fPIC", "--offload-arch=gfx950", "--offload-host-only", "-fuse-cuid=none",
-                        "-I", os.path.join(ROOT, "include"), "-c", os.path.join(ROOT, "tests", "host", "graph_model.hip"),
-                        "-o", obj], capture_output=True, text=True, timeout=300)
-    assert r.returncode == 0, r.stderr[-2000:]
-    host = os.path.join(PKG, "build", "libsogl_host.so")
-    rocm = os.path.dirname(os.path.dirname(HIPCC)) + "/lib"
-    r = subprocess.run(["g++", "-shared", "-Wl,-Bsymbolic", "-o", so, obj, host, f"-L{rocm}", "-lamdhip64",
-                        f"-Wl,-rpath,{rocm}", f"-Wl,-rpath,{os.path.dirname(host)}"], capture_output=True, text=True, timeout=300)
-    assert r.returncode == 0, r.stderr[-2000:]
-    return C.CDLL(so)
+    return host_lib.build("graph_model", str(tmp_path_factory.mktemp("graph_model")))
 
 
 def fill(n, pairs):
