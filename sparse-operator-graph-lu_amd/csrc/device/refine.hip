@@ -55,7 +55,8 @@ __global__ void k_axpy(double* x, const double* d, int64_t n) {
 // the caller's order, xo[new_order[i]] = x[i] (GOrder::reOrderResult, GPSOrder.cpp:41-53);
 // per column, over the first n rows, {||r||_2^2, ||x||_2^2, ||b||_2^2, ||r||_inf, ||x||_inf,
 // ||b||_inf} and, after the columns, whether a pass of the solve was aborted, to pinned host
-// memory `norms`, so that the host's one wait brings everything it decides by.  (As a
+// memory `norms`, so that the host's one wait brings everything it decides by.  Where a pass was
+// aborted, xo is left as it is; with xold, what xo held goes there first.  (As a
 // residual, norm, copy and output kernel with a copy of the control words and three waits,
 // and with every column in turn in one thread per row, it was half of a resident solve:
 // random band 4,099 x 100 columns 3.1 of 3.6 ms, 2D 64^2 0.13 of 0.24.)
@@ -80,12 +81,13 @@ __device__ inline double wave_reduce(double v) {
 template <int CW>
 __global__ __launch_bounds__(RES_NT) void k_residual(const int64_t* ptr, const int32_t* col, const double* val,
                                                      const double* b, const double* x, double* r, double* xo,
-                                                     const int32_t* new_order, int32_t n, int64_t N, int nrhs,
+                                                     double* xold, const int32_t* new_order, int32_t n, int64_t N, int nrhs,
                                                      double* part, int* count, const int* ctrl, double* norms) {
     __shared__ double s_w[RES_NT / 64][CW * NORM_VALUES];
     __shared__ int s_last;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, nb = gridDim.x;
     const int c0 = blockIdx.y * CW, cw = min(CW, nrhs - c0);
+    const bool aborted = ctrl[1] || ctrl[5];
     const double* xc[CW];  // a column past the last repeats it and is not stored
 #pragma unroll
     for (int c = 0; c < CW; c++) xc[c] = x + (int64_t)(c0 + min(c, cw - 1)) * N;
@@ -129,7 +131,11 @@ __global__ __launch_bounds__(RES_NT) void k_residual(const int64_t* ptr, const i
             const double bv = b[i + (int64_t)(c0 + c) * N], xv = xc[c][i], rv = bv - s[c];
             r[i + (int64_t)(c0 + c) * N] = rv;
             if (i < n) {
-                xo[o + (int64_t)(c0 + c) * n] = xv;
+                if (!aborted) {
+                    const int64_t q = o + (int64_t)(c0 + c) * n;
+                    if (xold) xold[q] = xo[q];
+                    xo[q] = xv;
+                }
                 acc[c][0] += rv * rv;
                 acc[c][1] += xv * xv;
                 acc[c][2] += bv * bv;
@@ -161,7 +167,7 @@ __global__ __launch_bounds__(RES_NT) void k_residual(const int64_t* ptr, const i
     if (!s_last) return;
     if (tid == 0) {
         count[blockIdx.y] = 0;  // for the next launch
-        if (blockIdx.y == 0) norms[(int64_t)nrhs * NORM_VALUES] = ctrl[1] || ctrl[5] ? 1.0 : 0.0;
+        if (blockIdx.y == 0) norms[(int64_t)nrhs * NORM_VALUES] = aborted ? 1.0 : 0.0;
     }
     for (int v = w; v < cw * NORM_VALUES; v += RES_NT / 64) {
         const double* q = part + ((int64_t)c0 * NORM_VALUES + v) * nb;
@@ -252,7 +258,9 @@ extern "C" int sogl_refine_attach(sogl_ctx* x, int32_t factor_id, const sogl_pla
     return SOGL_OK;
 }
 
-static int refined_core(Context* c, Factor* f, const double* d_b, double* d_x, int32_t nrhs, double tol,
+// d_old (n x nrhs): takes what d_x held, which gets it back where a correction's solve fails;
+// null: d_x may be left with an earlier iterate then.
+static int refined_core(Context* c, Factor* f, const double* d_b, double* d_x, double* d_old, int32_t nrhs, double tol,
                         int32_t max_iter, int32_t* iters, double* resid) {
     const int32_t n = f->n;
     const int64_t N = (int64_t)f->block_rows * TS;
@@ -289,18 +297,25 @@ static int refined_core(Context* c, Factor* f, const double* d_b, double* d_x, i
     double solve_ms = 0;
     int it = 0;
     double worst = 0;
+    auto fail = [&](int code) {
+        if (it > 0 && d_old) {
+            HIP_TRY(c, hipMemcpyAsync(d_x, d_old, (size_t)n * nrhs * 8, hipMemcpyDeviceToDevice, c->stream));
+            HIP_TRY(c, hipStreamSynchronize(c->stream));
+        }
+        return code;
+    };
     for (;;) {
         auto kern = cw == 1 ? k_residual<1> : k_residual<RES_CW>;
         hipLaunchKernelGGL(kern, dim3(nb, groups), dim3(RES_NT), 0, c->stream, (const int64_t*)f->csr_ptr.p,
                            (const int32_t*)f->csr_col.p, (const double*)f->csr_val.p, (const double*)db,
-                           (const double*)dx, dr, d_x, (const int32_t*)f->perm_d.p, n, N, nrhs, (double*)f->red.p, count,
-                           (const int*)w.ctrl, d_norms);
+                           (const double*)dx, dr, d_x, it == 0 ? d_old : nullptr, (const int32_t*)f->perm_d.p, n, N, nrhs,
+                           (double*)f->red.p, count, (const int*)w.ctrl, d_norms);
         HIP_TRY(c, hipGetLastError());
         HIP_TRY(c, hipStreamSynchronize(c->stream));
         float ms = 0;
         HIP_TRY(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
         solve_ms += ms;
-        if (c->norms_h[norms - 1] != 0) return solve_timeout(c);
+        if (c->norms_h[norms - 1] != 0) return fail(solve_timeout(c));
         worst = 0;
         for (int32_t r = 0; r < nrhs; r++) {
             const double* v = c->norms_h + (size_t)r * NORM_VALUES;
@@ -312,10 +327,10 @@ static int refined_core(Context* c, Factor* f, const double* d_b, double* d_x, i
             if (!(rel <= worst)) worst = rel;  // NaN propagates
         }
         if (worst <= tol || it >= max_iter || std::isnan(worst)) break;
-        if ((rc = solve_launch(c, f, w, dr, dd, nrhs))) return rc;
+        it++;
+        if ((rc = solve_launch(c, f, w, dr, dd, nrhs))) return fail(rc);
         hipLaunchKernelGGL(k_axpy, dim3(gA), dim3(256), 0, c->stream, dx, (const double*)dd, N * nrhs);
         HIP_TRY(c, hipGetLastError());
-        it++;
     }
     f->solve_ms = solve_ms;
     if (iters) *iters = it;
@@ -335,7 +350,9 @@ extern "C" int sogl_solve_refined_device(sogl_ctx* x, int32_t factor_id, const d
     if (!f) return set_error(c, SOGL_ERR_ARG, "unknown factor id");
     if (!f->has_refine) return set_error(c, SOGL_ERR_ARG, "sogl_refine_attach was not called");
     HIP_TRY(c, hipSetDevice(c->device));
-    return refined_core(c, f, d_b, d_x, nrhs, tol, max_iter, iters, resid);
+    int rc;
+    if (max_iter > 0 && (rc = dev_alloc(c, f->vec_io, (size_t)f->n * nrhs * 8, "earlier x"))) return rc;
+    return refined_core(c, f, d_b, d_x, max_iter > 0 ? (double*)f->vec_io.p : nullptr, nrhs, tol, max_iter, iters, resid);
 }
 
 extern "C" int sogl_solve_refined(sogl_ctx* x, int32_t factor_id, const double* b, double* xo,
@@ -354,7 +371,7 @@ extern "C" int sogl_solve_refined(sogl_ctx* x, int32_t factor_id, const double* 
     double* db = (double*)f->vec_io.p;
     double* dx = db + (size_t)f->n * nrhs;
     HIP_TRY(c, hipMemcpyAsync(db, b, bytes, hipMemcpyHostToDevice, c->stream));
-    int rc2 = refined_core(c, f, db, dx, nrhs, tol, max_iter, iters, resid);
+    int rc2 = refined_core(c, f, db, dx, nullptr, nrhs, tol, max_iter, iters, resid);
     if (rc2 != SOGL_OK && rc2 != SOGL_ERR_NOT_CONVERGED && rc2 != SOGL_ERR_NAN) return rc2;
     HIP_TRY(c, hipMemcpyAsync(xo, dx, bytes, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(c, hipStreamSynchronize(c->stream));
