@@ -206,10 +206,11 @@ int sogl_ctx_set_pool_reuse(sogl_ctx* ctx, int32_t mode);
  * a stage's ops on a thread pool); results are the same bits with any mask.
  *   SOGL_LINK_PANEL: the lu / llt task of an FP32 or FP64 factor runs its panels next to
  *     the diagonal and the next diagonal tile's last update itself, in LDS, and its
- *     workgroup goes on with that tile's lu (diagonal chains); where there would be too
- *     many such chains, or with SOGL_LINK_AFTER, the lu of an FP32 LU factor runs its
- *     most critical panel GEMM (A U^-1 or L^-1 A, one pair), from the inverse it keeps in
- *     LDS, and publishes both tiles at once.
+ *     workgroup goes on with that tile's lu (diagonal chains, in the runs that
+ *     sogl_factor_run_config names); where there would be too many such chains, or with
+ *     SOGL_LINK_AFTER, the lu of an FP32 LU factor runs its most critical panel GEMM
+ *     (A U^-1 or L^-1 A, one pair), from the inverse it keeps in LDS, and publishes both
+ *     tiles at once.
  *   SOGL_LINK_AFTER: the workgroup that made a tile on the critical path goes on, right
  *     after publishing it, to a one-pair GEMM that reads it, instead of handing it to
  *     another workgroup (measured slower: off by default).
@@ -250,7 +251,9 @@ int sogl_tile_order_ops(const sogl_plan* plan, sogl_op* ops, int64_t* n_ops, int
  * resident input tiles. */
 int sogl_factor_run(sogl_ctx* ctx, int32_t factor_id, int32_t exec_mode);
 /* Same with the persistent executor's queue settings: chunk = tasks taken per fetch
- * (1..64), wg_per_cu = resident workgroups per CU (0: as many as fit). */
+ * (1..64), wg_per_cu = resident workgroups per CU (0: one for a graph of few tasks per
+ * dependency level, else as many as fit).  Diagonal chains (SOGL_LINK_PANEL) run with chunk
+ * 1, one workgroup per CU and no dynamic chaining. */
 int sogl_factor_run_config(sogl_ctx* ctx, int32_t factor_id, int32_t exec_mode, int32_t chunk,
                            int32_t wg_per_cu);
 /* Autotuner: times each executor configuration `trials` times (best of) on this

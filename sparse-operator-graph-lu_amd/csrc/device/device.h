@@ -154,6 +154,8 @@ struct Factor {
     std::vector<int32_t> chain_head;       // per task: the queued task whose workgroup runs it
     int32_t chain_claims = 0;              // persistent executor: claims per finished task (0: off)
     std::vector<int32_t> queue;            // persistent executor: task indices handed out, in order
+    std::vector<int32_t> queue_all;        // and those of a run without the diagonal chains' links
+    DevBuf queue_all_d;                    // (part of index_d)
     DevBuf mask_d;                         // per slot: 16x16 block mask (uint32)
     int32_t epoch = 0;
     // triangular solve structure (block CSR by block row, off-diagonal only)

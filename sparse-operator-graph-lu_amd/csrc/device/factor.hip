@@ -179,6 +179,7 @@ struct Args {
     const ChainChk* chk;  // persistent executor: chain candidates' check entries
     int32_t chain;        // claims per finished task at most (0: no dynamic chaining)
     const DiagRec* diag;
+    int32_t diag_chains;  // persistent executor: run the diagonal chains' links (launch_factor)
     const int32_t* war;   // value ids whose readers a reused result slot waits for (DevTask)
 };
 
@@ -844,7 +845,8 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
     // LU kernels built for one workgroup per CU: lu tasks run their panel GEMMs
     // (DevTask::pan_l / pan_u) inside themselves, keeping copies of the inverses in LDS
     // beyond what any task kind uses.  The kernels built for two (no registers to spare)
-    // run them as after-links instead: right after the lu, in the same workgroup.
+    // run them as after-links instead: right after the lu, in the same workgroup (a diagonal
+    // chain's as queued tasks).
     constexpr bool ABSORB = !BF16 && !LLT && ONE;
     constexpr bool CHAINS = !BF16 && ONE;  // and lu / llt tasks run diagonal chains' steps
     constexpr int XCOPY_BYTES = CHAINS ? TS * lda<T>() * (int)sizeof(T) : 0;
@@ -854,9 +856,7 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
     T* const zcopy = ABSORB ? reinterpret_cast<T*>(lds + lds_bytes<T>() + XCOPY_BYTES) : nullptr;
     __shared__ uint32_t s_pmask[2][NT / 64];
     __shared__ uint32_t s_word;
-    // an absorbed panel, and the next diagonal tile's update, still to run as after-links
-    // (kernels without the copies)
-    __shared__ int s_pend, s_pend_d;
+    __shared__ int s_pend;  // an absorbed panel still to run as an after-link (kernels without the copies)
     __shared__ uint32_t s_words[3];
     __shared__ int s_task;
     __shared__ int s_abort;
@@ -878,7 +878,7 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
             s_abort = __hip_atomic_load(a.ctrl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             s_task = s_abort ? a.nqueue : atomicAdd(a.ctrl, a.chunk);
             s_ring_head = s_ring_n = 0;
-            s_pend = s_pend_d = -1;
+            s_pend = -1;
         }
         __syncthreads();
         // wave-uniform loop control: the exit branch must not depend on the lane
@@ -931,9 +931,10 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
         }
         // an lu with absorbed panels (wave-uniform task fields): the panels' descriptors
         // (with dynamic chaining on, panels run as after-links, whose outputs' candidates
-        // can be claimed)
-        const bool absorbs = CHAINS && !a.chain && t.kind == (LLT ? TK_LLT : TK_LU) && (t.pan_l >= 0 || t.pan_u >= 0);
-        const bool has_d = absorbs && t.rec >= 0;
+        // can be claimed); those of a diagonal chain's lu run inside it or from the queue
+        const bool absorbs = CHAINS && t.kind == (LLT ? TK_LLT : TK_LU) && (t.pan_l >= 0 || t.pan_u >= 0) &&
+                             (t.dia >= 0 ? a.diag_chains : !a.chain);
+        const bool has_d = absorbs && t.dia >= 0;
         const bool has_l = absorbs && !has_d && t.pan_l >= 0, has_u = absorbs && !has_d && t.pan_u >= 0;
         const DiagRec dr = const_load(a.diag + (has_d ? t.rec : 0));
         const DevTask pdl = const_load(a.tasks + (has_l ? t.pan_l : ti));
@@ -1068,8 +1069,8 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
             // barrier): the static chain's next task, else the after-link, else the
             // ring's head with its masks
             // (kernels without the inverses' copies run an lu's panels as after-links)
-            const int pl = !absorbs ? t.pan_l : -1;
-            const int pu = !absorbs ? t.pan_u : -1;
+            const int pl = !absorbs && t.dia < 0 ? t.pan_l : -1;
+            const int pu = !absorbs && t.dia < 0 ? t.pan_u : -1;
             if (nxt >= 0) {
                 s_next_ti = nxt;
                 s_next_mode = 1;
@@ -1079,7 +1080,6 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
             } else if (pl >= 0 || pu >= 0) {
                 s_next_ti = pl >= 0 ? pl : pu;
                 s_pend = pl >= 0 ? pu : -1;
-                s_pend_d = t.dia;
                 s_next_mode = 3;
             } else if (t.after >= 0) {
                 s_next_ti = t.after;
@@ -1087,10 +1087,6 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
             } else if (s_pend >= 0) {
                 s_next_ti = s_pend;
                 s_pend = -1;
-                s_next_mode = 3;
-            } else if (s_pend_d >= 0) {
-                s_next_ti = s_pend_d;
-                s_pend_d = -1;
                 s_next_mode = 3;
             } else if (s_ring_n > 0) {
                 const int h = s_ring_head;
@@ -1277,16 +1273,14 @@ void build_chains(Factor* f, HostGraph& hg) {
     std::vector<std::vector<int32_t>> cand(T);
     std::vector<int32_t> nchk(T, 0);
     std::vector<int32_t> order;
-    // after-links keep their chains in their heads' workgroups: neither end is claimed, nor the
-    // sum whose lu is one.  A workgroup runs what it has claimed when its chain ends, and with
-    // after-links no task of a chain waits for a later chain's; a diagonal chain's tasks wait
-    // for any earlier task, a claimed one included, so they claim none.
+    // after-links keep their chains in their heads' workgroups: neither end is claimed (diagonal
+    // chains do not run beside dynamic chaining)
     std::vector<char> linked(T, 0);
-    for (size_t t = 0; t < T; t++)
-        for (int32_t u : {f->tasks[t].after, f->tasks[t].pan_l, f->tasks[t].pan_u, f->tasks[t].dia})
+    for (size_t t = 0; t < T; t++) {
+        if (f->tasks[t].dia >= 0) continue;
+        for (int32_t u : {f->tasks[t].after, f->tasks[t].pan_l, f->tasks[t].pan_u})
             if (u >= 0) linked[(size_t)u] = linked[t] = 1;
-    for (size_t t = 0; t < T; t++)
-        if (f->tasks[t].next >= 0 && linked[(size_t)f->tasks[t].next]) linked[t] = 1;
+    }
     for (size_t u = 0; u < T; u++) {
         const DevTask& k = f->tasks[u];
         if (k.kind == TK_GEMM && k.b >= 1 && k.b <= CHAIN_MAX_PAIRS && !linked[u] &&
@@ -1304,7 +1298,7 @@ void build_chains(Factor* f, HostGraph& hg) {
         bool any = false;
         for (int l = 0; l < n; l++) {
             const int32_t p = slot_task[(size_t)sl[l]];
-            if (p < 0 || (f->n_diag_chains && linked[(size_t)p])) continue;
+            if (p < 0) continue;
             auto& cl = cand[(size_t)p];
             if (std::find(cl.begin(), cl.end(), u) != cl.end()) continue;
             if ((int)cl.size() >= CHAIN_MAX_CANDS || nchk[(size_t)p] + nent > CHAIN_MAX_CHECKS) continue;
@@ -2065,9 +2059,17 @@ int build_host_graph(Context* c, const sogl_factor_desc* d, Factor* f, HostGraph
         } else if (f->after_links || absorb) build_after_links(f, hg, chained, f->after_links, absorb, rank);
         else f->chain_head.clear();
         f->queue.clear();
+        f->queue_all.clear();
         for (size_t u = 0; u < f->tasks.size(); u++)
             if (!chained[u]) f->queue.push_back((int32_t)u);
         std::sort(f->queue.begin(), f->queue.end(), [&](int32_t x, int32_t y) { return rank[(size_t)x] < rank[(size_t)y]; });
+        if (f->n_diag_chains) {  // the queue of a run without the chains' links: all but the lus that follow their sum
+            std::vector<char> follows(f->tasks.size(), 0);
+            for (const DevTask& k : f->tasks)
+                if (k.next >= 0) follows[(size_t)k.next] = 1;
+            for (size_t u = 0; u < f->tasks.size(); u++)
+                if (!follows[u]) f->queue_all.push_back((int32_t)u);
+        }
     }
     build_chains(f, hg);
 
@@ -2247,6 +2249,15 @@ int validate_graph(Context* c, const sogl_factor_desc* d, const Factor* f, const
                 pred[(size_t)p] = (int32_t)t;
             }
         }
+        if (f->n_diag_chains) {  // the queue without the chains' links: every task but a static link's end, in index order
+            size_t i = 0;
+            for (size_t t = 0; t < T; t++) {
+                const bool follows = pred[t] >= 0 && f->tasks[(size_t)pred[t]].next == (int32_t)t;
+                if (!follows && (i >= f->queue_all.size() || f->queue_all[i++] != (int32_t)t))
+                    return bad("queue without chains at task " + std::to_string(t));
+            }
+            if (i != f->queue_all.size()) return bad("queue without chains");
+        }
         int32_t chains = 0;  // diagonal chains: the lu's panels, then their product and its lu
         for (size_t t = 0; t < T; t++) {
             const DevTask& k = f->tasks[t];
@@ -2288,8 +2299,6 @@ int validate_graph(Context* c, const sogl_factor_desc* d, const Factor* f, const
                     if (p > pred[t] && !(l.dia == (int32_t)t && (p == l.pan_l || p == l.pan_u)))
                         return bad("task " + std::to_string(t) + " of a diagonal chain waits for a later task");
                 }
-                if (k.chk_count || l.chk_count)
-                    return bad("task " + std::to_string(t) + " of a diagonal chain claims others");
                 if (in_chain.insert(head[t]).second && ++chains > DIAG_CHAINS) return bad("too many diagonal chains");
                 continue;
             }
@@ -2320,8 +2329,6 @@ int validate_graph(Context* c, const sogl_factor_desc* d, const Factor* f, const
             if (u.kind != TK_GEMM || u.b < 1 || u.b > CHAIN_MAX_PAIRS || (e.pos < 4 && e.pos >= 2 * u.b) ||
                 (e.pos == 4 && u.add < 0))
                 return bad("chain candidate " + std::to_string(e.task));
-            if (u.next >= 0 && f->tasks[(size_t)u.next].dia >= 0)
-                return bad("claimed task " + std::to_string(e.task) + " begins a diagonal chain");
             const Pair& pr = hg.pairs[(size_t)(u.a + (e.pos < 4 ? e.pos / 2 : 0))];
             const int32_t operand = e.pos == 4 ? u.add : ((e.pos & 1) ? pair_b(pr) : pair_a(pr));
             const bool own = operand == k.out0 || operand == k.out1 || operand == k.out2 || operand == k.out3;
@@ -2803,6 +2810,7 @@ int upload_graph(Context* c, const sogl_factor_desc* d, const InputCells* cells,
     add(f->u_rowptr, hg.up), add(f->u_col, hg.uc), add(f->u_slot, hg.us);
     add(f->l_diag_d, f->l_diag), add(f->u_diag_d, f->u_diag), add(f->linv_d, f->linv_slot), add(f->uinv_d, f->uinv_slot);
     add(f->pairx_d, hg.pair_x), add(f->pairy_d, hg.pair_y), add(f->inputs_d, f->input_slots), add(f->war_d, f->war);
+    add(f->queue_all_d, f->queue_all);
     add(f->lstep_ptr, ls.ptr), add(f->lstep_col, ls.col), add(f->lstep_slot, ls.slot);
     add(f->ustep_ptr, us.ptr), add(f->ustep_col, us.col), add(f->ustep_slot, us.slot);
     // (one record more: a kernel reads record 0 where a task has none, and one ahead)
@@ -3020,12 +3028,18 @@ int launch_factor(Context* c, Factor* f, int mode, int chunk, int wg_per_cu) {
         HIP_TRY(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, NT, 0));
         if (per_cu < 1) per_cu = 1;
         if (wg_per_cu > 0) per_cu = std::min(per_cu, wg_per_cu);  // never more than fit: all must be resident
-        int grid = std::max(1, std::min<int>(a.nqueue, c->num_cu * per_cu));
-        if (f->n_diag_chains) {  // see build_diag_chains; a chunk's entry behind a chain would wait for it
-            a.chunk = 1;
-            if (grid < a.nqueue && grid <= f->n_diag_chains)
-                return set_error(c, SOGL_ERR_UNSUPPORTED, "factor: fewer workgroups than diagonal chains");
+        // Diagonal chains run in the kernel that keeps their steps in LDS, with a workgroup more
+        // than there are chains (build_diag_chains), one queue entry at a time (a chunk's entry
+        // behind a chain would wait for it) and without dynamic chaining.  Otherwise their tasks
+        // come from the queue like any other: with the steps as after-links the two-per-CU kernel
+        // took 67.3 ms for 3D 48^3 FP64, 51.4 so; 2D 64^2 FP64 2.17 / 1.63, FP32 1.48 / 1.07.
+        const int room = c->num_cu * per_cu;
+        a.diag_chains = f->n_diag_chains > 0 && one && a.chunk == 1 && !a.chain && room > f->n_diag_chains;
+        if (f->n_diag_chains && !a.diag_chains) {
+            a.queue = (const int32_t*)f->queue_all_d.p;
+            a.nqueue = (int32_t)f->queue_all.size();
         }
+        const int grid = std::max(1, std::min<int>(a.nqueue, room));
         if (a.nqueue > 0) hipLaunchKernelGGL(kern, dim3(grid), dim3(NT), 0, st, a);
     } else if (mode == SOGL_EXEC_LEVELS) {
         launch_levels();
@@ -3388,9 +3402,10 @@ int run_factor(Context* c, Factor* f, int mode, int chunk, int wg_per_cu) {
 struct TuneCand {
     int mode, chunk, wg_per_cu;
 };
+constexpr int FULL = 1 << 10;  // workgroups per CU: more than ever fit
 constexpr TuneCand kTune[SOGL_TUNE_CANDIDATES] = {
-    {SOGL_EXEC_PERSISTENT, 1, 0}, {SOGL_EXEC_PERSISTENT, 2, 0}, {SOGL_EXEC_PERSISTENT, 4, 0},
-    {SOGL_EXEC_PERSISTENT, 1, 1}, {SOGL_EXEC_LEVELS, 1, 0},     {SOGL_EXEC_GRAPH, 1, 0},
+    {SOGL_EXEC_PERSISTENT, 1, FULL}, {SOGL_EXEC_PERSISTENT, 2, FULL}, {SOGL_EXEC_PERSISTENT, 4, FULL},
+    {SOGL_EXEC_PERSISTENT, 1, 1},    {SOGL_EXEC_LEVELS, 1, 0},        {SOGL_EXEC_GRAPH, 1, 0},
 };
 
 int autotune(Context* c, Factor* f, int trials, double* times_ms) {

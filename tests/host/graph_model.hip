@@ -43,17 +43,19 @@ int build(const sogl_factor_desc* desc, const int32_t* in_bi, const int32_t* in_
 struct Model {
     Factor& f;
     HostGraph& hg;
-    bool one;    // the kernels built for one workgroup per CU: a chain's step inside its lu
-    int claims;  // dynamic chaining
+    bool chains;  // a diagonal chain's step inside its lu; else its tasks come from the queue
+    int claims;   // dynamic chaining
+    const std::vector<int32_t>& queue;
     std::vector<int32_t> maker;
     std::vector<char> done, claimed;
     size_t taken = 0, finished = 0;
     struct Wg {
-        int32_t t = -1, mode = 0, pend = -1, pend_d = -1;
+        int32_t t = -1, mode = 0, pend = -1;
         std::deque<int32_t> ring;
     };
 
-    Model(Graph& g, bool one_, int claims_) : f(g.f), hg(g.hg), one(one_), claims(claims_) {
+    Model(Graph& g, bool chains_, int claims_)
+        : f(g.f), hg(g.hg), chains(chains_), claims(claims_), queue(chains || !f.n_diag_chains ? f.queue : f.queue_all) {
         maker.assign((size_t)f.n_slots, -1);
         for (size_t t = 0; t < f.tasks.size(); t++)
             for (int32_t o : {f.tasks[t].out0, f.tasks[t].out1, f.tasks[t].out2, f.tasks[t].out3})
@@ -77,8 +79,8 @@ struct Model {
     // One turn of a workgroup; false: it waits (or the queue is empty).
     bool turn(Wg& w) {
         if (w.t < 0) {
-            if (taken >= f.queue.size()) return false;
-            w.t = f.queue[taken++];
+            if (taken >= queue.size()) return false;
+            w.t = queue[taken++];
             w.mode = 0;
             if (claimed[(size_t)w.t]) w.t = -1;
             return true;
@@ -86,8 +88,7 @@ struct Model {
         const DevTask& k = f.tasks[(size_t)w.t];
         if (claimed[(size_t)w.t] && w.mode == 0) return w.t = -1, true;  // dropped
         if (w.mode != 1 && !ready(w.t)) return false;
-        const bool step = one && !claims && k.dia >= 0;
-        if (step) {  // the lu waits for what its panels and the update read as well
+        if (chains && k.dia >= 0) {  // the lu waits for what its panels and the update read as well
             const DevTask& d = f.tasks[(size_t)k.dia];
             for (int32_t p : {k.pan_l, k.pan_u})
                 if (p >= 0 && !ready(p, w.t)) return false;
@@ -109,12 +110,10 @@ struct Model {
             }
         auto go = [&](int32_t t, int mode) { w.t = t, w.mode = mode; };
         if (k.next >= 0) go(k.next, 1);
-        else if (k.pan_l >= 0 || k.pan_u >= 0) {
+        else if (k.dia < 0 && (k.pan_l >= 0 || k.pan_u >= 0)) {
             go(k.pan_l >= 0 ? k.pan_l : k.pan_u, 3);
             w.pend = k.pan_l >= 0 ? k.pan_u : -1;
-            w.pend_d = k.dia;
         } else if (w.pend >= 0) go(w.pend, 3), w.pend = -1;
-        else if (w.pend_d >= 0) go(w.pend_d, 3), w.pend_d = -1;
         else if (!w.ring.empty()) go(w.ring.front(), 2), w.ring.pop_front();
         else w.t = -1;
         return true;
@@ -132,28 +131,20 @@ struct Model {
 
 }  // namespace
 
-// out: tasks, those that `workgroups` workgroups finish, diagonal chains' steps, chains, tasks of
-// theirs that can claim others
-extern "C" int model(const sogl_factor_desc* desc, const int32_t* in_bi, const int32_t* in_bj, int workgroups, int one,
+// out: tasks, those that `workgroups` workgroups finish, diagonal chains' steps, chains
+extern "C" int model(const sogl_factor_desc* desc, const int32_t* in_bi, const int32_t* in_bj, int workgroups, int chains,
                      int claims, int64_t* out) {
     Graph g;
     int rc = build(desc, in_bi, in_bj, g);
     if (rc == SOGL_OK) rc = validate_graph(nullptr, &g.d, &g.f, g.hg);
     if (rc) return rc;
-    int64_t steps = 0, claimers = 0;
-    for (const DevTask& k : g.f.tasks) {
-        if (k.dia < 0) continue;
-        steps++;
-        claimers += k.chk_count > 0;
-        for (int32_t p : {k.pan_l, k.pan_u, k.dia})
-            if (p >= 0) claimers += g.f.tasks[(size_t)p].chk_count > 0;
-    }
-    Model m(g, one != 0, claims);
+    int64_t steps = 0;
+    for (const DevTask& k : g.f.tasks) steps += k.dia >= 0;
+    Model m(g, chains != 0, claims);
     out[0] = (int64_t)g.f.tasks.size();
     out[1] = (int64_t)m.run(workgroups);
     out[2] = steps;
     out[3] = g.f.n_diag_chains;
-    out[4] = claimers;
     return SOGL_OK;
 }
 

@@ -1,7 +1,7 @@
 """The order in which the persistent executor's workgroups can run a task graph with diagonal chains, on
 the CPU: host/graph_model.hip builds the graph with the executor's own code and plays the queue without
-times.  Every number of workgroups above the number of chains has to finish every task, with the chain's
-steps inside its lu (one workgroup per CU), after it (two), and with dynamic chaining."""
+times.  Every number of workgroups above the number of chains has to finish every task with the chains'
+steps inside their lus, and any number without (two workgroups per CU, dynamic chaining)."""
 import ctypes as C
 
 import numpy as np
@@ -73,11 +73,11 @@ def describe(n, pairs, symmetric, precision):
     return d, (keep, bi, bj), bi.ctypes.data_as(C.c_void_p), bj.ctypes.data_as(C.c_void_p)
 
 
-def play(lib, desc, workgroups, one, claims):
+def play(lib, desc, workgroups, chains, claims):
     d, _, bi, bj = desc
-    out = np.zeros(5, np.int64)
-    assert lib.model(C.byref(d), bi, bj, workgroups, one, claims, out.ctypes.data_as(C.c_void_p)) == sogl.OK
-    return dict(zip(("tasks", "finished", "steps", "chains", "claimers"), (int(v) for v in out)))
+    out = np.zeros(4, np.int64)
+    assert lib.model(C.byref(d), bi, bj, workgroups, chains, claims, out.ctypes.data_as(C.c_void_p)) == sogl.OK
+    return dict(zip(("tasks", "finished", "steps", "chains"), (int(v) for v in out)))
 
 
 PATTERNS = {
@@ -90,12 +90,12 @@ PATTERNS = {
 
 @pytest.mark.parametrize("symmetric", [False, True])
 @pytest.mark.parametrize("name", sorted(PATTERNS))
-@pytest.mark.parametrize("one,claims", [(1, 0), (0, 0), (1, 4), (0, 4)])
-def test_every_task_finishes(lib, name, symmetric, one, claims):
+@pytest.mark.parametrize("chains,claims", [(1, 0), (0, 0), (0, 4)])
+def test_every_task_finishes(lib, name, symmetric, chains, claims):
     desc = describe(*PATTERNS[name](), symmetric, sogl.FP64)
-    chains = play(lib, desc, 64, one, claims)["chains"]
-    for workgroups in range(chains + 1, chains + 8):
-        r = play(lib, desc, workgroups, one, claims)
+    least = play(lib, desc, 64, chains, claims)["chains"] if chains else 0
+    for workgroups in range(least + 1, least + 8):
+        r = play(lib, desc, workgroups, chains, claims)
         assert r["finished"] == r["tasks"], (workgroups, r)
 
 
@@ -202,11 +202,10 @@ def claims_before_a_chain():
 
 @pytest.mark.parametrize("make", [claims_inside_a_chain, claims_before_a_chain])
 def test_claims_beside_a_chain(lib, make):
-    """Dynamic chaining: a workgroup runs the tasks it has claimed when its chain ends, so a workgroup on a
-    diagonal chain may hold none."""
+    """Dynamic chaining: a workgroup runs the tasks it has claimed when its chain ends, so it runs no diagonal
+    chain (one that waits for a task it holds never ends)."""
     desc = make()
-    for claims in (0, 1, 8):
-        for workgroups in (2, 3, 8):
-            r = play(lib, desc, workgroups, 0, claims)
+    for workgroups in (2, 3, 8):
+        for claims in (0, 1, 8):
+            r = play(lib, desc, workgroups, int(claims == 0), claims)
             assert r["steps"] > 0 and r["finished"] == r["tasks"], (claims, workgroups, r)
-    assert r["claimers"] == 0
