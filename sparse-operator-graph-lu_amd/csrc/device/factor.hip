@@ -3015,12 +3015,14 @@ int launch_factor(Context* c, Factor* f, int mode, int chunk, int wg_per_cu) {
         a.queue = (const int32_t*)f->queue_d.p;
         a.nqueue = (int32_t)f->queue.size();
         // one workgroup per CU: the kernel built for that occupancy.  Where none is asked for,
-        // it takes the graphs of fewer than NARROW tasks per dependency level, whose time is
-        // the latency of the chain through the diagonal: its tasks are 10 to 30% shorter
-        // there (a CU of its own, twice the registers).  Factor ms, two per CU / one:
-        // 14 to 33 tasks per level: C2 FP64 56.7 / 51.3, symmetric 3D 37^3 FP64 25.9 / 21.8,
-        // 2D 64^2 FP64 1.93 / 1.68; 358: C3 FP32 35.7 / 39.5, FP64 61.2 / 75.5.
-        constexpr size_t NARROW = 64;
+        // it takes the graphs of few tasks per dependency level, whose time is the latency of the
+        // chain through the diagonal: its tasks are shorter there (a CU of its own, twice the
+        // registers) and it runs diagonal chains.  Factor ms, one per CU / two, by tasks per
+        // level: FP64 2 (2D 64^2) 1.62 / 1.60, 16 (symmetric 3D 37^3) 18.2 / 23.4, 33 (3D 48^3)
+        // 50.4 / 51.0, 54 (random band, n = 4,099) 2.44 / 2.25, 82 (6,000) 5.19 / 4.27, 358
+        // (16,384) 74.9 / 56.4; FP32 33 28.4 / 33.3, 54 1.38 / 1.50, 82 2.94 / 2.78, 358 40.4 /
+        // 34.0; bf16, which has no chains, 33 28.3 / 29.7, 54 1.34 / 1.29, 82 2.92 / 2.59.
+        constexpr size_t NARROW = sizeof(T) == 4 && !BF16 ? 64 : 48;
         const bool one = wg_per_cu == 1 || (wg_per_cu == 0 && f->tasks.size() < NARROW * (f->level_begin.size() - 1));
         auto kern = one ? k_factor_persistent<T, BF16, LLT, MASKS, true, COH>
                         : k_factor_persistent<T, BF16, LLT, MASKS, false, COH>;
