@@ -232,12 +232,13 @@ int sogl_ctx_set_task_links(sogl_ctx* ctx, int32_t links);
  * each) that make the solve's two-row blocks: per pair of block rows 2p, 2p+1, two for
  * the L block when L_2p+1,2p is present and two for the U block when U_2p,2p+1 is, and
  * the after-links and the absorbed panels (see sogl_ctx_set_task_links), which the check
- * builds whatever the context's setting. */
+ * builds whatever the context's setting.  The _plan form takes the counts from the plan's
+ * own op list and checks the list it is factored by (sogl_tile_order_ops) as well. */
 int sogl_graph_check(const sogl_factor_desc* desc, int64_t* info);
 int sogl_graph_check_plan(const sogl_plan* plan, int32_t precision, int64_t* info);
 /* sogl_factor_load from a host plan.  The factorisation is the plan's, tile for tile, in
  * tile-column order (sogl_tile_order_ops) where the plan allows it, else by the plan's own
- * op list; sogl_graph_check_plan looks at the latter. */
+ * op list. */
 int sogl_factor_load_plan(sogl_ctx* ctx, const sogl_plan* plan, int32_t precision,
                           int32_t* factor_id);
 /* The op list sogl_factor_load_plan factors a plan by: for every block row the sum of its

@@ -3192,7 +3192,7 @@ extern "C" int sogl_factor_load(sogl_ctx* x, const sogl_factor_desc* d, int32_t*
 namespace {
 // cells: the inputs come as the plan's cells (they can be scattered again before each
 // run, so their slots may be taken over)
-int graph_check(const sogl_factor_desc* d, bool cells, int64_t* info) {
+int graph_check(const sogl_factor_desc* d, bool cells, int64_t* info, bool tile_order = false) {
     if (!d || d->n_ids <= 0 || d->n_ops < 0 || d->n_inputs < 0 || d->block_rows <= 0 ||
         (d->n_ops && !d->ops) || (d->n_inputs && !d->input_ids))
         return set_error(nullptr, SOGL_ERR_ARG, "bad factor description");
@@ -3200,6 +3200,7 @@ int graph_check(const sogl_factor_desc* d, bool cells, int64_t* info) {
     f.precision = d->precision;
     f.elem = d->precision == SOGL_FP64 ? 8 : 4;
     f.n_inputs = d->n_inputs;
+    f.tile_order = tile_order;
     f.after_links = true;  // checked with the after-links and absorbed panels (head order included)
     f.absorb_panels = true;
     HostGraph hg;
@@ -3230,6 +3231,7 @@ int graph_check(const sogl_factor_desc* d, bool cells, int64_t* info) {
     g.precision = f.precision;
     g.elem = f.elem;
     g.n_inputs = f.n_inputs;
+    g.tile_order = tile_order;
     g.absorb_panels = true;
     HostGraph hd;
     rc = build_host_graph(nullptr, d, &g, hd);
@@ -3244,10 +3246,34 @@ int graph_check(const sogl_factor_desc* d, bool cells, int64_t* info) {
 
 extern "C" int sogl_graph_check(const sogl_factor_desc* d, int64_t* info) { return graph_check(d, false, info); }
 
+namespace {
+// the factorisation the plan describes, in tile-column order (tile_order.h)
+bool plan_tile_order(const sogl_plan* plan, const sogl_factor_desc* d, TileOrderOps& to) {
+    sogl::PlanView pv;
+    try {
+        return sogl::plan_view(plan, &pv) && tile_order_ops(d, pv.in_bi, pv.in_bj, to);
+    } catch (const std::bad_alloc&) {  // no host memory for a second list: the plan's own
+        return false;
+    }
+}
+// its description with that list, which `to` holds
+void use_tile_order(const TileOrderOps& to, sogl_factor_desc* d) {
+    d->ops = to.ops.data();
+    d->n_ops = (int64_t)to.ops.size();
+    d->n_ids = to.n_ids;
+}
+}  // namespace
+
 extern "C" int sogl_graph_check_plan(const sogl_plan* plan, int32_t precision, int64_t* info) {
     sogl_factor_desc d;
     if (!sogl::plan_factor_desc(plan, precision, &d)) return set_error(nullptr, SOGL_ERR_ARG, "null plan");
-    return graph_check(&d, true, info);
+    int rc = graph_check(&d, true, info);
+    TileOrderOps to;
+    if (rc == SOGL_OK && plan_tile_order(plan, &d, to)) {  // and the graph that is run
+        use_tile_order(to, &d);
+        rc = graph_check(&d, true, nullptr, true);
+    }
+    return rc;
 }
 
 extern "C" int sogl_ctx_set_task_links(sogl_ctx* x, int32_t links) {
@@ -3267,18 +3293,6 @@ extern "C" int sogl_ctx_set_pool_reuse(sogl_ctx* x, int32_t mode) {
     x->c.pool_reuse = mode;
     return SOGL_OK;
 }
-
-namespace {
-// the factorisation the plan describes, in tile-column order (tile_order.h)
-bool plan_tile_order(const sogl_plan* plan, const sogl_factor_desc* d, TileOrderOps& to) {
-    sogl::PlanView pv;
-    try {
-        return sogl::plan_view(plan, &pv) && tile_order_ops(d, pv.in_bi, pv.in_bj, to);
-    } catch (const std::bad_alloc&) {  // no host memory for a second list: the plan's own
-        return false;
-    }
-}
-}  // namespace
 
 extern "C" int sogl_tile_order_ops(const sogl_plan* plan, sogl_op* ops, int64_t* n_ops, int32_t* n_ids) {
     sogl_factor_desc d;
@@ -3305,11 +3319,7 @@ extern "C" int sogl_factor_load_plan(sogl_ctx* x, const sogl_plan* plan, int32_t
         return set_error(x ? &x->c : nullptr, SOGL_ERR_ARG, "null plan");
     TileOrderOps to;
     const bool tile_order = plan_tile_order(plan, &d, to);
-    if (tile_order) {
-        d.ops = to.ops.data();
-        d.n_ops = (int64_t)to.ops.size();
-        d.n_ids = to.n_ids;
-    }
+    if (tile_order) use_tile_order(to, &d);
     return load_factor(x, &d, &cells, factor_id, tile_order);
 }
 

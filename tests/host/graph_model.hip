@@ -1,16 +1,10 @@
 // Host-only build of the executor's graph code (no device code, no GPU) with an untimed model of
 // the persistent kernels' queue: which tasks a given number of workgroups can finish.
 #include "../../sparse-operator-graph-lu_amd/csrc/device/factor.hip"
+#include "no_device.h"
 
 using namespace sogl_dev;
 
-// The HIP fat binary and its registration: nothing is launched here.
-extern "C" {
-const char __hip_fatbin[8] = {0};
-void** __hipRegisterFatBinary(const void*) { static void* h; return &h; }
-void __hipRegisterFunction(void**, const void*, char*, const char*, unsigned, void*, void*, void*, void*, int*) {}
-void __hipUnregisterFatBinary(void**) {}
-}
 namespace sogl_dev {
 void noalloc_scratch_init(int) {}
 }

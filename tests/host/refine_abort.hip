@@ -6,15 +6,11 @@
 #include "../../sparse-operator-graph-lu_amd/csrc/device/solve.hip"
 #undef HIP_TRY
 #include "../../sparse-operator-graph-lu_amd/csrc/device/refine.hip"
+#include "no_device.h"
 
 static int abort_at = 0, solves = 0;
 
 extern "C" {
-const char __hip_fatbin[8] = {0};
-void** __hipRegisterFatBinary(const void*) { static void* h; return &h; }
-void __hipRegisterFunction(void**, const void*, char*, const char*, unsigned, void*, void*, void*, void*, int*) {}
-void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
-void __hipUnregisterFatBinary(void**) {}
 hipError_t hipMalloc(void** p, size_t bytes) {
     *p = malloc(bytes);
     return hipSuccess;
