@@ -22,11 +22,12 @@
 
 namespace sogl_dev {
 
-// Updates per partial sum.  A GEMM task holds its workgroup while it waits for its last
+// Block columns per partial sum.  A GEMM task holds its workgroup while it waits for its last
 // update, and one that starts late multiplies all of them on the spot: parts bound that
-// work, and are made, as tasks of their own, as soon as their operands are.  The parts of
-// the tiles of a block row end at different columns (i + k + j), so that they do not all
-// become ready at once.  Measured: C3 FP32 (sums of up to 255) 48.8 ms whole, 37.3 in
+// work, and are made, as tasks of their own, as soon as their operands are.  A part of tile
+// (i, k) begins where i + k + j is a multiple of SUM_PAIRS (an update by that column j there
+// is), so that the parts of a block row's tiles do not all become ready at once: a dense sum
+// has parts of SUM_PAIRS updates, a sparse one more or fewer in each.  Measured: C3 FP32 (sums of up to 255) 48.8 ms whole, 37.3 in
 // parts of 64, 38.3 of 32, 45.4 of 16; C2 FP32 (up to 27) 39.2, 39.2, 37.8, 35.4.
 constexpr int32_t SUM_PAIRS = 32;
 
@@ -103,7 +104,8 @@ inline bool tile_order_ops(const sogl_factor_desc* d, const int32_t* in_bi, cons
         out.ops.push_back(sogl_op{src, src2, code, res, res2, stage, seq++, 0});
     };
     // S_ik: the input tile (i, k) less its updates by block columns before min(i, k); 0: none
-    // (products at stage st, part p's sum at st + 1 + p)
+    // (products at stage st, part p's sum at st + 1 + p; most: the parts of the longest sum so far)
+    int32_t most = 0;
     auto sum = [&](int32_t i, int32_t k, int32_t st) {
         int32_t a = 0;
         const auto& ar = arow[(size_t)i];
@@ -138,26 +140,34 @@ inline bool tile_order_ops(const sogl_factor_desc* d, const int32_t* in_bi, cons
             }
         }
         if (acc) close();
+        most = std::max(most, part);
         return a;
+    };
+    // an op that follows the sums of its step: its stage, counted from the end of theirs, is made
+    // absolute when the step's sums are all there
+    std::vector<size_t> after;
+    auto emit_after = [&](int32_t code, int32_t src, int32_t src2, int32_t res, int32_t res2, int32_t stage) {
+        after.push_back(out.ops.size());
+        emit(code, src, src2, res, res2, stage);
     };
     int32_t stage = 1;
     for (int32_t k = 0; k < R; k++) {
         const auto& lc = lcol[(size_t)k];
         const auto& ur = urow[(size_t)k];
         std::vector<int32_t> s_l(lc.size(), -1), s_u(ur.size(), -1);
-        // at most size / SUM_PAIRS + 3 parts in any sum of this step
-        const int32_t done = stage + (int32_t)(std::max(lrow[(size_t)k].size(), ucol[(size_t)k].size()) / SUM_PAIRS) + 4;
+        most = 0;
+        after.clear();
         const int32_t x = next++, z = llt ? 0 : next++;
         bool ok = true;
         auto panel_l = [&](size_t q) {
             if (s_l[q] < 0) s_l[q] = sum(lc[q].first, k, stage);
             ok &= s_l[q] != 0;  // else: a listed tile that nothing fills
-            emit(llt ? SOGL_OP_MULT : SOGL_OP_MUL, s_l[q], llt ? x : z, lc[q].second, 0, done + 2);
+            emit_after(llt ? SOGL_OP_MULT : SOGL_OP_MUL, s_l[q], llt ? x : z, lc[q].second, 0, 2);
         };
         auto panel_u = [&](size_t q) {
             if (s_u[q] < 0) s_u[q] = sum(k, ur[q].first, stage);
             ok &= s_u[q] != 0;
-            emit(SOGL_OP_MUL, x, s_u[q], ur[q].second, 0, done + 2);
+            emit_after(SOGL_OP_MUL, x, s_u[q], ur[q].second, 0, 2);
         };
         // the sums of the two panels next to the diagonal come before the diagonal's own:
         // the lu that runs those panels itself then finds them handed out earlier
@@ -165,15 +175,17 @@ inline bool tile_order_ops(const sogl_factor_desc* d, const int32_t* in_bi, cons
         if (!ur.empty() && ur[0].first == k + 1) s_u[0] = sum(k, k + 1, stage);
         const int32_t s = sum(k, k, stage);
         if (!s) return false;
-        emit(llt ? SOGL_OP_LLT : SOGL_OP_LU, s, 0, ldiag[(size_t)k], llt ? 0 : udiag[(size_t)k], done);
-        emit(SOGL_OP_LOWER_INV, ldiag[(size_t)k], 0, x, 0, done + 1);
-        if (!llt) emit(SOGL_OP_UPPER_INV, udiag[(size_t)k], 0, z, 0, done + 1);
+        emit_after(llt ? SOGL_OP_LLT : SOGL_OP_LU, s, 0, ldiag[(size_t)k], llt ? 0 : udiag[(size_t)k], 0);
+        emit_after(SOGL_OP_LOWER_INV, ldiag[(size_t)k], 0, x, 0, 1);
+        if (!llt) emit_after(SOGL_OP_UPPER_INV, udiag[(size_t)k], 0, z, 0, 1);
         for (size_t q = 0; q < std::max(lc.size(), ur.size()); q++) {
             if (q < lc.size()) panel_l(q);
             if (q < ur.size()) panel_u(q);
         }
         if (!ok) return false;
-        stage = done + 3;
+        stage += most + 1;
+        for (size_t o : after) out.ops[o].stage += stage;
+        stage += 3;
     }
     int64_t inputs = 0;
     for (const auto& e : arow) inputs += (int64_t)e.size();

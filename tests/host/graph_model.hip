@@ -164,3 +164,11 @@ extern "C" int plant_late_sum(const sogl_factor_desc* desc, const int32_t* in_bi
     }
     return -1;
 }
+
+// The tile-column op list of a description (ops may be null): its length, -1 where there is none.
+extern "C" int64_t tile_ops(const sogl_factor_desc* desc, const int32_t* in_bi, const int32_t* in_bj, sogl_op* ops) {
+    TileOrderOps to;
+    if (!tile_order_ops(desc, in_bi, in_bj, to)) return -1;
+    if (ops) std::copy(to.ops.begin(), to.ops.end(), ops);
+    return (int64_t)to.ops.size();
+}

@@ -88,6 +88,29 @@ PATTERNS = {
 }
 
 
+# a row coupled to every 32nd: each of its diagonal's updates is a part of its own
+STAGED = dict(PATTERNS, band_40=lambda: band(90, 40), every_32nd=lambda: (641, [(640, 32 * q) for q in range(20)]),
+              every_32nd_beside_a_band=lambda: (200, band(200, 2)[1] + [(160, 32 * q) for q in range(5)]))
+
+
+@pytest.mark.parametrize("symmetric", [False, True])
+@pytest.mark.parametrize("name", sorted(STAGED))
+def test_stages_follow_their_operands(lib, name, symmetric):
+    """The tile-column list's stages are a schedule: an op comes after the ops that make what it reads, and
+    the products of one sum share a stage."""
+    d, _, bi, bj = describe(*STAGED[name](), symmetric, sogl.FP64)
+    lib.tile_ops.restype = C.c_int64
+    ops = np.zeros((lib.tile_ops(C.byref(d), bi, bj, None), 8), np.int32)
+    lib.tile_ops(C.byref(d), bi, bj, ops.ctypes.data_as(C.c_void_p))
+    made = {}
+    for src, src2, _, res, res2, stage, _, _ in ops.tolist():
+        for r in (res, res2):
+            if r:
+                assert made.setdefault(r, stage) == stage
+    for src, src2, _, res, _, stage, _, _ in ops.tolist():
+        assert all(stage > made.get(a, 0) for a in (src, src2) if a), (src, src2, res, stage)
+
+
 @pytest.mark.parametrize("symmetric", [False, True])
 @pytest.mark.parametrize("name", sorted(PATTERNS))
 @pytest.mark.parametrize("chains,claims", [(1, 0), (0, 0), (0, 4)])
