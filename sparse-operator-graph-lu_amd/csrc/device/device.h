@@ -164,6 +164,7 @@ struct Factor {
     // the same by pairs of block rows and of block columns (pair_steps)
     DevBuf lstep_ptr, lstep_col, lstep_slot, ustep_ptr, ustep_col, ustep_slot;
     int64_t solve_entries = 0;  // off-diagonal tiles of L and U
+    int64_t solve_rows = 0;     // block rows that have some
     DevBuf pairx_d, pairy_d;  // per row pair: slot of X_p / Y_p (the two-row solve steps), -1: zero
     DevBuf solve_ctrl, vec_b, vec_x, vec_y;
     size_t vec_cap = 0;  // doubles per vector buffer

@@ -2736,6 +2736,14 @@ PairSteps pair_steps(const std::vector<int32_t>& rp, const std::vector<int32_t>&
     return s;
 }
 
+// The triangular solve's off-diagonal tiles, and the block rows that have one.
+void count_solve_tiles(Factor* f, const HostGraph& hg) {
+    f->solve_entries = (int64_t)hg.lc.size() + (int64_t)hg.uc.size();
+    f->solve_rows = 0;
+    for (int32_t i = 0; i < f->block_rows; i++)
+        f->solve_rows += hg.lp[(size_t)i + 1] > hg.lp[(size_t)i] || hg.up[(size_t)i + 1] > hg.up[(size_t)i];
+}
+
 // The records of the diagonal chains' steps, in the order of their lus, after the slots are
 // assigned.
 void make_diag_records(Factor* f, const HostGraph& hg) {
@@ -2797,7 +2805,7 @@ int upload_graph(Context* c, const sogl_factor_desc* d, const InputCells* cells,
         HIP_TRY(c, hipMemcpy(f->chk_d.p, f->chk.data(), f->chk.size() * sizeof(ChainChk), hipMemcpyHostToDevice));
     // the index arrays: parts of one allocation, filled by one copy (an allocation and a copy
     // each, they were a tenth of a small drop-in solve)
-    f->solve_entries = (int64_t)hg.lc.size() + (int64_t)hg.uc.size();
+    count_solve_tiles(f, hg);
     const PairSteps ls = pair_steps(hg.lp, hg.lc, hg.ls), us = pair_steps(hg.up, hg.uc, hg.us);
     struct Part {
         DevBuf* b;

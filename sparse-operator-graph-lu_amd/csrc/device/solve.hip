@@ -26,12 +26,14 @@ namespace sogl_dev {
 
 constexpr long long SOLVE_SPIN_LIMIT = 20LL * 100 * 1000 * 1000;
 constexpr int TRSM_MIN_RHS = 16;   // from this many right-hand sides the block-row sums run on MFMA
-// FP64 solves of 1-15 columns: off-diagonal tiles per block row, over L and U, less the share
-// of zero blocks, from which the kernel that loads a whole step ahead (KEEP) is taken (where
-// most of the tiles are skipped, 2D convection-diffusion 1000^2, it takes 22.7 ms for 19.0).  A solve without / with it: 1.1 tiles
-// a row (2D 64^2) 0.103 / 0.116 ms, 1.9 (2D 128^2) 0.376 / 0.426; 3.6 (2D 253^2) 1.99 / 1.71,
-// 5.5 (2D 400^2) 7.8 / 5.1, 14 (3D 31^3) 1.83 / 1.41, 34 (3D 48^3) 8.1 / 7.0.
-constexpr int KEEP_ENTRIES = 2;
+// FP64 solves of 1-15 columns: off-diagonal tiles of L and U together per block row that has one
+// (padding rows have none), less the share of zero blocks, from which the kernel that loads a
+// whole step ahead (KEEP) is taken.  A solve of one column without / with it, ms, by that
+// number: 1.6 (2D 64^2) 0.093 / 0.112, 3.3 (2D convection-diffusion 300^2) 1.89 / 2.15, 4.2
+// (2D 200^2) 0.99 / 1.07, 4.6 (3D 16^3) 0.122 / 0.126, 4.75 (2D 230^2) 1.48 / 1.42, 5.4 (2D
+// 256^2) 2.21 / 1.78, 6.8 (3D 20^3) 0.308 / 0.234, 8.2 (2D 400^2) 7.78 / 5.08, 16 (3D 31^3)
+// 1.82 / 1.39.
+constexpr double KEEP_TILES = 4.7;
 constexpr int MAX_RHS = 1024;      // columns per launch: pairs x panels fit the 32-bit task counter
 
 struct SolveArgs {
@@ -679,6 +681,10 @@ namespace {
         if (_rc != SOGL_OK) return _rc;                          \
     } while (0)
 
+bool whole_steps_ahead(const Factor* f) {
+    return (1 - f->zero_blocks) * (double)f->solve_entries >= KEEP_TILES * (double)f->solve_rows;
+}
+
 template <typename T>
 int launch_pass(Context* c, Factor* f, const SolveWork& w, bool mfma, bool forward, const double* in, double* out,
                 int nrhs) {
@@ -703,8 +709,7 @@ int launch_pass(Context* c, Factor* f, const SolveWork& w, bool mfma, bool forwa
     const int64_t ntask = (int64_t)((a.nbr + 1) / 2) * (mfma ? (nrhs + PC - 1) / PC : nrhs);
     auto kern = mfma ? k_trsm_persistent<T> : k_trsv_persistent<T, false>;
     if constexpr (sizeof(T) == 8)
-        if (!mfma && (1 - f->zero_blocks) * (double)f->solve_entries >= KEEP_ENTRIES * 2.0 * a.nbr)
-            kern = k_trsv_persistent<T, true>;
+        if (!mfma && whole_steps_ahead(f)) kern = k_trsv_persistent<T, true>;
     int per_cu = 0;
     HIP_TRY(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, NTP, 0));
     if (per_cu < 1) per_cu = 1;

@@ -1,5 +1,5 @@
-// Host-only build of the solve's buffer handling (no device code, no GPU): device allocations come from
-// malloc, the n-th of them fails.
+// Host-only build of the solve's buffer handling and of its choice of kernel (no device code, no GPU):
+// device allocations come from malloc, the n-th of them fails.
 #include "../../sparse-operator-graph-lu_amd/csrc/device/factor.hip"
 #undef HIP_TRY
 #include "../../sparse-operator-graph-lu_amd/csrc/device/solve.hip"
@@ -37,4 +37,23 @@ extern "C" int grow_after_failure(int fail, int again) {
         sogl_dev::dev_free(*b);
     }
     return out;
+}
+
+// Whether an FP64 solve of a band of `rows` block rows, `half` of them to either side, then padding up to
+// `block_rows`, loads whole steps ahead.
+extern "C" int steps_ahead(int rows, int half, int block_rows, double zero_blocks) {
+    sogl_dev::Factor f;
+    sogl_dev::HostGraph hg;
+    f.block_rows = block_rows;
+    f.zero_blocks = zero_blocks;
+    hg.lp.assign(1, 0);
+    hg.up.assign(1, 0);
+    for (int i = 0; i < block_rows; i++) {
+        for (int j = std::max(0, i - half); i < rows && j < std::min(rows, i + half + 1); j++)
+            if (j != i) (j < i ? hg.lc : hg.uc).push_back(j);
+        hg.lp.push_back((int32_t)hg.lc.size());
+        hg.up.push_back((int32_t)hg.uc.size());
+    }
+    sogl_dev::count_solve_tiles(&f, hg);
+    return sogl_dev::whole_steps_ahead(&f);
 }
