@@ -74,6 +74,17 @@ EXECUTORS = {"auto": (sogl.EXEC_AUTO, 0), "persistent": (sogl.EXEC_PERSISTENT, 0
 EXTRA = {"sym": (lambda: W.symmetric_lower(W.diffusion_varcoef(48, 3, 23)), "sym_diffusion3d_48")}
 
 
+def run_ops(plan):
+    """(unit ops, products among them, stages) of the op list a plan is factored by: the
+    tile-column list, or the plan's own where it keeps that."""
+    got = sogl.tile_order_ops(plan)
+    if got is None:
+        i = plan.info
+        return int(i.n_ops), int(i.n_mul + i.n_mulneg + i.n_mult), int(i.n_stages)
+    ops = got[0]
+    return ops.shape[0], int(np.isin(ops[:, 2], (8, 9, 11)).sum()), int(ops[:, 5].max())
+
+
 def compare_executors(dev, plan, per_op: bool, reuse_mode: int):
     """FP64 factor time of every executor on one resident factor (ms, best of 2), the
     autotuner's choice, and the per-op executor (one launch per unit op) once (the
@@ -98,7 +109,7 @@ def compare_executors(dev, plan, per_op: bool, reuse_mode: int):
         dev.factor(fid, sogl.EXEC_PER_OP)
         out["per_op_ms"] = round(dev.stats(fid).exec_ms, 3)
         out["per_op_wall_s"] = round(time.perf_counter() - t0, 3)
-        out["per_op_launches"] = int(plan.info.n_ops)
+        out["per_op_launches"] = run_ops(plan)[0]
     dev.release(fid)
     return out
 
@@ -323,7 +334,8 @@ def main():
                      symmetric=prob.symmetric)
     t_plan = time.perf_counter() - t0
     info = plan.info
-    gemm_flops = (info.n_mul + info.n_mulneg + info.n_mult) * 2.0 * 64 ** 3
+    unit_ops, gemm_ops, stages = run_ops(plan)
+    gemm_flops = gemm_ops * 2.0 * 64 ** 3
     nrhs = 1 if prob.b.ndim == 1 else prob.b.shape[1]
     solve_bytes = {k: (info.n_l_tiles + info.n_u_tiles) * 64 * 64 * s + 2 * plan.N * 8 * nrhs
                    for k, s in (("fp64", 8), ("fp32", 4))}
@@ -361,7 +373,7 @@ def main():
         lu_same = run_path(dev, lu_plan, full, sogl.FP64, tol, 0, args.steps, args.warmup, *mode)
         lu_same.pop("x")
         lu_same = {k: (float(f"{v:.6g}") if isinstance(v, float) else v) for k, v in lu_same.items()}
-        lu_same["unit_ops"] = int(lu_plan.info.n_ops)
+        lu_same["unit_ops"] = run_ops(lu_plan)[0]
         del lu_plan
     dev.close()
 
@@ -448,8 +460,8 @@ def main():
         "data": "synthetic",
         "config": {"workload": f"{args.config}: {desc}", "tol": tol,
                    "executor": args.exec if head["executor"] is None else f"autotuned: {head['executor']}",
-                   "n": prob.n, "nnz": prob.nnz, "unit_ops": int(info.n_ops),
-                   "gemm_ops": int(info.n_mul + info.n_mulneg + info.n_mult), "stages": int(info.n_stages),
+                   "n": prob.n, "nnz": prob.nnz, "unit_ops": unit_ops,
+                   "gemm_ops": gemm_ops, "stages": stages,
                    "gemm_gflop": round(gemm_flops / 1e9, 3), "host_plan_s": round(t_plan, 3),
                    "task_links": args.task_links},
         "roofline": {"bound": "mfma", "achieved": round(head["gemm_tflops"], 4), "peak": PEAK["fp32"],
