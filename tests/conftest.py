@@ -16,6 +16,23 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "slow: larger workloads")
 
 
+# The integration tests build and run a harness from the reference's sources.  Where the reference
+# folder is empty or absent (__graft_entry__.build's own condition) and no harness was built where it
+# is not, there is nothing for them to test.
+REFERENCE = "/root/reference"
+HARNESS = os.path.join(ROOT, "oracle", "_ref", "ref_dump_gpu")
+
+
+def pytest_collection_modifyitems(items):
+    if os.path.isdir(REFERENCE) and os.listdir(REFERENCE):
+        return
+    for item in items:
+        if item.path.name != "test_integration.py":
+            continue
+        if "gpu" not in item.keywords or not os.path.exists(HARNESS):
+            item.add_marker(pytest.mark.skip(reason="the reference's sources are absent, and with them the harness"))
+
+
 @pytest.fixture(scope="session")
 def golden():
     import numpy as np
