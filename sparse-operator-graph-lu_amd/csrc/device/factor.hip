@@ -179,7 +179,8 @@ struct Args {
     const ChainChk* chk;  // persistent executor: chain candidates' check entries
     int32_t chain;        // claims per finished task at most (0: no dynamic chaining)
     const DiagRec* diag;
-    int32_t diag_chains;  // persistent executor: run the diagonal chains' links (launch_factor)
+    int32_t pan_after;    // persistent executor: an lu that does not run its panels runs them as after-links
+    int32_t diag_chains;  // and a diagonal chain's lu runs its step (launch_factor)
     const int32_t* war;   // value ids whose readers a reused result slot waits for (DevTask)
 };
 
@@ -1069,8 +1070,8 @@ __global__ __launch_bounds__(NT, ONE ? 1 : 2) void k_factor_persistent(Args a) {
             // barrier): the static chain's next task, else the after-link, else the
             // ring's head with its masks
             // (kernels without the inverses' copies run an lu's panels as after-links)
-            const int pl = !absorbs && t.dia < 0 ? t.pan_l : -1;
-            const int pu = !absorbs && t.dia < 0 ? t.pan_u : -1;
+            const int pl = !absorbs && a.pan_after ? t.pan_l : -1;
+            const int pu = !absorbs && a.pan_after ? t.pan_u : -1;
             if (nxt >= 0) {
                 s_next_ti = nxt;
                 s_next_mode = 1;
@@ -1273,14 +1274,12 @@ void build_chains(Factor* f, HostGraph& hg) {
     std::vector<std::vector<int32_t>> cand(T);
     std::vector<int32_t> nchk(T, 0);
     std::vector<int32_t> order;
-    // after-links keep their chains in their heads' workgroups: neither end is claimed (diagonal
-    // chains do not run beside dynamic chaining)
+    // after-links keep their chains in their heads' workgroups: neither end is claimed (nor are
+    // diagonal chains' tasks, which come from the queue in a run with claims)
     std::vector<char> linked(T, 0);
-    for (size_t t = 0; t < T; t++) {
-        if (f->tasks[t].dia >= 0) continue;
-        for (int32_t u : {f->tasks[t].after, f->tasks[t].pan_l, f->tasks[t].pan_u})
+    for (size_t t = 0; t < T; t++)
+        for (int32_t u : {f->tasks[t].after, f->tasks[t].pan_l, f->tasks[t].pan_u, f->tasks[t].dia})
             if (u >= 0) linked[(size_t)u] = linked[t] = 1;
-    }
     for (size_t u = 0; u < T; u++) {
         const DevTask& k = f->tasks[u];
         if (k.kind == TK_GEMM && k.b >= 1 && k.b <= CHAIN_MAX_PAIRS && !linked[u] &&
@@ -1470,10 +1469,12 @@ void build_after_links(Factor* f, const HostGraph& hg, std::vector<char>& linked
     f->chain_head = head;
 }
 
-// Diagonal chains (FP32 and FP64 factors; L L^T ones with one panel, diag_step_llt).  Where the lu of block column k makes, through
-// its two panels next to the diagonal, the last update of the next diagonal tile
-// (S_{k+1,k+1} = P - L_{k+1,k} U_{k,k+1}, tile_order.h), its workgroup runs all three and the
-// next lu after them: the diagonal of a banded factor is one workgroup's work (diag_step).
+// Diagonal chains (FP32 and FP64 factors; L L^T ones with one panel, diag_step_llt).  Where the
+// lu of block column k makes, through its two panels next to the diagonal, the last update of the
+// next diagonal tile (S_{k+1,k+1} = P - L_{k+1,k} U_{k,k+1}, tile_order.h), its workgroup runs all
+// three and the next lu after them: the diagonal of a banded factor is one workgroup's work
+// (diag_step).  launch_factor says which runs take the chains; the others take every task but the
+// lus that follow their sum from queue_all.
 // Deadlock freedom: every wait in such a chain, and every other wait, is for a task of lower
 // index than the waiting one's, and the queue hands tasks out by index.  The dependency levels
 // give it for every task by itself; but the lu waits for what its panels and the update read
@@ -3045,6 +3046,7 @@ int launch_factor(Context* c, Factor* f, int mode, int chunk, int wg_per_cu) {
         // took 67.3 ms for 3D 48^3 FP64, 51.4 so; 2D 64^2 FP64 2.17 / 1.63, FP32 1.48 / 1.07.
         const int room = c->num_cu * per_cu;
         a.diag_chains = f->n_diag_chains > 0 && one && a.chunk == 1 && !a.chain && room > f->n_diag_chains;
+        a.pan_after = !f->n_diag_chains;  // (their other runs take the panels from the queue)
         if (f->n_diag_chains && !a.diag_chains) {
             a.queue = (const int32_t*)f->queue_all_d.p;
             a.nqueue = (int32_t)f->queue_all.size();
