@@ -368,7 +368,7 @@ int sogl_solve_refined(sogl_ctx* ctx, int32_t factor_id, const double* b, double
  * by the caller, e.g. with sogl_device_alloc): the permutation, padding, solves,
  * FP64 residuals and corrections all stay in HBM.  max_iter = 0 gives a plain
  * solve plus its residual.  d_x may be d_b; it keeps what it held where the call ends with
- * SOGL_ERR_TIMEOUT. */
+ * SOGL_ERR_TIMEOUT (for calls that may correct, where the device has room for a copy). */
 int sogl_solve_refined_device(sogl_ctx* ctx, int32_t factor_id, const double* d_b, double* d_x,
                               int32_t nrhs, double tol, int32_t max_iter, int32_t* iters,
                               double* resid);

@@ -350,9 +350,9 @@ extern "C" int sogl_solve_refined_device(sogl_ctx* x, int32_t factor_id, const d
     if (!f) return set_error(c, SOGL_ERR_ARG, "unknown factor id");
     if (!f->has_refine) return set_error(c, SOGL_ERR_ARG, "sogl_refine_attach was not called");
     HIP_TRY(c, hipSetDevice(c->device));
-    int rc;
-    if (max_iter > 0 && (rc = dev_alloc(c, f->vec_io, (size_t)f->n * nrhs * 8, "earlier x"))) return rc;
-    return refined_core(c, f, d_b, d_x, max_iter > 0 ? (double*)f->vec_io.p : nullptr, nrhs, tol, max_iter, iters, resid);
+    // (no room for what d_x holds is no reason to refuse the solve)
+    const bool old = max_iter > 0 && dev_alloc(c, f->vec_io, (size_t)f->n * nrhs * 8, "earlier x") == SOGL_OK;
+    return refined_core(c, f, d_b, d_x, old ? (double*)f->vec_io.p : nullptr, nrhs, tol, max_iter, iters, resid);
 }
 
 extern "C" int sogl_solve_refined(sogl_ctx* x, int32_t factor_id, const double* b, double* xo,

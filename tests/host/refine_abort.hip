@@ -9,9 +9,11 @@
 #include "no_device.h"
 
 static int abort_at = 0, solves = 0;
+static size_t refuse = 0;  // allocations of this many bytes fail
 
 extern "C" {
 hipError_t hipMalloc(void** p, size_t bytes) {
+    if (bytes == refuse) return hipErrorOutOfMemory;
     *p = malloc(bytes);
     return hipSuccess;
 }
@@ -65,8 +67,9 @@ hipError_t hipLaunchKernel(const void* k, dim3, dim3, void** a, size_t, hipStrea
 }
 
 // x after a refined solve of up to max_iter corrections into an x of -1 whose solve number `at` times out
-// (0: none); the return code in rc.
-extern "C" double x_after_abort(int at, int max_iter, int* rc) {
+// (0: none), without room for a copy of x (`full`); the return code in rc.
+extern "C" double x_after_abort(int at, int max_iter, int full, int* rc) {
+    refuse = full ? 100 * sizeof(double) : 0;
     sogl_ctx x;
     Factor f;
     f.block_rows = 2;

@@ -19,12 +19,14 @@ def lib(tmp_path_factory):
 @pytest.mark.parametrize("at,max_iter", [(1, 0), (1, 3), (2, 3), (4, 3)])
 def test_timeout_leaves_x(lib, at, max_iter):
     rc = C.c_int()
-    assert lib.x_after_abort(at, max_iter, C.byref(rc)) == -1.0
+    assert lib.x_after_abort(at, max_iter, 0, C.byref(rc)) == -1.0
     assert rc.value == TIMEOUT
 
 
+@pytest.mark.parametrize("full", [0, 1])
 @pytest.mark.parametrize("max_iter", [0, 3])
-def test_no_timeout_gives_the_last_iterate(lib, max_iter):
+def test_no_timeout_gives_the_last_iterate(lib, max_iter, full):
+    """(also where there is no room for the copy)"""
     rc = C.c_int()
-    assert lib.x_after_abort(0, max_iter, C.byref(rc)) == max_iter + 1
+    assert lib.x_after_abort(0, max_iter, full, C.byref(rc)) == max_iter + 1
     assert rc.value == NOT_CONVERGED
