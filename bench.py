@@ -297,8 +297,8 @@ def main():
                          "tile loads); 0: one slot per value; 2 (default): reuse when the values would "
                          "take over a quarter of the device's HBM")
     ap.add_argument("--task-links", type=int, default=sogl.LINK_PANEL, choices=(0, 1, 2, 3),
-                    help="mask of sogl_ctx_set_task_links: 2 (default) = the lu task runs its most "
-                         "critical panel GEMM itself; 1 = after-links (measured slower); 0 = none")
+                    help="mask of sogl_ctx_set_task_links: 2 (default) = lu tasks run their panels themselves "
+                         "(diagonal chains); 1 = after-links (measured slower); 0 = none")
     ap.add_argument("--no-reuse-leg", action="store_true",
                     help="skip the FP64 leg that factors with pool slot reuse forced on")
     ap.add_argument("--no-chain", action="store_true",
